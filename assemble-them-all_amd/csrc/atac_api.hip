@@ -473,7 +473,7 @@ static void release_plan(atac_batch b) {
 // partial row per work item: mode 0-2 the evaluation's, 3 the adjoint's, 4 the
 // fused pass's (wrench and adjoint)
 static int64_t part_width_of(int mode) {
-    return mode == 4 ? kFmOut + kVjpOut : mode == 3 ? kVjpOut : (mode == 2 ? 24 + 288 : (mode == 1 ? 24 : 12));
+    return mode == 4 ? kFmOut + kVjpOut : mode == 3 ? kVjpOut : (mode == 2 ? kJacRow : (mode == 1 ? 24 : 12));
 }
 
 // Allocates what an evaluation of this mode and precision (or the adjoint,
@@ -882,7 +882,7 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
     ra.overflow_out = overflow_out;
     ra.host_dst = overflow_out ? 1 : 0;   // the small-batch graph's outputs are its pinned staging
     hipEvent_t t3 = stage_begin(b, st);
-    ATAC_HIP(launch_reduce(ra, st));
+    ATAC_HIP(mode == 2 ? launch_reduce_jacobian(ra, st) : launch_reduce(ra, st));
     stage_end(b, ST_REDUCE, t3, st);
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     ATAC_HIP(hipStreamIsCapturing(st, &cs));

@@ -75,7 +75,7 @@ struct ContactArgs {
     int32_t* counters;
     int32_t chunk_cap;
     int32_t pad;
-    double* partial;            // per work item: fm 12 | p6 12 | Km 144 | Dm 144 (as the mode has them);
+    double* partial;            // per work item: fm 12 | p6 12 | Km/Dm block sums 135 (as the mode has them);
                                 // the fused pass: fm 12 | kVjpOut
     const double* g_fm;         // the fused pass: d(loss)/d(wrench) per instance (n_inst x 12)
 };
@@ -153,6 +153,8 @@ hipError_t launch_vjp(const VjpArgs& a, bool precise, int grid, hipStream_t st);
 hipError_t launch_fused(const ContactArgs& a, bool precise, int grid, hipStream_t st);
 const void* vjp_kernel_ptr(bool precise);
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st);
+// the same after the Km/Dm pass: rows of kJacRow, dst = fm, dfm_dp6, Km, Dm
+hipError_t launch_reduce_jacobian(const ReduceArgs& a, hipStream_t st);
 hipError_t launch_grid_setup(const GridDev& G, float4* cells, hipStream_t st);
 // the cell classification of a grid for one col_th (cls_bytes(G) bytes)
 hipError_t launch_cls_setup(const GridDev& G, double col_th, uint8_t* cls, hipStream_t st);

@@ -16,18 +16,20 @@
 //                  record slots and work items of the bounded record pool.
 //   slow_kernel    the FP64 FD-stencil samples of the few active points whose
 //                  stencil leaves their cell.
-//   contact_kernel work items of kChunk active points, one wavefront each (one
-//                  workgroup each with Km/Dm): builds
+//   contact_kernel work items of kChunk active points, one wavefront each: builds
 //                  the records (sample of phi, grad phi, Hessian) and sums the
-//                  wrench (optionally the p6 column and Km/Dm tangent columns)
-//                  into the item's partial row.
+//                  wrench (optionally the p6 column) into the item's partial row.
+//   jacobian_kernel the same with Km/Dm, one workgroup per item: sums the wrench,
+//                  the p6 column and the 3x3 blocks that Km and Dm are made of.
 //   vjp_kernel     the adjoint of the same records.
-//   reduce_kernel  per-instance sums of the partial rows in a fixed order.
+//   reduce_kernel  per-instance sums of the partial rows in a fixed order
+//                  (reduce_jacobian_kernel: then Km and Dm from the block sums).
 // Plain path (the one-launch-per-instance baseline): plain_kernel, one lane per
 // point, inline contact math, FP64 atomics.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 #include "atac_kernels.h"
 #include "contact_math.h"
 
@@ -445,27 +447,36 @@ __device__ __forceinline__ double lds_column_sums(double* s, const double (&v)[N
 }
 
 // ------------------------------------------------------------------ batched contact pass
-// Work items of kChunk records, one wavefront each: the wrench (and p6 column,
-// and the Km/Dm tangent columns) of every record, summed per lane, then over
-// the wave in a fixed order into the item's partial row.
-template <int MODE, typename R>
+// A lane's active contact `j` of a work item: its record, built from the packed
+// cell and stored for the adjoint on the fast path, read back on the slow one.
+template <typename Rec>
+__device__ __forceinline__ Rec item_record(const GridDev& G, const InstDev& in, uint32_t e, float qx, float qy, float qz,
+                                           Rec* rec) {
+    if (e & kActSlow) return load_rec(rec);   // written by the slow pass
+    Rec r;
+    double cc[3], fd[3];
+    int idx[3];
+    grid_coords(in, qx, qy, qz, cc);
+    cell_of_c(G, cc, idx, fd);
+    const Corners cr = G.fast ? load_cell(G, idx[0], idx[1], idx[2]) : load_corners(G, idx[0], idx[1], idx[2]);
+    r.a[0] = qx; r.a[1] = qy; r.a[2] = qz; r.a[3] = __uint_as_float(e);
+    record_fast(G, in, cr, fd, r);
+    store_rec(rec, r);
+    return r;
+}
+
+// Work items of kChunk records, one wavefront each: the wrench (and p6 column) of
+// every record, summed per lane, then over the wave in a fixed order into the
+// item's partial row.
+template <bool P6, typename R>
 __global__ __launch_bounds__(256) void contact_kernel(ContactArgs a) {
     using Rec = typename RecOf<R>::type;
-    constexpr bool P6 = MODE >= 1;
-    constexpr bool DERIV = MODE >= 2;
     constexpr int NF = P6 ? 24 : 12;
-    constexpr int NACC = NF + (DERIV ? 288 : 0);
-    // records per lane: a wavefront takes a whole work item (kChunk records, 4 per lane),
-    // except with the Km/Dm columns, where the 24 tangent columns and their wave sums
-    // dominate and a workgroup takes an item, its wave w records [64 w, 64 w + 64): four
-    // times the wavefronts for the same work, which small batches need to fill the GPU
-    constexpr int U = DERIV ? 1 : kChunk / 64;
-    __shared__ double s_km[DERIV ? 4 : 1][DERIV ? 288 : 1];
+    constexpr int U = kChunk / 64;   // records per lane
     __shared__ double s_red[4][64 * NF];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int total = min(a.counters[CNT_CHUNKS], a.chunk_cap);
-    const int j0 = DERIV ? 64 * w : 0;
-    for (int c = DERIV ? (int)blockIdx.x : wave_id(); c < total; c += DERIV ? (int)gridDim.x : wave_count()) {
+    for (int c = wave_id(); c < total; c += wave_count()) {
         const ChunkDev ch = as_const(a.chunks)[c];
         const InstDev in = as_const(a.inst)[ch.inst];
         const GridDev G = as_const(a.grids)[in.grid];
@@ -476,13 +487,11 @@ __global__ __launch_bounds__(256) void contact_kernel(ContactArgs a) {
         LaneAcc<R> acc[NF];
 #pragma unroll
         for (int k = 0; k < NF; ++k) acc[k].zero();
-        if (DERIV)
-            for (int k = lane; k < 288; k += 64) s_km[DERIV ? w : 0][DERIV ? k : 0] = 0.0;
         // this lane's active-list entries and points, all loaded first
         uint32_t e[U];
         float qx[U], qy[U], qz[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) e[u] = (j0 + u * 64 + lane < n) ? act[j0 + u * 64 + lane] : kActSlow;
+        for (int u = 0; u < U; ++u) e[u] = (u * 64 + lane < n) ? act[u * 64 + lane] : kActSlow;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t off = e[u] & ~kActSlow;
@@ -492,24 +501,10 @@ __global__ __launch_bounds__(256) void contact_kernel(ContactArgs a) {
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int j = j0 + u * 64 + lane;
-            const bool have = j < n;
-            ContactFwd<R> s;
-            if (have) {
-                Rec r;
-                if (e[u] & kActSlow) {
-                    r = load_rec(rec + j);   // written by the slow pass
-                } else {
-                    // fast-path record: the sample from the packed cell, kept for the adjoint
-                    double cc[3], fd[3];
-                    int idx[3];
-                    grid_coords(in, qx[u], qy[u], qz[u], cc);
-                    cell_of_c(G, cc, idx, fd);
-                    const Corners cr = G.fast ? load_cell(G, idx[0], idx[1], idx[2]) : load_corners(G, idx[0], idx[1], idx[2]);
-                    r.a[0] = qx[u]; r.a[1] = qy[u]; r.a[2] = qz[u]; r.a[3] = __uint_as_float(e[u]);
-                    record_fast(G, in, cr, fd, r);
-                    store_rec(rec + j, r);
-                }
+            const int j = u * 64 + lane;
+            if (j < n) {
+                const Rec r = item_record(G, in, e[u], qx[u], qy[u], qz[u], rec + j);
+                ContactFwd<R> s;
                 record_decode(r, a.slow_diag, in, s);
                 R p6[12];
                 contact_forward<R>(I, s, P6 ? p6 : nullptr);
@@ -520,50 +515,124 @@ __global__ __launch_bounds__(256) void contact_kernel(ContactArgs a) {
                     for (int k = 0; k < 12; ++k) acc[P6 ? 12 + k : 0].add(p6[k]);
                 }
             }
-            if (DERIV) {
-                // columns of Km (jj < 12) and Dm (jj >= 12); every lane takes part in the sums
-                for (int jj = 0; jj < 24; ++jj) {
-                    R col[12];
-#pragma unroll
-                    for (int r = 0; r < 12; ++r) col[r] = (R)0;
-                    if (have) contact_jvp<R>(I, s, unit_tangent<R>(jj), col);
-                    const int obase = (jj < 12) ? jj : 144 + (jj - 12);
-                    double mine = 0.0;   // lane r < 12 keeps row r of the column
-#pragma unroll
-                    for (int r = 0; r < 12; ++r) {
-                        const double v = wave_sum((double)col[r]);
-                        mine = (lane == r) ? v : mine;
-                    }
-                    if (lane < 12) s_km[DERIV ? w : 0][DERIV ? obase + 12 * lane : 0] += mine;
-                }
-            }
         }
-        double* dst = a.partial + (int64_t)c * NACC;
+        double* dst = a.partial + (int64_t)c * NF;
         double lv[NF];
 #pragma unroll
         for (int k = 0; k < NF; ++k) lv[k] = acc[k].value();
-        if (!DERIV) {
-            const double col = lds_column_sums<NF>(&s_red[w][0], lv);
-            if (lane < NF) dst[lane] = col;
+        const double col = lds_column_sums<NF>(&s_red[w][0], lv);
+        if (lane < NF) dst[lane] = col;
+    }
+}
+
+// ------------------------------------------------------------------ wrench and Jacobian sums
+// Values a wavefront sums over its lanes, handed over one at a time (put<k>, in
+// order of k): 32 columns wait in LDS (64 rows of 33 doubles: conflict-free writes
+// by row and reads by column), then two lanes add each column, 32 rows each, and
+// the sums go to `out`. Rows at or past `n` (lanes without a contact) are left
+// out. One LDS write, one read and one add per value: the butterfly over the
+// lanes it replaces took about 25 VALU instructions.
+template <int N>
+struct WaveColumns {
+    static constexpr int W = 32, STRIDE = 33, SIZE = 64 * STRIDE;
+    double* s;     // SIZE doubles of this wavefront
+    double* out;   // N rounded up to W
+    int lane, n;
+    template <int K>
+    __device__ __forceinline__ void put(double v) const {
+        s[lane * STRIDE + K % W] = v;
+        if constexpr (K % W == W - 1 || K == N - 1) flush(out + K / W * W);
+    }
+    template <int K0, int... I>
+    __device__ __forceinline__ void put_all(const double* v, std::integer_sequence<int, I...>) const {
+        (put<K0 + I>(v[I]), ...);
+    }
+    __device__ __forceinline__ void flush(double* to) const {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int r0 = lane & 32;
+        const double* p = s + r0 * STRIDE + (lane & 31);
+        double q[4] = {0.0, 0.0, 0.0, 0.0};
+        if (n >= 64) {
+#pragma unroll
+            for (int i = 0; i < 32; i += 4)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) q[j] += p[(i + j) * STRIDE];
         } else {
-            // the item's row. The wrench (and p6) sums in the order of the one-wavefront
-            // modes: per lane the records 64 apart in turn (wave order), then the lanes'
-            // column sums; the Km/Dm sums in wave order.
-#pragma unroll
-            for (int k = 0; k < NF; ++k) s_red[w][lane * NF + k] = lv[k];
-            __syncthreads();
-            if (w == 0) {
-#pragma unroll
-                for (int k = 0; k < NF; ++k)
-                    lv[k] = ((s_red[0][lane * NF + k] + s_red[1][lane * NF + k]) + s_red[2][lane * NF + k]) +
-                            s_red[3][lane * NF + k];
-                const double col = lds_column_sums<NF>(&s_red[0][0], lv);
-                if (lane < NF) dst[lane] = col;
+#pragma unroll 1
+            for (int i = 0; i < min(n, 32); ++i) {
+                const double v = p[i * STRIDE];
+                q[0] += r0 + i < n ? v : 0.0;
             }
-            for (int k = threadIdx.x; k < 288; k += 256)
-                dst[NF + k] = ((s_km[0][k] + s_km[DERIV ? 1 : 0][k]) + s_km[DERIV ? 2 : 0][k]) + s_km[DERIV ? 3 : 0][k];
-            __syncthreads();
         }
+        double v = (q[0] + q[1]) + (q[2] + q[3]);
+        v += __shfl_xor(v, 32, 64);
+        if (lane < W) to[lane] = v;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();   // the columns are free for the next round
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+};
+using JacColumns = WaveColumns<kJacRow>;
+constexpr int kJacRowPad = (kJacRow + JacColumns::W - 1) / JacColumns::W * JacColumns::W;
+
+// A contact's wrench, p6 column and Jacobian blocks into the columns (kJacRow
+// values), from its forward state.
+template <typename R>
+__device__ __forceinline__ void put_jac_row(const JacColumns& col, const JacInst& J, const ContactFwd<R>& s, const R p6[12]) {
+    double f[24];
+#pragma unroll
+    for (int k = 0; k < 12; ++k) { f[k] = (double)s.f[k]; f[12 + k] = (double)p6[k]; }
+    col.put_all<0>(f, std::make_integer_sequence<int, 24>());
+    const double H[6] = {s.H[0], s.H[1], s.H[2], s.H[3], s.H[4], s.H[5]};
+    contact_jac(J, mk3<double>(s.xi1.x, s.xi1.y, s.xi1.z), (double)s.d, mk3<double>(s.g.x, s.g.y, s.g.z), H, s.fric, s.stat,
+                [&](auto b, const m3<double>& M) {
+                    col.put_all<24 + 9 * decltype(b)::value>(M.a, std::make_integer_sequence<int, 9>());
+                });
+}
+
+// Work items of kChunk records, one workgroup each, wavefront w taking records
+// [64 w, 64 w + 64), one per lane: the wrench, the p6 column and the blocks Km and
+// Dm are made of (contact_jac), summed over the item into its partial row
+// (kJacRow values). Bound by instruction issue: about 1,700 instructions per 64
+// contacts, where 24 tangents per contact and their 288 wave sums took about 13,000
+// (an evaluation of 256 poses x 5,000 points with Km/Dm: 149 -> 57 us; of 26 poses
+// from host memory: 132 -> 80 us). 64 contacts per wavefront rather than 256:
+// small batches have few items and need the waves.
+template <typename R>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void jacobian_kernel(ContactArgs a) {
+    using Rec = typename RecOf<R>::type;
+    __shared__ double s_col[4][JacColumns::SIZE];
+    __shared__ double s_part[4][kJacRowPad];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int total = min(a.counters[CNT_CHUNKS], a.chunk_cap);
+    for (int c = (int)blockIdx.x; c < total; c += (int)gridDim.x) {
+        const ChunkDev ch = as_const(a.chunks)[c];
+        const int n = ch.n - 64 * w;   // this wavefront's records
+        if (n > 0) {
+            const InstDev in = as_const(a.inst)[ch.inst];
+            const GridDev G = as_const(a.grids)[in.grid];
+            // lanes past the end repeat the last record; their rows are not summed
+            const int j = 64 * w + min(lane, n - 1);
+            Rec* rec = static_cast<Rec*>(a.rec) + ch.rec0 + j;
+            const uint32_t e = (as_global(a.act) + ch.rec0)[j], off = e & ~kActSlow;
+            const Rec r = item_record(G, in, e, as_global(in.px)[off], as_global(in.py)[off], as_global(in.pz)[off], rec);
+            ContactFwd<R> s;
+            R p6[12];
+            record_decode(r, a.slow_diag, in, s);
+            contact_forward<R>(make_inst<R>(in), s, p6);
+            put_jac_row<R>(JacColumns{&s_col[w][0], &s_part[w][0], lane, n}, jac_inst(in), s, p6);
+        }
+        __syncthreads();
+        const int k = (int)threadIdx.x;
+        if (k < kJacRow && ch.n > 0) {
+            double v = s_part[0][k];
+            for (int i = 1; i < 4; ++i)
+                if (ch.n > 64 * i) v += s_part[i][k];
+            a.partial[(int64_t)c * kJacRow + k] = v;
+        }
+        __syncthreads();
     }
 }
 
@@ -753,6 +822,80 @@ __global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
     if (a.n_active) {
         const int n = (int)wave_sum((double)nact);
         if (lane == 0) a.n_active[i] = ovf ? -1 : n;
+    }
+    if (a.host_dst) __threadfence_system();   // the stores reach host memory before the launch completes
+}
+
+// The per-instance reduction of jacobian_kernel's rows, one workgroup per
+// instance: thread k sums component k of the instance's rows, in tile order and
+// each tile's items in order (the rows of 64 tiles listed in LDS first, so that
+// their reads go out together); the wrench and p6 sums are outputs, and the
+// threads form the 288 entries of Km and Dm from the block sums (jac_entry).
+__global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
+    constexpr int kRows = 64 * 32;   // a tile holds at most 8192 / kChunk items
+    __shared__ int s_rows[kRows];
+    __shared__ int s_nrows, s_nact;
+    __shared__ double s_sum[kJacRow], s_R[9], s_t[3];
+    const int k = (int)threadIdx.x, i = (int)blockIdx.x;
+    const bool ovf = a.counters[CNT_OVERFLOW] != 0;
+    if (a.overflow_out && i == 0 && k == 0) *a.overflow_out = ovf ? 1 : 0;
+    const InstDev in = as_const(a.inst)[i];
+    const auto part = as_global(a.partial);
+    double sum = 0.0;
+    int nact = 0;
+    for (int g0 = 0; g0 < in.tile_count; g0 += 64) {
+        if (k < 64) {
+            int cnt = 0, c0 = 0;
+            if (g0 + k < in.tile_count) {   // tile_chunk0 is only meaningful when cnt > 0
+                cnt = a.tile_active[in.tile_begin + g0 + k];
+                c0 = a.tile_chunk0[in.tile_begin + g0 + k];
+            }
+            const int nch = (cnt + kChunk - 1) / kChunk;
+            int pos = nch;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int v = __shfl_up(pos, d, 64);
+                if (k >= d) pos += v;
+            }
+            for (int j = 0; j < nch; ++j) s_rows[pos - nch + j] = c0 + j;
+            nact += cnt;
+            if (k == 63) s_nrows = pos;
+        }
+        __syncthreads();
+        const int nr = s_nrows;
+        if (k < kJacRow) {
+            int j = 0;
+            for (; j + 8 <= nr; j += 8) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = part[(int64_t)s_rows[j + u] * kJacRow + k];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) sum += v[u];
+            }
+            for (; j < nr; ++j) sum += part[(int64_t)s_rows[j] * kJacRow + k];
+        }
+        __syncthreads();
+    }
+    if (k < kJacRow) s_sum[k] = ovf ? __builtin_nan("") : sum;
+    if (k < 64) {
+        nact = (int)wave_sum((double)nact);
+        if (k == 0) s_nact = nact;
+    }
+    if (k == 64) {
+        const JacInst J = jac_inst(in);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) s_R[q] = J.R.a[q];
+        s_t[0] = J.t.x; s_t[1] = J.t.y; s_t[2] = J.t.z;
+    }
+    __syncthreads();
+    if (k < 12 && a.dst[0]) a.dst[0][(int64_t)i * 12 + k] = s_sum[k];
+    if (k >= 12 && k < 24 && a.dst[1]) a.dst[1][(int64_t)i * 12 + k - 12] = s_sum[k];
+    if (k == 0 && a.n_active) a.n_active[i] = ovf ? -1 : s_nact;
+    if (a.dst[2] || a.dst[3]) {
+        for (int e = k; e < 288; e += 256) {
+            const int row = e / 24, col = e % 24;
+            double* dst = col < 12 ? a.dst[2] : a.dst[3];
+            if (dst) dst[(int64_t)i * 144 + 12 * row + (col < 12 ? col : col - 12)] = jac_entry(s_sum + 24, s_sum + 9, s_R, s_t, row, col);
+        }
     }
     if (a.host_dst) __threadfence_system();   // the stores reach host memory before the launch completes
 }
@@ -1050,12 +1193,14 @@ hipError_t launch_slow(const SlowArgs& a, bool precise, int grid, hipStream_t st
     return hipGetLastError();
 }
 
-template <int MODE, typename R>
-static const void* contact_ptr_t() { return (const void*)&contact_kernel<MODE, R>; }
+template <typename R>
+static const void* contact_ptr_t(int mode) {
+    return mode == 0   ? (const void*)&contact_kernel<false, R>
+           : mode == 1 ? (const void*)&contact_kernel<true, R> : (const void*)&jacobian_kernel<R>;
+}
 
 const void* contact_kernel_ptr(int mode, bool precise) {
-    if (precise) return mode == 0 ? contact_ptr_t<0, double>() : mode == 1 ? contact_ptr_t<1, double>() : contact_ptr_t<2, double>();
-    return mode == 0 ? contact_ptr_t<0, float>() : mode == 1 ? contact_ptr_t<1, float>() : contact_ptr_t<2, float>();
+    return precise ? contact_ptr_t<double>(mode) : contact_ptr_t<float>(mode);
 }
 
 hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, int grid, hipStream_t st) {
@@ -1083,6 +1228,12 @@ const void* vjp_kernel_ptr(bool precise) {
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st) {
     if (a.n_inst <= 0) return hipSuccess;
     hipLaunchKernelGGL(reduce_kernel, dim3((a.n_inst + 3) / 4), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_reduce_jacobian(const ReduceArgs& a, hipStream_t st) {
+    if (a.n_inst <= 0) return hipSuccess;
+    hipLaunchKernelGGL(reduce_jacobian_kernel, dim3(a.n_inst), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

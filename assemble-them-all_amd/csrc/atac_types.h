@@ -137,8 +137,7 @@ enum {
 
 constexpr int kFmOut = 12;          // wrench of both bodies
 constexpr int kP6Out = 12;          // d fm / d contact_scale (reference p6 column)
-constexpr int kKmOut = 144;
-constexpr int kDmOut = 144;
+constexpr int kJacRow = 12 + 12 + 135;   // with Km/Dm: wrench, p6 column and the Jacobian's block sums
 constexpr int kVjpOut = 26;         // q1(6) q2(6) phi1(6) phi2(6) kn(1) kt(1)
 
 }  // namespace atac

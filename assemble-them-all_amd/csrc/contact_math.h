@@ -23,6 +23,7 @@
 #include <hip/hip_runtime.h>
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
 #include "atac_types.h"
 
 #define ATAC_HD __host__ __device__ __forceinline__
@@ -1255,6 +1256,230 @@ ATAC_HD void contact_jvp(const InstR<R>& I, const ContactFwd<R>& s, const Tangen
     }
     df[0] = a1.x; df[1] = a1.y; df[2] = a1.z; df[3] = l1.x; df[4] = l1.y; df[5] = l1.z;
     df[6] = a2.x; df[7] = a2.y; df[8] = a2.z; df[9] = l2.x; df[10] = l2.y; df[11] = l2.z;
+}
+
+// ------------------------------------------------------------------ Km / Dm as sums of 3x3 blocks
+// contact_jvp costs 24 tangents per contact and 288 sums over the contacts. Both
+// bodies being rigid, one contact's 12 x 24 Jacobian is made of few 3x3 blocks.
+// In the SDF body's axes, with R = R2^T R1, X = R xi1, Y = xi2 and F the contact
+// force (f1 = R^T F, f2 = -F), F is a function of the point x = X + t
+// (t = R2^T (p1 - p2)), the relative velocity c = R u1 - v2 and w2, and w2 acts as
+// dc = dw2-cross terms Y x w2p:
+//   dF = A dx + B (dc + Y x w2p) - T (r . om), A = dF/dx, B = dF/dc
+// (T = the tangential velocity and r: the dynamic friction scale also follows the
+// lever arm |xi1 x n1|, which turns with the relative rotation om = R om1 - om2).
+// Its columns for the body 2 pose follow from those for the body 1 pose (a common
+// motion of both bodies changes nothing), and the rotation by R is the same for
+// every contact of an instance: so the contacts sum the 15 blocks
+//   A, [X]A, V = -[Y]A + [F]Z, W = [Y](C + [F]) - [F]Z[X], C = A[X] + B[U] + T r^T - [F], [X]C,
+//   B, [X]B, [Y]B, B[X], [X]B[X], [Y]B[X], B[Y], [X]B[Y], [Y]B[Y]
+// ([v] the cross-product matrix, U = R u1, Z = d xi2 / dx), and jac_entry forms the
+// 288 entries of Km and Dm from the sums, once per instance. In FP64 for both
+// arithmetics (FP64 and unpacked FP32 issue at the same rate on gfx950); the
+// sample, the friction branch and, in the FP32 arithmetic, the wrench are the
+// forward pass's. The poses are rigid (R^T R = I), as everywhere in the wrench.
+constexpr int kJacBlocks = 15, kJacSums = 9 * kJacBlocks;
+enum { JB_A, JB_XA, JB_V, JB_W, JB_C, JB_XC, JB_B, JB_XB, JB_YB, JB_BX, JB_XBX, JB_YBX, JB_BY, JB_XBY, JB_YBY };
+
+// [v] M and M [v]
+ATAC_HD m3<double> skew_left(v3<double> v, const m3<double>& M) {
+    m3<double> o;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        o.a[j] = v.y * M.a[6 + j] - v.z * M.a[3 + j];
+        o.a[3 + j] = v.z * M.a[j] - v.x * M.a[6 + j];
+        o.a[6 + j] = v.x * M.a[3 + j] - v.y * M.a[j];
+    }
+    return o;
+}
+ATAC_HD m3<double> skew_right(const m3<double>& M, v3<double> v) {
+    m3<double> o;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        o.a[3 * i] = M.a[3 * i + 1] * v.z - M.a[3 * i + 2] * v.y;
+        o.a[3 * i + 1] = M.a[3 * i + 2] * v.x - M.a[3 * i] * v.z;
+        o.a[3 * i + 2] = M.a[3 * i] * v.y - M.a[3 * i + 1] * v.x;
+    }
+    return o;
+}
+// M += s a b^T
+ATAC_HD void add_outer(m3<double>& M, double s, v3<double> a, v3<double> b) {
+    const double p[3] = {s * a.x, s * a.y, s * a.z};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) { M.a[3 * i] += p[i] * b.x; M.a[3 * i + 1] += p[i] * b.y; M.a[3 * i + 2] += p[i] * b.z; }
+}
+// M += s [v]
+ATAC_HD void add_skew(m3<double>& M, double s, v3<double> v) {
+    M.a[1] -= s * v.z; M.a[2] += s * v.y; M.a[3] += s * v.z; M.a[5] -= s * v.x; M.a[6] -= s * v.y; M.a[7] += s * v.x;
+}
+
+// What contact_jac needs of an instance: R = R2^T R1, t = R2^T (p1 - p2), the
+// twists and the force parameters.
+struct JacInst {
+    m3<double> R;
+    v3<double> t, w1, v1, w2, v2;
+    double kn, kt, mu, c;
+};
+ATAC_HD JacInst jac_inst(const InstDev& in) {
+    JacInst J;
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            J.R.a[3 * r + c] = in.R2[r] * in.R1[c] + in.R2[3 + r] * in.R1[3 + c] + in.R2[6 + r] * in.R1[6 + c];
+    const double q0 = in.p1[0] - in.p2[0], q1 = in.p1[1] - in.p2[1], q2 = in.p1[2] - in.p2[2];
+    J.t = mk3<double>(in.R2[0] * q0 + in.R2[3] * q1 + in.R2[6] * q2, in.R2[1] * q0 + in.R2[4] * q1 + in.R2[7] * q2,
+                      in.R2[2] * q0 + in.R2[5] * q1 + in.R2[8] * q2);
+    J.w1 = mk3<double>(in.w1[0], in.w1[1], in.w1[2]); J.v1 = mk3<double>(in.v1[0], in.v1[1], in.v1[2]);
+    J.w2 = mk3<double>(in.w2[0], in.w2[1], in.w2[2]); J.v2 = mk3<double>(in.v2[0], in.v2[1], in.v2[2]);
+    J.kn = in.kn; J.kt = in.kt; J.mu = in.mu; J.c = in.damping;
+    return J;
+}
+
+template <int B>
+using jac_block = std::integral_constant<int, B>;
+
+// The 15 blocks of one contact, handed to put(jac_block<JB_*>(), matrix) in order: its point
+// xi1, sample (d, g, H as in ContactFwd) and friction branch.
+template <typename Put>
+ATAC_HD void contact_jac(const JacInst& J, v3<double> xi1, double d, v3<double> g, const double H[6], bool fric,
+                         bool stat, Put&& put) {
+    const v3<double> X = mv(J.R, xi1), U = mv(J.R, cross(J.w1, xi1) + J.v1), x = X + J.t;
+    const double gn = norm(g), rg = 1.0 / gn;
+    const v3<double> e = rg * g, Y = x - d * e, c = U - J.v2, xd = cross(x, J.w2) + c;
+    const double ddot = dot(g, xd), lam = -J.kn * d + J.c * ddot * d;
+    // E = d e / dx = (I - e e^T) H / gn
+    const v3<double> he = symv(H, e);
+    m3<double> E;
+    const double h9[9] = {H[0], H[3], H[4], H[3], H[1], H[5], H[4], H[5], H[2]};
+#pragma unroll
+    for (int k = 0; k < 9; ++k) E.a[k] = rg * h9[k];
+    add_outer(E, -rg, e, he);
+    // Z = d xi2 / dx = I - e g^T - d E
+    m3<double> Z;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) Z.a[k] = ((k & 3) == 0 ? 1.0 : 0.0) - d * E.a[k];
+    add_outer(Z, -1.0, e, g);
+    const double cd = J.c * d;
+    const v3<double> lx = (J.c * ddot - J.kn) * g + cd * (symv(H, xd) + cross(J.w2, g)), lc = cd * g;
+    v3<double> F = lam * e;
+    m3<double> A, B;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) { A.a[k] = lam * E.a[k]; B.a[k] = 0.0; }
+    add_outer(A, 1.0, e, lx);
+    add_outer(B, 1.0, e, lc);
+    v3<double> T = zero3<double>(), r = zero3<double>();
+    if (fric) {
+        const v3<double> q = c - cross(J.w2, Y);
+        const double eq = dot(e, q);
+        T = q - eq * e;
+        // Q = dT / dx = (I - e e^T) (-[w2] Z) - (e.q) E - e (q^T E)
+        m3<double> Q = skew_left(-J.w2, Z);
+        const v3<double> eQ = mtv(Q, e) + mtv(E, q);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) Q.a[k] -= eq * E.a[k];
+        add_outer(Q, -1.0, e, eQ);
+        double al = J.kt;
+        if (!stat) {
+            // al = mu |lam| m / |T|, m^2 = 1 + |X x e|^2
+            const v3<double> a = cross(X, e);
+            const double m2 = 1.0 + dot(a, a), fcn = sqrt(lam * lam * m2), tn = norm(T);
+            const double k1 = J.mu * lam / (fcn * tn), k2 = k1 * lam;
+            al = J.mu * fcn / tn;
+            const double k3 = al / (tn * tn);
+            const v3<double> ax = (k1 * m2) * lx + k2 * mtv(E, cross(a, X)) - k3 * mtv(Q, T);
+            const v3<double> ac = (k1 * m2) * lc - k3 * T;
+            add_outer(A, -1.0, T, ax);
+            add_outer(B, -1.0, T, ac);
+            r = (-k2 * dot(X, e)) * a;
+        }
+        F = F - al * T;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) { A.a[k] -= al * Q.a[k]; B.a[k] -= (k & 3) == 0 ? al : 0.0; }
+        add_outer(B, al, e, e);
+    }
+    put(jac_block<JB_A>(), A);
+    put(jac_block<JB_XA>(), skew_left(X, A));
+    {   // V and W's part of Z
+        m3<double> FZ = skew_left(F, Z), V = FZ;
+        const m3<double> ya = skew_left(Y, A);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) V.a[k] -= ya.a[k];
+        put(jac_block<JB_V>(), V);
+        m3<double> C = skew_right(A, X);
+        const m3<double> bu = skew_right(B, U);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) C.a[k] += bu.a[k];
+        if (fric && !stat) add_outer(C, 1.0, T, r);
+        m3<double> W = skew_left(Y, C);
+        const m3<double> fzx = skew_right(FZ, X);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) W.a[k] -= fzx.a[k];
+        put(jac_block<JB_W>(), W);
+        add_skew(C, -1.0, F);
+        put(jac_block<JB_C>(), C);
+        put(jac_block<JB_XC>(), skew_left(X, C));
+    }
+    put(jac_block<JB_B>(), B);
+    put(jac_block<JB_XB>(), skew_left(X, B));
+    put(jac_block<JB_YB>(), skew_left(Y, B));
+    const m3<double> BX = skew_right(B, X);
+    put(jac_block<JB_BX>(), BX);
+    put(jac_block<JB_XBX>(), skew_left(X, BX));
+    put(jac_block<JB_YBX>(), skew_left(Y, BX));
+    const m3<double> BY = skew_right(B, Y);
+    put(jac_block<JB_BY>(), BY);
+    put(jac_block<JB_XBY>(), skew_left(X, BY));
+    put(jac_block<JB_YBY>(), skew_left(Y, BY));
+}
+
+// Entry (row, col) of [Km | Dm] (col < 12: Km) from the summed blocks S (9 per
+// block, JB_* order), body 2's summed force f2 (= -F), R and t.
+ATAC_HD double jac_entry(const double* S, const double* f2, const double* R, const double* t, int row, int col) {
+    const int rb = row / 3, ri = row - 3 * rb, cb = col / 3, cj = col - 3 * cb;
+    auto blk = [&](int b, int i, int j) { return S[9 * b + 3 * i + j]; };
+    // columns om1 and v1 of the pose (in R-turned axes)
+    auto om1 = [&](int i, int j) {
+        if (rb == 0) return -blk(JB_XC, i, j);
+        if (rb == 1) return -blk(JB_C, i, j);
+        if (rb == 2) return blk(JB_W, i, j);
+        double v = blk(JB_C, i, j);   // C + [F]
+        if (i != j) {
+            const int k = 3 - i - j;
+            v += (j == (i + 1) % 3) ? f2[k] : -f2[k];
+        }
+        return v;
+    };
+    auto v1 = [&](int i, int j) {
+        return rb == 0 ? blk(JB_XA, i, j) : rb == 1 ? blk(JB_A, i, j) : rb == 2 ? blk(JB_V, i, j) : -blk(JB_A, i, j);
+    };
+    const int db = rb == 0 ? JB_XB : rb == 2 ? JB_YB : JB_B;   // its [X] and [Y] products 3 and 6 behind
+    const double ds = rb >= 2 ? -1.0 : 1.0;
+    auto el = [&](int i, int j) {
+        switch (cb) {
+            case 0: return om1(i, j);
+            case 1: return v1(i, j);
+            case 2: {
+                const int j1 = (j + 1) % 3, j2 = (j + 2) % 3;   // (M [t])_ij = M_ij1 t_j2 - M_ij2 t_j1
+                return v1(i, j1) * t[j2] - v1(i, j2) * t[j1] - om1(i, j);
+            }
+            case 3: return -v1(i, j);
+            case 4: return -ds * blk(db + (JB_BX - JB_B), i, j);
+            case 5: return ds * blk(db, i, j);
+            case 6: return ds * blk(db + (JB_BY - JB_B), i, j);
+            default: return -ds * blk(db, i, j);
+        }
+    };
+    const bool turn_c = (cb & 2) == 0;   // body 1 columns: the tangent in body 1's axes
+    double v = 0.0;
+    for (int i = 0; i < 3; ++i) {
+        if (rb >= 2 && i != ri) continue;
+        double q = 0.0;
+        if (turn_c) for (int j = 0; j < 3; ++j) q += el(i, j) * R[3 * j + cj];
+        else q = el(i, cj);
+        v += rb < 2 ? R[3 * i + ri] * q : q;   // body 1 rows: R^T
+    }
+    return v;
 }
 
 // Adjoint of contact_jvp: given gb = d(loss)/d(wrench), returns

@@ -221,6 +221,41 @@ int hc_eval(const float* vals, const int32_t n[3], const double minb[3], const d
     return 0;
 }
 
+// Km and Dm of one force object (FP64 arithmetic) as the batched path forms them:
+// contact_jac's blocks summed over the contacts, then jac_entry.
+int hc_jacobian_blocks(const float* vals, const int32_t n[3], const double minb[3], const double maxb[3],
+                       const double d[3], const float* px, const float* py, const float* pz, int64_t npts,
+                       const atac_instance* inst, double* Km, double* Dm, int64_t counts[3]) {
+    HostGrid hg;
+    host_grid(vals, n, minb, maxb, d, hg);
+    InstDev in;
+    std::memset(&in, 0, sizeof in);
+    compose_instance(*inst, hg.G, px, py, pz, npts, in);
+    host_cls(hg, in);
+    const InstR<double> I = make_inst<double>(in);
+    const JacInst J = jac_inst(in);
+    double S[kJacSums] = {}, f2[3] = {};
+    for (int64_t o = 0; o < npts; ++o) {
+        if (!detect_active(hg.G, in, px[o], py[o], pz[o])) continue;
+        ContactFwd<double> s;
+        const bool slow = sample_via_record<double>(hg.G, in, o, s);
+        contact_forward<double>(I, s, nullptr);
+        ++counts[slow ? 2 : (s.fric && !s.stat ? 1 : 0)];
+        for (int k = 0; k < 3; ++k) f2[k] += s.f[9 + k];
+        contact_jac(J, s.xi1, s.d, s.g, s.H, s.fric, s.stat, [&](auto b, const m3<double>& M) {
+            for (int k = 0; k < 9; ++k) S[9 * decltype(b)::value + k] += M.a[k];
+        });
+    }
+    const double t[3] = {J.t.x, J.t.y, J.t.z};
+    for (int r = 0; r < 12; ++r)
+        for (int c = 0; c < 24; ++c) {
+            const double v = jac_entry(S, f2, J.R.a, t, r, c);
+            if (c < 12) Km[12 * r + c] = v;
+            else Dm[12 * r + c - 12] = v;
+        }
+    return 0;
+}
+
 // Detection values of every point (query_SDF + col_th, +inf outside).
 int hc_detect(const float* vals, const int32_t n[3], const double minb[3], const double maxb[3], const double d[3],
               const float* px, const float* py, const float* pz, int64_t npts, const atac_instance* inst, float* out) {
