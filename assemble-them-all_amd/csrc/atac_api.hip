@@ -1522,13 +1522,13 @@ struct atac_mesh_s {
     int32_t* d_tri = nullptr;
     int32_t* d_F = nullptr;
     int32_t* d_FE = nullptr;
-    double* d_V = nullptr;
+    double* d_tv = nullptr;
     double* d_FN = nullptr;
     double* d_EN = nullptr;
     double* d_VN = nullptr;
     void release() {
         dfree(d_nodes); dfree(d_tri); dfree(d_F); dfree(d_FE);
-        dfree(d_V); dfree(d_FN); dfree(d_EN); dfree(d_VN);
+        dfree(d_tv); dfree(d_FN); dfree(d_EN); dfree(d_VN);
     }
 };
 
@@ -1553,7 +1553,7 @@ int atac_mesh_create(const double* V, int64_t nv, const int64_t* F, int64_t nf, 
     if (!rc) rc = upload(&m->d_tri, h.tri);
     if (!rc) rc = upload(&m->d_F, h.F);
     if (!rc) rc = upload(&m->d_FE, h.FE);
-    if (!rc) rc = upload(&m->d_V, h.V);
+    if (!rc) rc = upload(&m->d_tv, h.tv);
     if (!rc) rc = upload(&m->d_FN, h.FN);
     if (!rc) rc = upload(&m->d_EN, h.EN);
     if (!rc) rc = upload(&m->d_VN, h.VN);
@@ -1563,10 +1563,10 @@ int atac_mesh_create(const double* V, int64_t nv, const int64_t* F, int64_t nf, 
         return rc;
     }
     MeshDev& D = m->dev;
-    D.nodes = m->d_nodes; D.tri = m->d_tri; D.V = m->d_V; D.F = m->d_F;
+    D.nodes = m->d_nodes; D.tri = m->d_tri; D.tv = m->d_tv; D.F = m->d_F;
     D.FN = m->d_FN; D.FE = m->d_FE; D.EN = m->d_EN; D.VN = m->d_VN;
     for (int a = 0; a < 3; ++a) { D.bmin[a] = h.bmin[a]; D.bmax[a] = h.bmax[a]; }
-    D.n_nodes = (int32_t)(h.nodes.size() / 2);
+    D.n_leaves = (int32_t)(h.tri.size() / kBvhWidth);
     D.nf = (int32_t)nf;
     *out = m;
     return ATAC_OK;
@@ -1633,11 +1633,10 @@ int atac_bvh_force_host(atac_mesh m, const atac_instance* inst, const double* xi
     double *dx = nullptr, *dout = nullptr, *dpart = nullptr;
     int64_t *dna = nullptr, *dcnt = nullptr;
     const int64_t nb = bvh_force_blocks(n);
-    if (nb >= ((int64_t)1 << 31)) return fail(ATAC_ERR_INVALID, "atac_bvh_force_host: too many points");
     int rc = dalloc(&dx, (size_t)std::max<int64_t>(3 * n, 1));
     if (!rc) rc = dalloc(&dout, (size_t)kBvhOut);
     if (!rc) rc = dalloc(&dna, 1);
-    if (!rc) rc = dalloc(&dpart, (size_t)(nb * kBvhOut));
+    if (!rc) rc = dalloc(&dpart, (size_t)(nb * kJacRow));
     if (!rc) rc = dalloc(&dcnt, (size_t)nb);
     hipError_t e = hipSuccess;
     std::vector<double> h(kBvhOut);
@@ -1688,7 +1687,7 @@ int atac_bvh_force_noalloc(atac_mesh m, const atac_instance* inst, const double*
     // every workgroup writes its whole row and count, and the reduction reads
     // only the rows of this launch: nothing needs clearing between calls
     a.part = part;
-    a.part_cnt = reinterpret_cast<int64_t*>(part + kBvhScratchBlocks * kBvhOut);
+    a.part_cnt = reinterpret_cast<int64_t*>(part + kBvhMaxBlocks * kJacRow);
     ATAC_HIP(launch_bvh_force(a, (hipStream_t)stream));
     return ATAC_OK;
 }

@@ -3,7 +3,7 @@
 // Body/BVH/AABBTree.h:74-82, i.e. libigl's AABB tree and
 // signed_distance_pseudonormal, libigl not vendored in the reference):
 //   * the closest point over all triangles (FP64, Ericson's closest point on a
-//     triangle by Voronoi regions), the BVH only prunes;
+//     triangle by Voronoi regions), the BVH (bvh.hip's traversal) only prunes;
 //   * the sign from the angle-weighted pseudonormal (Baerentzen & Aanaes 2005) of
 //     the feature the closest point lies on: the face normal in the interior, the
 //     uniform edge normal on an edge, the angle-weighted vertex normal at a vertex,
@@ -20,23 +20,33 @@
 
 namespace atac {
 
-// Node n of the BVH: lo/hi of its box (FP32, rounded outward from the FP64
-// vertices), and in the w lanes: internal node (w0 >= 0): children w0 and w0 + 1;
-// leaf (w0 < 0): triangles tri[-w0 - 1 .. -w0 - 1 + w1) of the leaf order.
+// A node of the BVH is 8 entries, entry n at nodes[2n], nodes[2n + 1]: lo/hi of a
+// child's box (FP32, rounded outward from the FP64 vertices) and, in lo.w, what it
+// is: an internal node (>= 0: the index of its first entry), leaf l (-l - 1:
+// triangles 8l .. 8l + 7 of the leaf order) or nothing (kBvhEmpty). The root's
+// entries are 0 .. 7. The leaf order fills every leaf but the last; its vertices
+// are stored per leaf as 9 coordinates x 8 triangles, so the 8 lanes that test a
+// leaf read 64 bytes per coordinate.
+constexpr int kBvhWidth = 8;
+constexpr int32_t kBvhEmpty = INT32_MIN;
+constexpr int32_t kNoTriangle = INT32_MIN;
 struct MeshDev {
-    const float4* nodes;    // 2 per node: (lo, w0) (hi, w1), w as int bits
-    const int32_t* tri;     // leaf order -> face index f, stored as ~f for a degenerate face
-    const double* V;        // nv x 3
+    const float4* nodes;    // 2 per entry: (lo, code) (hi, 0), the code as int bits
+    const int32_t* tri;     // leaf order -> face index f, stored as ~f for a degenerate face; kNoTriangle past the last
+    const double* tv;       // per leaf: a.x of its 8 triangles, a.y, a.z, b.x, .. c.z
     const int32_t* F;       // nf x 3
     const double* FN;       // nf x 3 face normals (zero for a degenerate face)
     const int32_t* FE;      // nf x 3: edge (opposite corner c) of face f
     const double* EN;       // ne x 3 edge normals
     const double* VN;       // nv x 3 vertex normals
     double bmin[3], bmax[3];  // the vertices' bounding box (BodyMeshObj.cpp:179-182)
-    int32_t n_nodes, nf;
+    int32_t n_leaves, nf;
 };
 
-constexpr int kBvhStack = 64;        // traversal stack (the build keeps the depth below it)
+// Entries waiting during a traversal: each visited node leaves at most 7 of its 8,
+// over at most 9 levels (fewer than 2^30 triangles, 8 per leaf, 8-wide), plus the
+// 8 of the last one.
+constexpr int kBvhStack = 80;
 constexpr double kPseudoEps = 1e-12; // barycentric threshold of the feature test
 
 struct D3 {
@@ -146,58 +156,33 @@ ATAC_HD D3 pseudonormal(const MeshDev& M, int f, const double b[3]) {
     return row3(M.FN, f);
 }
 
-// Signed distance of p (body frame) to the mesh, its pseudonormal and face:
-// libigl's signed_distance_pseudonormal (sign s = +1 when (p - c) . n >= 0).
-ATAC_HD double mesh_signed_distance(const MeshDev& M, D3 p, D3& normal, int& face) {
-    int stack[kBvhStack];
-    int sp = 0;
-    double best = INFINITY;
-    int bf = -1;
-    D3 bc = p;
-    double bb[3] = {1.0, 0.0, 0.0};
-    int node = 0;
-    if (M.n_nodes > 0) {
-        for (;;) {
-            const float4 lo = M.nodes[2 * node], hi = M.nodes[2 * node + 1];
-            const int w0 = node_w(lo.w);
-            if (w0 < 0) {   // leaf
-                const int first = -w0 - 1, cnt = node_w(hi.w);
-                for (int k = 0; k < cnt; ++k) {
-                    const int tf = M.tri[first + k];
-                    const int f = tf < 0 ? ~tf : tf;
-                    double b[3];
-                    const D3 c = closest_on_triangle(p, row3(M.V, M.F[3 * f]), row3(M.V, M.F[3 * f + 1]),
-                                                     row3(M.V, M.F[3 * f + 2]), b, tf < 0);
-                    const D3 pc = sub(p, c);
-                    const double d2 = dt(pc, pc);
-                    if (d2 < best || (d2 == best && f < bf)) {
-                        best = d2; bf = f; bc = c;
-                        bb[0] = b[0]; bb[1] = b[1]; bb[2] = b[2];
-                    }
-                }
-            } else {        // nearer child first; a child is skipped if its box is farther than the best
-                const float4 l0 = M.nodes[2 * w0], h0 = M.nodes[2 * w0 + 1];
-                const float4 l1 = M.nodes[2 * (w0 + 1)], h1 = M.nodes[2 * (w0 + 1) + 1];
-                const double e0 = box_dist2(p, l0, h0), e1 = box_dist2(p, l1, h1);
-                const int near = e0 <= e1 ? w0 : w0 + 1, far = e0 <= e1 ? w0 + 1 : w0;
-                const double en = fmin(e0, e1), ef = fmax(e0, e1);
-                if (ef <= best && sp < kBvhStack) stack[sp++] = far;
-                if (en <= best) { node = near; continue; }
-            }
-            // next node from the stack whose box can still hold the closest point
-            bool found = false;
-            while (sp > 0) {
-                const int n2 = stack[--sp];
-                if (box_dist2(p, M.nodes[2 * n2], M.nodes[2 * n2 + 1]) <= best) { node = n2; found = true; break; }
-            }
-            if (!found) break;
+// The closest point found so far (over the triangles one lane has tested).
+struct MeshHit {
+    double d2 = INFINITY;
+    int f = -1;
+    D3 c;
+    double b[3];
+    // Triangle f = (v0, v1, v2); the smaller face wins among equal distances.
+    ATAC_HD void test(D3 p, D3 v0, D3 v1, D3 v2, int face, bool degenerate) {
+        double bb[3];
+        const D3 q = closest_on_triangle(p, v0, v1, v2, bb, degenerate);
+        const D3 pc = sub(p, q);
+        const double e = dt(pc, pc);
+        if (e < d2 || (e == d2 && face < f)) {
+            d2 = e; f = face; c = q;
+            b[0] = bb[0]; b[1] = bb[1]; b[2] = bb[2];
         }
     }
-    face = bf;
-    if (bf < 0) { normal = d3(0.0, 0.0, 0.0); return INFINITY; }
-    normal = pseudonormal(M, bf, bb);
-    const double s = dt(sub(p, bc), normal) >= 0.0 ? 1.0 : -1.0;
-    return s * sqrt(best);
+};
+
+// Signed distance and pseudonormal for the closest point h of p: libigl's
+// signed_distance_pseudonormal (sign s = +1 when (p - c) . n >= 0); infinity and
+// a zero normal when no triangle was found (a point with a NaN coordinate).
+ATAC_HD double mesh_hit_distance(const MeshDev& M, D3 p, const MeshHit& h, D3& normal) {
+    if (h.f < 0) { normal = d3(0.0, 0.0, 0.0); return INFINITY; }
+    normal = pseudonormal(M, h.f, h.b);
+    const double s = dt(sub(p, h.c), normal) >= 0.0 ? 1.0 : -1.0;
+    return s * sqrt(h.d2);
 }
 
 // Inside the vertices' bounding box (BodyMeshObj::filter_single, BodyMeshObj.cpp:278-286).

@@ -10,6 +10,7 @@
 #include <utility>
 #include "atac.h"
 #include "bvh_host.h"
+#include "wave_ops.h"
 
 namespace atac {
 
@@ -33,9 +34,8 @@ void normalize_rows(std::vector<double>& a) {
     }
 }
 
-constexpr int kLeafTris = 4;
-constexpr int kMaxDepth = 48;   // < kBvhStack
-
+// Median splits along the longest axis of the centroids, three levels to a node,
+// at multiples of the leaf size: every leaf but the last holds kBvhWidth triangles.
 struct Builder {
     const MeshHost& m;
     std::vector<double> cen;      // centroids, nf x 3
@@ -57,17 +57,12 @@ struct Builder {
         hi = make_float4(f32_up(h[0]), f32_up(h[1]), f32_up(h[2]), 0.0f);
     }
     static float bits(int v) { float f; std::memcpy(&f, &v, sizeof f); return f; }
+    static int32_t leaves(int32_t b, int32_t e) { return (e - b + kBvhWidth - 1) / kBvhWidth; }
 
-    // fills node n with faces idx[b, e)
-    void build(int32_t n, int32_t b, int32_t e, int depth) {
-        float4 lo, hi;
-        box_of(b, e, lo, hi);
-        if (e - b <= kLeafTris || depth >= kMaxDepth) {
-            lo.w = bits(-(b + 1));
-            hi.w = bits(e - b);
-            nodes[2 * n] = lo; nodes[2 * n + 1] = hi;
-            return;
-        }
+    // Faces idx[b, e) into at most 2^levels ranges of whole leaves.
+    void split(int32_t b, int32_t e, int levels, std::vector<std::pair<int32_t, int32_t>>& out) {
+        const int32_t n = leaves(b, e);
+        if (levels == 0 || n <= 1) { out.push_back({b, e}); return; }
         double cl[3] = {INFINITY, INFINITY, INFINITY}, ch[3] = {-INFINITY, -INFINITY, -INFINITY};
         for (int32_t k = b; k < e; ++k)
             for (int a = 0; a < 3; ++a) {
@@ -77,18 +72,33 @@ struct Builder {
         int ax = 0;
         for (int a = 1; a < 3; ++a)
             if (ch[a] - cl[a] > ch[ax] - cl[ax]) ax = a;
-        const int32_t mid = b + (e - b) / 2;
+        const int32_t mid = b + kBvhWidth * (n / 2);
         std::nth_element(idx.begin() + b, idx.begin() + mid, idx.begin() + e, [&](int32_t p, int32_t q) {
             const double cp = cen[3 * (int64_t)p + ax], cq = cen[3 * (int64_t)q + ax];
             return cp < cq || (cp == cq && p < q);
         });
-        const int32_t child = (int32_t)(nodes.size() / 2);
-        nodes.resize(nodes.size() + 4);
-        lo.w = bits(child);
-        hi.w = bits(0);
-        nodes[2 * n] = lo; nodes[2 * n + 1] = hi;
-        build(child, b, mid, depth + 1);
-        build(child + 1, mid, e, depth + 1);
+        split(b, mid, levels - 1, out);
+        split(mid, e, levels - 1, out);
+    }
+
+    // Appends the node over faces idx[b, e) and, behind it, its children; returns its first entry.
+    int32_t build(int32_t b, int32_t e) {
+        std::vector<std::pair<int32_t, int32_t>> kids;
+        split(b, e, 3, kids);
+        const int32_t first = (int32_t)(nodes.size() / 2);
+        for (int c = 0; c < kBvhWidth; ++c) {
+            nodes.push_back(make_float4(INFINITY, INFINITY, INFINITY, bits(kBvhEmpty)));
+            nodes.push_back(make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f));
+        }
+        for (size_t c = 0; c < kids.size(); ++c) {
+            const int32_t kb = kids[c].first, ke = kids[c].second;
+            float4 lo, hi;
+            box_of(kb, ke, lo, hi);
+            lo.w = bits(ke - kb <= kBvhWidth ? -(kb / kBvhWidth) - 1 : build(kb, ke));
+            nodes[2 * (first + (int32_t)c)] = lo;
+            nodes[2 * (first + (int32_t)c) + 1] = hi;
+        }
+        return first;
     }
 };
 
@@ -159,26 +169,120 @@ std::string mesh_build(const double* V, int64_t nv, const int64_t* F, int64_t nf
                                 m.V[3 * (int64_t)m.F[3 * f + 2] + a]) / 3.0;
     B.idx.resize(nf);
     std::iota(B.idx.begin(), B.idx.end(), 0);
-    B.nodes.resize(2);
-    B.build(0, 0, (int32_t)nf, 0);
+    B.build(0, (int32_t)nf);
     m.nodes = std::move(B.nodes);
-    m.tri = std::move(B.idx);
-    for (int32_t& f : m.tri)
-        if (degenerate[f]) f = ~f;
+    const int64_t nl = (nf + kBvhWidth - 1) / kBvhWidth;
+    m.tri.assign(nl * kBvhWidth, kNoTriangle);
+    m.tv.assign(nl * kBvhWidth * 9, 0.0);
+    for (int64_t k = 0; k < nf; ++k) {
+        const int32_t f = B.idx[k];
+        m.tri[k] = degenerate[f] ? ~f : f;
+        for (int c = 0; c < 3; ++c)
+            for (int a = 0; a < 3; ++a)
+                m.tv[(k / kBvhWidth) * 9 * kBvhWidth + (3 * c + a) * kBvhWidth + k % kBvhWidth] =
+                    m.V[3 * (int64_t)m.F[3 * (int64_t)f + c] + a];
+    }
     return "";
 }
 
 // ------------------------------------------------------------------ kernels
-// Sum over the 64 lanes (every lane active), a fixed butterfly: the same order on
-// every run, the result on every lane.
-__device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+// Lane values across the 8 lanes of a group (aligned groups of a DPP row): the
+// value of lane gl ^ X.
+template <int X>
+__device__ __forceinline__ uint32_t group_xor(uint32_t v) {
+    constexpr int kQuad[4] = {0xE4, 0xB1, 0x4E, 0x1B};   // quad_perm of lane ^ 0 .. 3
+    int r = (int)v;
+    if constexpr (X & 4) r = dpp_i<0x141>(r);            // row_half_mirror: lane ^ 7
+    constexpr int Q = (X & 4) ? (X ^ 7) : X;
+    if constexpr (Q != 0) r = dpp_i<kQuad[Q]>(r);
+    return (uint32_t)r;
+}
+__device__ __forceinline__ double group_min(double v) {
+    v = fmin(v, dpp_move<0xB1>(v));
+    v = fmin(v, dpp_move<0x4E>(v));
+    return fmin(v, dpp_move<0x141>(v));
 }
 
+// The closest triangle to p, searched by the 8 lanes of a group (all with the same
+// p; gl = the lane's place in it): each lane tests one child box of a node, or one
+// triangle of a leaf, and keeps the best triangle it has tested; the group's bound
+// is the least of them. A node's children whose boxes can hold a closer point go on
+// the group's stack (LDS), the nearest on top: an entry is the child's code and a
+// key, the squared box distance rounded toward zero with the lane in its last three
+// bits, so keys differ and never exceed the distance. One lane per point is limited
+// by its chain of dependent reads (1.08 ms for 60,000 points, 4,224 triangles, under
+// one wavefront per SIMD, and a stack in scratch); eight lanes make eight times the
+// wavefronts and an eighth of the steps.
+__device__ __forceinline__ MeshHit mesh_closest(const MeshDev& M, D3 p, int gl, uint2* stack) {
+    MeshHit h;
+    h.c = p;
+    h.b[0] = h.b[1] = h.b[2] = 0.0;
+    double best = INFINITY;
+    int code = 0, sp = 0;
+    const int shift = (int)(threadIdx.x & 63) & ~7;
+    const auto nodes = as_global(M.nodes);
+    const auto tri = as_global(M.tri);
+    const auto tv = as_global(M.tv);
+    // the next entry that can hold a closer point, or none
+    auto pop = [&]() {
+        while (sp > 0) {
+            const uint2 e = stack[--sp];
+            if ((double)__uint_as_float(e.y) <= best) { code = (int)e.x; return true; }
+        }
+        return false;
+    };
+    for (bool more = true; more;) {
+        while (more && code >= 0) {   // internal nodes, until a leaf is on top
+            const float4 lo = nodes[2 * (code + gl)], hi = nodes[2 * (code + gl) + 1];
+            const double e = box_dist2(p, lo, hi);
+            const bool push = node_w(lo.w) != kBvhEmpty && e <= best;
+            const uint32_t key = push ? (__float_as_uint(__double2float_rz(e)) & ~7u) | (uint32_t)gl : 0u;
+            int rank = 0;   // children on top of this one are nearer, those below it farther
+            rank += group_xor<1>(key) > key;
+            rank += group_xor<2>(key) > key;
+            rank += group_xor<3>(key) > key;
+            rank += group_xor<4>(key) > key;
+            rank += group_xor<5>(key) > key;
+            rank += group_xor<6>(key) > key;
+            rank += group_xor<7>(key) > key;
+            if (push) stack[sp + rank] = make_uint2((uint32_t)node_w(lo.w), key);
+            sp += __popcll((__ballot(push) >> shift) & 0xffull);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            more = pop();
+        }
+        if (!more) break;
+        const int at = (-code - 1) * kBvhWidth;
+        const int t = tri[at + gl];
+        if (t != kNoTriangle) {
+            const auto v = tv + (int64_t)at * 9 + gl;
+            h.test(p, d3(v[0], v[8], v[16]), d3(v[24], v[32], v[40]), d3(v[48], v[56], v[64]), t < 0 ? ~t : t, t < 0);
+        }
+        best = group_min(h.d2);
+        more = pop();
+    }
+    return h;
+}
+
+// Does this lane hold the group's closest triangle (the smallest face among equal
+// distances)? Exactly one lane does; lane 0 when no triangle was found.
+__device__ __forceinline__ bool mesh_winner(const MeshHit& h, int gl) {
+    const double best = group_min(h.d2);
+    uint32_t f = h.d2 == best && h.f >= 0 ? (uint32_t)h.f : 0xffffffffu;
+    uint32_t m = f;
+    m = min(m, group_xor<1>(m));
+    m = min(m, group_xor<2>(m));
+    m = min(m, group_xor<7>(m));
+    return m == 0xffffffffu ? gl == 0 : f == m;
+}
+
+constexpr int kBvhStackStride = kBvhStack + 1;   // odd: the groups' stacks start in different banks
+
 __global__ __launch_bounds__(256) void mesh_distance_kernel(MeshQueryArgs a) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ uint2 s_stack[32][kBvhStackStride];
+    const int gl = threadIdx.x & 7, g = threadIdx.x >> 3;
+    const int64_t i = (int64_t)blockIdx.x * 32 + g;
     if (i >= a.n) return;
     const double q0 = a.xw[3 * i] - a.p2[0], q1 = a.xw[3 * i + 1] - a.p2[1], q2 = a.xw[3 * i + 2] - a.p2[2];
     const D3 x = d3(a.R2[0] * q0 + a.R2[3] * q1 + a.R2[6] * q2, a.R2[1] * q0 + a.R2[4] * q1 + a.R2[7] * q2,
@@ -186,140 +290,173 @@ __global__ __launch_bounds__(256) void mesh_distance_kernel(MeshQueryArgs a) {
     double d = 10.0;   // BodyBVHObj.cpp:326-327: points outside the box keep d = 10, normal 0
     D3 nrm = d3(0.0, 0.0, 0.0);
     int f = -1;
-    if (mesh_box_filter(a.M, x)) d = mesh_signed_distance(a.M, x, nrm, f) + a.col_th;
+    bool mine = gl == 0;
+    if (mesh_box_filter(a.M, x)) {
+        const MeshHit h = mesh_closest(a.M, x, gl, &s_stack[g][0]);
+        mine = mesh_winner(h, gl);
+        if (mine) {
+            d = mesh_hit_distance(a.M, x, h, nrm) + a.col_th;
+            f = h.f;
+        }
+    }
+    if (!mine) return;
     a.d[i] = d;
     if (a.normal) { a.normal[3 * i] = nrm.x; a.normal[3 * i + 1] = nrm.y; a.normal[3 * i + 2] = nrm.z; }
     if (a.face) a.face[i] = f;
 }
 
-// One force object over workgroups of 256 (4 wavefronts), kBvhBlockPoints points
-// each: wave w of workgroup b takes points b*kBvhBlockPoints + w*64 + lane, + 256,
-// ...; a point inside the mesh's box with d = signed distance + col_th < 0 is a
-// contact (collision_detection_general_BVH, CollisionDetection.cpp:150-185)
-// evaluated with the FP64 contact math. Lane sums in FP64, column sums per wave
-// through LDS, the four waves added in order into the workgroup's partial row;
-// bvh_reduce_kernel adds the rows in workgroup order: the same result on every run.
-__global__ __launch_bounds__(256) void bvh_force_kernel(BvhForceArgs a) {
-    constexpr int NF = 24;
-    __shared__ double s_red[4][64 * NF];
-    __shared__ double s_km[4][288];
-    __shared__ double s_row[4][NF];
-    __shared__ int s_cnt[4];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+// One force object over workgroups of 8 wavefronts, block_points points each,
+// kBvhStep at a time: 8 lanes find each point's signed distance; a point inside
+// the mesh's box with d = signed distance + col_th < 0 is a contact
+// (collision_detection_general_BVH, CollisionDetection.cpp:150-185). The first
+// wavefront gathers the step's contacts, in point order, one per lane, and sums
+// their wrench, p6 column and Jacobian blocks (FP64, put_jac_row); the steps'
+// sums are added in order into the workgroup's partial row, and
+// bvh_reduce_kernel adds the rows in a fixed order: the same result on every run.
+// Small steps rather than many points per workgroup: a body has a few thousand
+// points, and the traversal needs every CU (10,242 points in 6 workgroups of one
+// lane per point: 2.46 ms).
+__global__ __launch_bounds__(512) void bvh_force_kernel(BvhForceArgs a) {
+    __shared__ union {
+        uint2 stack[kBvhStep][kBvhStackStride];
+        double col[JacColumns::SIZE];
+    } s;
+    __shared__ double s_part[kJacRowPad];
+    __shared__ double s_hit[4][kBvhStep];   // d, normal
+    __shared__ int s_idx[kBvhStep], s_m;
+    const int tid = (int)threadIdx.x, gl = tid & 7, g = tid >> 3, lane = tid & 63;
     const bool p6on = (a.flags & ATAC_EVAL_P6) != 0u, deriv = (a.flags & ATAC_EVAL_DERIV) != 0u;
-    const InstR<double> I = make_inst<double>(a.in);
-    double acc[NF];
-#pragma unroll
-    for (int k = 0; k < NF; ++k) acc[k] = 0.0;
-    for (int k = lane; k < 288; k += 64) s_km[w][k] = 0.0;
-    int cnt = 0;
-    const int64_t b0 = (int64_t)blockIdx.x * kBvhBlockPoints;
-    const int64_t b1 = b0 + kBvhBlockPoints < a.n ? b0 + kBvhBlockPoints : a.n;
-    for (int64_t base = b0 + (int64_t)w * 64; base < b1; base += 256) {
-        const int64_t i = base + lane;
-        ContactFwd<double> s;
-        bool have = false;
+    const int nrow = deriv ? kJacRow : 24;
+    const int64_t b0 = (int64_t)blockIdx.x * a.block_points;
+    const int64_t b1 = b0 + a.block_points < a.n ? b0 + a.block_points : a.n;
+    double acc = 0.0;   // thread k < kJacRow: component k of the row
+    int64_t cnt = 0;
+    for (int64_t base = b0; base < b1; base += kBvhStep) {
+        const int64_t i = base + g;
+        bool mine = gl == 0;
+        double d = 1.0;   // no contact
+        D3 nrm = d3(0.0, 0.0, 0.0);
         if (i < b1) {
             double x[3];
             body2_point(a.in, a.xi[3 * i], a.xi[3 * i + 1], a.xi[3 * i + 2], x);
             const D3 xb = d3(x[0], x[1], x[2]);
             if (mesh_box_filter(a.M, xb)) {
-                D3 nrm;
-                int f;
-                const double d = mesh_signed_distance(a.M, xb, nrm, f) + a.in.col_th;
-                if (d < 0.0) {
-                    have = true;
-                    s.xi1 = mk3<double>(a.xi[3 * i], a.xi[3 * i + 1], a.xi[3 * i + 2]);
-                    s.x = mk3<double>(x[0], x[1], x[2]);
-                    s.d = d;
-                    s.g = mk3<double>(nrm.x, nrm.y, nrm.z);
-                    for (int k = 0; k < 6; ++k) s.H[k] = 0.0;
-                    s.slow = false;
+                const MeshHit h = mesh_closest(a.M, xb, gl, &s.stack[g][0]);
+                mine = mesh_winner(h, gl);
+                if (mine) d = mesh_hit_distance(a.M, xb, h, nrm) + a.in.col_th;
+            }
+        }
+        if (mine) { s_hit[0][g] = d; s_hit[1][g] = nrm.x; s_hit[2][g] = nrm.y; s_hit[3][g] = nrm.z; }
+        __syncthreads();   // the stacks are done with: their room holds the columns
+        if (tid < 64) {
+            const bool have = s_hit[0][lane] < 0.0;
+            const uint64_t bal = __ballot(have);
+            const int m = __popcll(bal);
+            if (have) s_idx[__popcll(bal & ((1ull << lane) - 1ull))] = lane;
+            if (lane == 0) s_m = m;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (m > 0) {
+                const int at = s_idx[min(lane, m - 1)];   // lanes past the last repeat it; their rows are not summed
+                const int64_t j = base + at;
+                ContactFwd<double> c;
+                double x[3], p6[12];
+                body2_point(a.in, a.xi[3 * j], a.xi[3 * j + 1], a.xi[3 * j + 2], x);
+                c.xi1 = mk3<double>(a.xi[3 * j], a.xi[3 * j + 1], a.xi[3 * j + 2]);
+                c.x = mk3<double>(x[0], x[1], x[2]);
+                c.d = s_hit[0][at];
+                c.g = mk3<double>(s_hit[1][at], s_hit[2][at], s_hit[3][at]);
+#pragma unroll
+                for (int k = 0; k < 6; ++k) c.H[k] = 0.0;
+                c.slow = false;
+                contact_forward<double>(make_inst<double>(a.in), c, p6);
+                if (!p6on) {
+#pragma unroll
+                    for (int k = 0; k < 12; ++k) p6[k] = 0.0;
                 }
+                if (deriv) put_jac_row<double>(JacColumns{s.col, s_part, lane, m}, jac_inst(a.in), c, p6);
+                else put_wrench_row<double>(WaveColumns<24>{s.col, s_part, lane, m}, c, p6);
             }
         }
-        if (have) {
-            double p6[12];
-            contact_forward<double>(I, s, p6on ? p6 : nullptr);
-#pragma unroll
-            for (int k = 0; k < 12; ++k) acc[k] += s.f[k];
-            if (p6on) {
-#pragma unroll
-                for (int k = 0; k < 12; ++k) acc[12 + k] += p6[k];
-            }
-            ++cnt;
+        __syncthreads();
+        if (s_m > 0) {
+            if (tid < nrow) acc += s_part[tid];
+            cnt += s_m;
         }
-        if (deriv && __ballot(have) != 0ull) {
-            // columns of Km (jj < 12) and Dm (jj >= 12): lane r < 12 keeps row r
-            for (int jj = 0; jj < 24; ++jj) {
-                double col[12];
-#pragma unroll
-                for (int r = 0; r < 12; ++r) col[r] = 0.0;
-                if (have) contact_jvp<double>(I, s, unit_tangent<double>(jj), col);
-                const int obase = (jj < 12) ? jj : 144 + (jj - 12);
-                double mine = 0.0;
-#pragma unroll
-                for (int r = 0; r < 12; ++r) {
-                    const double v = wave_sum_f64(col[r]);
-                    mine = (lane == r) ? v : mine;
-                }
-                if (lane < 12) s_km[w][obase + 12 * lane] += mine;
-            }
-        }
+        __syncthreads();
     }
-    // per-wave column sums, then the waves in order
-    double* red = &s_red[w][0];
-#pragma unroll
-    for (int k = 0; k < NF; ++k) red[lane * NF + k] = acc[k];
-    const int wc = (int)wave_sum_f64((double)cnt);
-    __syncthreads();
-    if (lane < NF) {
-        double q[4] = {0.0, 0.0, 0.0, 0.0};
-        for (int r = 0; r < 64; r += 4)
-            for (int j = 0; j < 4; ++j) q[j] += red[(r + j) * NF + lane];
-        s_row[w][lane] = (q[0] + q[1]) + (q[2] + q[3]);
-    }
-    if (lane == 0) s_cnt[w] = wc;
-    __syncthreads();
-    double* row = a.part + (int64_t)blockIdx.x * kBvhOut;
-    for (int k = threadIdx.x; k < kBvhOut; k += 256) {
-        double v;
-        if (k < NF) v = ((s_row[0][k] + s_row[1][k]) + s_row[2][k]) + s_row[3][k];
-        else v = ((s_km[0][k - NF] + s_km[1][k - NF]) + s_km[2][k - NF]) + s_km[3][k - NF];
-        row[k] = v;
-    }
-    if (threadIdx.x == 0) a.part_cnt[blockIdx.x] = (int64_t)s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+    if (tid < kJacRow) a.part[(int64_t)blockIdx.x * kJacRow + tid] = acc;
+    if (tid == 0) a.part_cnt[blockIdx.x] = cnt;
 }
 
-// The workgroups' partial rows added in workgroup order.
-__global__ __launch_bounds__(320) void bvh_reduce_kernel(BvhForceArgs a, int nb) {
-    const int k = threadIdx.x;
-    if (k < kBvhOut) {
+// The workgroups' partial rows, added six rows apart in order and the six sums in
+// order; then Km and Dm from the block sums (zeros when not asked for).
+__global__ __launch_bounds__(1024) void bvh_reduce_kernel(BvhForceArgs a, int nb) {
+    constexpr int W = 160, G = 6;
+    static_assert(kJacRow <= W && G * W <= 1024, "six rows at a time");
+    __shared__ double s_sum[G][W], s_R[9], s_t[3];
+    __shared__ int64_t s_cnt[64];
+    const int tid = (int)threadIdx.x, g = tid / W, k = tid % W;
+    if (g < G && k < kJacRow) {
         double v = 0.0;
-        for (int b = 0; b < nb; ++b) v += a.part[(int64_t)b * kBvhOut + k];
-        a.out[k] = v;
+        int b = g;
+        for (; b + 7 * G < nb; b += 8 * G) {
+            double q[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) q[u] = a.part[(int64_t)(b + u * G) * kJacRow + k];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v += q[u];
+        }
+        for (; b < nb; b += G) v += a.part[(int64_t)b * kJacRow + k];
+        s_sum[g][k] = v;
     }
-    if (k == 0 && a.n_active) {
+    if (tid >= G * W) {   // the last wavefront
+        const int l = tid - G * W;
         int64_t c = 0;
-        for (int b = 0; b < nb; ++b) c += a.part_cnt[b];
+        for (int b = l; b < nb; b += 64) c += a.part_cnt[b];
+        s_cnt[l] = c;
+        if (l == 0) {
+            const JacInst J = jac_inst(a.in);
+#pragma unroll
+            for (int q = 0; q < 9; ++q) s_R[q] = J.R.a[q];
+            s_t[0] = J.t.x; s_t[1] = J.t.y; s_t[2] = J.t.z;
+        }
+    }
+    __syncthreads();
+    if (tid < kJacRow) {
+        double v = s_sum[0][tid];
+        for (int q = 1; q < G; ++q) v += s_sum[q][tid];
+        s_sum[0][tid] = v;
+    }
+    __syncthreads();
+    if (tid < 24) a.out[tid] = s_sum[0][tid];
+    const bool deriv = (a.flags & ATAC_EVAL_DERIV) != 0u;
+    if (tid < 288) {
+        const int m = tid / 144, row = (tid % 144) / 12, col = 12 * m + tid % 12;
+        a.out[24 + tid] = deriv ? jac_entry(&s_sum[0][24], &s_sum[0][9], s_R, s_t, row, col) : 0.0;
+    }
+    if (tid == 0 && a.n_active) {
+        int64_t c = 0;
+        for (int l = 0; l < 64; ++l) c += s_cnt[l];
         *a.n_active = c;
     }
 }
 
 hipError_t launch_mesh_distance(const MeshQueryArgs& a, hipStream_t st) {
     if (a.n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(mesh_distance_kernel, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(mesh_distance_kernel, dim3((unsigned)((a.n + 31) / 32)), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
 // ------------------------------------------------------------------ fixed scratch
 // The partial rows and contact counts of the force launches of
-// atac_bvh_force_noalloc: kBvhScratchBlocks workgroups' rows (kBvhOut doubles
+// atac_bvh_force_noalloc: kBvhMaxBlocks workgroups' rows (kJacRow doubles
 // each), then their counts (one 8-byte word each). One copy per device, held
 // until the process ends. Host code never passes `scratch` itself to a kernel
 // (on the host it names a stand-in, not device memory): it uses the address
 // hipGetSymbolAddress gave for the device, kept in g_scratch_addr.
-static __device__ __align__(256) double scratch[kBvhScratchBlocks * (kBvhOut + 1)];
+static __device__ __align__(256) double scratch[kBvhMaxBlocks * (kJacRow + 1)];
 
 namespace {
 constexpr int kScratchDevices = 64;
@@ -349,12 +486,13 @@ void* bvh_scratch_address(int device) {
     return g_scratch_addr[device];
 }
 
-hipError_t launch_bvh_force(const BvhForceArgs& a, hipStream_t st) {
+hipError_t launch_bvh_force(BvhForceArgs a, hipStream_t st) {
+    a.block_points = bvh_block_points(a.n);
     const int nb = (int)bvh_force_blocks(a.n);
-    hipLaunchKernelGGL(bvh_force_kernel, dim3(nb), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(bvh_force_kernel, dim3(nb), dim3(512), 0, st, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(bvh_reduce_kernel, dim3(1), dim3(320), 0, st, a, nb);
+    hipLaunchKernelGGL(bvh_reduce_kernel, dim3(1), dim3(1024), 0, st, a, nb);
     return hipGetLastError();
 }
 

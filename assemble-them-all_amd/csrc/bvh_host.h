@@ -12,7 +12,7 @@ namespace atac {
 struct MeshHost {
     std::vector<float4> nodes;
     std::vector<int32_t> tri, F, FE;
-    std::vector<double> V, FN, EN, VN;
+    std::vector<double> V, tv, FN, EN, VN;
     double bmin[3], bmax[3];
     int64_t ne = 0;
 };
@@ -42,20 +42,28 @@ struct BvhForceArgs {
     uint32_t flags;       // ATAC_EVAL_* (DERIV, P6)
     double* out;          // 12 fm, 12 p6, 144 Km, 144 Dm
     int64_t* n_active;
-    double* part;         // per workgroup: kBvhOut partial sums
+    double* part;         // per workgroup: kJacRow partial sums
     int64_t* part_cnt;    // per workgroup: contacts
+    int64_t block_points; // points per workgroup, a multiple of kBvhStep
 };
 constexpr int kBvhOut = 12 + 12 + 288;
-constexpr int kBvhBlockPoints = 2048;   // points per force workgroup
-inline int64_t bvh_force_blocks(int64_t n) { return n > 0 ? (n + kBvhBlockPoints - 1) / kBvhBlockPoints : 1; }
+
+// A force workgroup takes kBvhStep points at a time, 8 lanes each; one step per
+// workgroup as long as kBvhMaxBlocks workgroups (two per CU) cover the points.
+constexpr int kBvhStep = 64;
+constexpr int64_t kBvhMaxBlocks = 512;
+inline int64_t bvh_block_points(int64_t n) {
+    const int64_t steps = (n + kBvhStep - 1) / kBvhStep;
+    return kBvhStep * (steps > kBvhMaxBlocks ? (steps + kBvhMaxBlocks - 1) / kBvhMaxBlocks : 1);
+}
+inline int64_t bvh_force_blocks(int64_t n) { return n > 0 ? (n + bvh_block_points(n) - 1) / bvh_block_points(n) : 1; }
 
 hipError_t launch_mesh_distance(const MeshQueryArgs& a, hipStream_t st);
-hipError_t launch_bvh_force(const BvhForceArgs& a, hipStream_t st);
+hipError_t launch_bvh_force(BvhForceArgs a, hipStream_t st);
 
-// Fixed scratch of atac_bvh_force_noalloc: room for the partial rows and counts of
-// kBvhScratchBlocks force workgroups (kBvhNoAllocMaxPoints points), per device.
+// Fixed scratch of atac_bvh_force_noalloc: the partial rows and counts of the at
+// most kBvhMaxBlocks force workgroups of a call, per device.
 constexpr int64_t kBvhNoAllocMaxPoints = (int64_t)1 << 20;
-constexpr int64_t kBvhScratchBlocks = kBvhNoAllocMaxPoints / kBvhBlockPoints;
 // Looks up the device's copy of the scratch array; `device` must be current.
 // Idempotent per device.
 hipError_t bvh_scratch_setup(int device);
