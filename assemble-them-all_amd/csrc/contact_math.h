@@ -987,7 +987,7 @@ ATAC_HD void contact_sample(const GridDev& G, const InstDev& in, double px, doub
     double fd[3];
     if (sizeof(R) == sizeof(double) && fast_cell(G, x, idx, f, fd)) {
         // FP64 contact path: value and partials in FP64 from the same corners
-        Corners c = load_corners(G, idx[0], idx[1], idx[2]);
+        Corners c = G.fast ? load_cell(G, idx[0], idx[1], idx[2]) : load_corners(G, idx[0], idx[1], idx[2]);
         double val, g[3], H[6];
         sdf_cell64(G, c, fd, val, g, H);
         val += in.col_th;
@@ -996,7 +996,7 @@ ATAC_HD void contact_sample(const GridDev& G, const InstDev& in, double px, doub
         for (int k = 0; k < 6; ++k) s.H[k] = (R)H[k];
         s.slow = false;
     } else if (fast_cell(G, x, idx, f, fd)) {
-        Corners c = load_corners(G, idx[0], idx[1], idx[2]);
+        Corners c = G.fast ? load_cell(G, idx[0], idx[1], idx[2]) : load_corners(G, idx[0], idx[1], idx[2]);
         float val, g[3], H[6];
         sdf_cell32(G, c, f, val, g, H);
         // the penetration depth of an active contact is taken in FP64 from the
