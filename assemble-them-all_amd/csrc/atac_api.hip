@@ -1453,12 +1453,15 @@ int atac_sdf_from_mesh(const float* x, int64_t nv, const uint32_t* tri, int64_t 
     uint32_t* d_tri = nullptr;
     unsigned long long* d_best = nullptr;
     float* d_phi = nullptr;
-    int32_t *d_closest = nullptr, *d_count = nullptr;
+    ls::Tri* d_tris = nullptr;
+    int32_t *d_sync = nullptr, *d_count = nullptr;
+    int32_t gave_up = 0;
     int rc = dalloc(&d_x, (size_t)std::max<int64_t>(3 * nv, 1));
     if (!rc) rc = dalloc(&d_tri, (size_t)std::max<int64_t>(3 * nf, 1));
     if (!rc) rc = dalloc(&d_best, (size_t)n);
     if (!rc) rc = dalloc(&d_phi, (size_t)n);
-    if (!rc) rc = dalloc(&d_closest, (size_t)n);
+    if (!rc) rc = dalloc(&d_tris, (size_t)std::max<int64_t>(nf, 1));
+    if (!rc) rc = dalloc(&d_sync, kLsSync);
     if (!rc) rc = dalloc(&d_count, (size_t)n);
     hipError_t e = hipSuccess;
     if (!rc && nv > 0) e = hipMemcpy(d_x, x, sizeof(float) * 3 * nv, hipMemcpyHostToDevice);
@@ -1466,11 +1469,13 @@ int atac_sdf_from_mesh(const float* x, int64_t nv, const uint32_t* tri, int64_t 
     if (!rc && e == hipSuccess) e = hipMemset(d_best, 0xff, sizeof(unsigned long long) * n);
     if (!rc && e == hipSuccess) e = hipMemset(d_count, 0, sizeof(int32_t) * n);
     if (!rc && e == hipSuccess) {
-        a.x = d_x; a.tri = d_tri; a.best = d_best; a.phi = d_phi; a.closest = d_closest; a.count = d_count;
+        a.x = d_x; a.tri = d_tri; a.best = d_best; a.phi = d_phi; a.tris = d_tris; a.sync = d_sync; a.count = d_count;
         e = ls_build(a, nullptr);
         if (e == hipSuccess) e = hipMemcpy(phi, d_phi, sizeof(float) * n, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) e = hipMemcpy(&gave_up, d_sync + kLsGaveUp, sizeof gave_up, hipMemcpyDeviceToHost);
+        if (e == hipSuccess && gave_up) rc = fail(ATAC_ERR_HIP, "atac_sdf_from_mesh: a sweep waited for its neighbour in vain");
     }
-    dfree(d_x); dfree(d_tri); dfree(d_best); dfree(d_phi); dfree(d_closest); dfree(d_count);
+    dfree(d_x); dfree(d_tri); dfree(d_best); dfree(d_phi); dfree(d_tris); dfree(d_sync); dfree(d_count);
     if (rc) return rc;
     if (e != hipSuccess) return fail(ATAC_ERR_HIP, hipGetErrorString(e));
     return ATAC_OK;

@@ -68,6 +68,67 @@ ATAC_HD float tri_dist(const F3& x0, const F3& x1, const F3& x2, const F3& x3) {
     return lmin(distf(x0, seg_closest(x0, x1, a1)), distf(x0, seg_closest(x0, b0, x3)));
 }
 
+// What tri_dist needs of a triangle besides its vertices, formed once per triangle
+// by the same operations: 80 bytes.
+struct Tri {
+    F3 x1;
+    float m13;
+    F3 x2;
+    float m23;
+    F3 x3;
+    float d;
+    float invdet, m12;
+    double r12, r13, r23;   // 1 / squared edge length
+};
+static_assert(sizeof(Tri) == 80, "five 16-byte reads");
+ATAC_HD Tri make_tri(const F3& x1, const F3& x2, const F3& x3) {
+    Tri t;
+    const F3 x13 = sub(x1, x3), x23 = sub(x2, x3);
+    t.x1 = x1; t.x2 = x2; t.x3 = x3;
+    t.m13 = mag2(x13); t.m23 = mag2(x23); t.d = dotf(x13, x23);
+    t.invdet = 1.0f / lmax(t.m13 * t.m23 - t.d * t.d, 1e-30f);
+    t.m12 = mag2(sub(x2, x1));
+    t.r12 = 1.0 / (double)t.m12; t.r13 = 1.0 / (double)t.m13; t.r23 = 1.0 / (double)t.m23;
+    return t;
+}
+
+// The squared length of seg_closest's offset. Its parameter is a FP64 quotient
+// rounded to FP32: the product with the reciprocal is within 2^-51 of that quotient,
+// so when both ends of a 2^-50 band around it round to one FP32 value, that is the
+// parameter; otherwise (about one in 2^26, and zero-length edges) it is divided out.
+ATAC_HD float seg_mag2(const F3& x0, const F3& x1, const F3& x2, float m2, double r) {
+    const F3 d = sub(x2, x1);
+    const double p = (double)dotf(sub(x2, x0), d), q = p * r;
+    const float lo = (float)(q * (1.0 - 0x1p-50)), hi = (float)(q * (1.0 + 0x1p-50));
+    float s = lo == hi ? lo : (float)(p / (double)m2);
+    s = s < 0.0f ? 0.0f : (s > 1.0f ? 1.0f : s);
+    return mag2(sub(x0, add(scale(s, x1), scale(1.0f - s, x2))));
+}
+
+// tri_dist(x0, t) if it can be below p, else infinity: the same bits where it
+// matters. The nearer of two edges is chosen by the squared lengths (the rounded
+// square root is monotonic), and the root is left out when the square exceeds p^2 by
+// more than its rounding (2^-24) can hide.
+ATAC_HD float tri_dist_below(const F3& x0, const Tri& t, float p) {
+    const F3 x13 = sub(t.x1, t.x3), x23 = sub(t.x2, t.x3), x03 = sub(x0, t.x3);
+    const float a = dotf(x13, x03), b = dotf(x23, x03);
+    const float w23 = t.invdet * (t.m23 * a - t.d * b);
+    const float w31 = t.invdet * (t.m13 * b - t.d * a);
+    const float w12 = 1.0f - w23 - w31;
+    float s;
+    if (w23 >= 0.0f && w31 >= 0.0f && w12 >= 0.0f) {
+        s = mag2(sub(x0, add(add(scale(w23, t.x1), scale(w31, t.x2)), scale(w12, t.x3))));
+    } else {
+        const bool p23 = w23 > 0.0f, p31 = w31 > 0.0f;   // edges 1-2 and 1-3; 1-2 and 2-3; 1-3 and 2-3
+        const bool first12 = p23 || p31;
+        const float s1 = seg_mag2(x0, t.x1, first12 ? t.x2 : t.x3, first12 ? t.m12 : t.m13, first12 ? t.r12 : t.r13);
+        const float s2 = seg_mag2(x0, p23 ? t.x1 : t.x2, t.x3, p23 ? t.m13 : t.m23, p23 ? t.r13 : t.r23);
+        s = lmin(s1, s2);
+    }
+    if (s > p * p * 1.000001f) return INFINITY;
+    return sqrtf(s);
+}
+
 // sign of the doubled area of (0,0)-(x1,y1)-(x2,y2), ties broken by the
 // coordinates (0 only for a degenerate triangle)
 ATAC_HD int orientation(double x1, double y1, double x2, double y2, double& area2) {

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include "levelset.h"
 
 namespace atac {
 
@@ -14,14 +15,19 @@ struct LsArgs {
     int32_t ni, nj, nk;
     int32_t band;             // exact band, in cells
     float phi0;               // initial (upper-bound) distance
-    unsigned long long* best; // per node: (distance bits << 32) | triangle, min over the band
+    // per node, first (distance bits << 32) | triangle, the band's minimum; then the
+    // sweeps' state: (tag << 32) | word, see ls_sweep_kernel
+    unsigned long long* best;
     float* phi;               // per node: distance, then signed distance
-    int32_t* closest;         // per node: closest triangle so far (-1: none)
+    ls::Tri* tris;            // per triangle: its vertices and what its distances share
     int32_t* count;           // per node: x-ray crossings in (i - 1, i]
+    int32_t* sync;            // kLsSync words: tiles handed out per sweep, and the give-up flag
 };
+constexpr int kLsSweeps = 16, kLsGaveUp = kLsSweeps, kLsSync = kLsSweeps + 1;
 
 // Launches the whole construction on `st`: band distances and crossing counts,
-// 2 x 8 fast-sweeping passes (one launch per diagonal plane), signs.
+// 2 x 8 fast-sweeping passes (one launch each), signs. sync[kLsGaveUp] is set when
+// a sweep waited for a neighbour in vain (its values are then wrong).
 hipError_t ls_build(const LsArgs& a, hipStream_t st);
 
 }  // namespace atac
