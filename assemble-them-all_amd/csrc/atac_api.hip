@@ -2,6 +2,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -104,9 +106,13 @@ struct atac_batch_s {
     int32_t* d_tile_active = nullptr;
     uint32_t* d_tile_live = nullptr;  // per tile: the groups the culling pass keeps
     bool last_culled = false;         // the last evaluation enqueued ran the culling pass
+    bool one_per_instance = false;    // the plan allows instance_kernel
+    int64_t most_points = 0;          // of an instance
+    int32_t host_call = 0;            // calls of atac_batch_eval_instances_host so far
+    int32_t chunk_total = 0;          // work items if every point were a contact
     int32_t* d_tile_chunk0 = nullptr;
     ChunkDev* d_chunks = nullptr;
-    int32_t* d_counters = nullptr;    // CNT_WORDS
+    int32_t* d_counters = nullptr;    // CNT_ALL
     // per-evaluation buffers, allocated on first use
     uint32_t* d_act = nullptr;        // rec_cap: active point offsets, a tile's in one range
     Rec32* d_rec32 = nullptr;         // rec_cap
@@ -134,7 +140,8 @@ struct atac_batch_s {
     double* h_grad = nullptr;     // 26 per instance
     // pinned host staging of the host-buffer entry points' results: the device-to-host
     // copies run as DMA without the runtime's pageable staging, then one wait
-    char* pin = nullptr;          // 312 doubles per instance | n_active per instance | overflow flag
+    char* pin = nullptr;          // 312 doubles per instance | n_active per instance | overflow flag | number of
+                                  // the finished call per instance | number of the call
     InstDev* pin_inst = nullptr;  // pinned instance records for atac_batch_eval_instances_host
     // graphs of atac_batch_eval_instances_host per flag combination, valid while no device
     // buffer has been (re)allocated since their capture (buf_gen)
@@ -404,6 +411,16 @@ static void compose_for(atac_batch b, const atac_instance& s, InstDev& d) {
     d.gbox = P.d_gbox ? P.d_gbox + 8 * P.gseg[s.segment] : nullptr;
 }
 
+// The same for an instance of a planned batch: its place in the plan stays.
+static void recompose(atac_batch b, int i, const atac_instance& s) {
+    InstDev& d = b->inst_dev[i];
+    const int32_t tb = d.tile_begin, tc = d.tile_count, c0 = d.chunk0;
+    compose_for(b, s, d);
+    d.tile_begin = tb;
+    d.tile_count = tc;
+    d.chunk0 = c0;
+}
+
 // A classification table for every (grid, col_th) the instances use, built on
 // first use (synchronously) and set in their device records; tables no longer
 // used are freed once the device is idle.
@@ -486,7 +503,8 @@ static int ensure_buffers(atac_batch b, int mode, bool precise) {
         if (!rc && precise && !b->d_rec64) rc = dalloc(&b->d_rec64, (size_t)b->rec_cap);
         if (!rc && !precise && !b->d_rec32) rc = dalloc(&b->d_rec32, (size_t)b->rec_cap);
         if (!rc && !b->d_slow) rc = dalloc(&b->d_slow, (size_t)b->slow_cap);
-        if (!rc && !precise && !b->d_slow_diag) rc = dalloc(&b->d_slow_diag, (size_t)b->slow_cap * 4);
+        if (!rc && !precise && !b->d_slow_diag)
+            rc = dalloc(&b->d_slow_diag, (size_t)(b->one_per_instance ? b->rec_cap : b->slow_cap) * 4);
         const void* after[5] = {b->d_act, b->d_rec64, b->d_rec32, b->d_slow, b->d_slow_diag};
         for (int k = 0; k < 5; ++k) b->buf_gen += before[k] != after[k];
     }
@@ -511,6 +529,13 @@ static int ensure_buffers(atac_batch b, int mode, bool precise) {
 static int wave_span_of(int tile_points, int block) {
     const int nw = block / 64, ng = (tile_points + kGroup - 1) / kGroup;
     return (ng + nw - 1) / nw * kGroup;
+}
+
+static bool default_tuning(const atac_tuning& t) {
+    const atac_tuning zero{};
+    return t.tile_points == zero.tile_points && t.detect_block == zero.detect_block && t.blocks_per_cu == zero.blocks_per_cu &&
+           t.order == zero.order && t.points_per_lane == zero.points_per_lane && t.max_active == zero.max_active &&
+           t.group_cull == zero.group_cull;
 }
 
 static int plan(atac_batch b, const atac_tuning* t) {
@@ -550,6 +575,7 @@ static int plan(atac_batch b, const atac_tuning* t) {
     for (size_t i = 0; i < b->inst_dev.size(); ++i) {
         InstDev& d = b->inst_dev[i];
         d.tile_begin = (int32_t)b->tiles.size();
+        d.chunk0 = (int32_t)chunks;
         for (int64_t o = 0; o < d.pt_count; o += T) {
             TileDev td;
             td.inst = (int32_t)i;
@@ -576,6 +602,15 @@ static int plan(atac_batch b, const atac_tuning* t) {
     // work items: at most one partial item per tile beyond the full ones of the pool
     b->chunk_cap = std::min<int64_t>(chunks, b->rec_cap / kChunk + b->tiles.size());
     b->n_tiles = (int32_t)b->tiles.size();
+    b->chunk_total = (int32_t)std::min<int64_t>(chunks, INT32_MAX);
+    // one workgroup per instance (instance_kernel): default plans of small instances, as
+    // many as the GPU holds at once (two per CU); with 1,024 instances of 500 points the
+    // pipeline's finer pieces fill it better (37 us against 42; 512: 34 against 25)
+    b->one_per_instance = (!t || default_tuning(*t)) && b->rec_cap == slot && b->inst_dev.size() <= (size_t)(2 * b->n_cu) &&
+                          T >= inst_points(0);
+    b->most_points = 0;
+    for (const InstDev& d : b->inst_dev) b->most_points = std::max(b->most_points, (int64_t)d.pt_count);
+    b->one_per_instance = b->one_per_instance && b->most_points <= inst_points(0);
     // tile queues: 1 = one queue in instance order; 2 = one queue grouped by grid;
     // 3 = grouped by grid and cut into one queue per XCD with balanced point counts;
     // 4 = one queue per XCD by the tile's place in its instance's point order: a
@@ -618,13 +653,13 @@ static int plan(atac_batch b, const atac_tuning* t) {
     int rc = dalloc(&b->d_tiles, b->n_tiles);
     if (!rc) rc = dalloc(&b->d_order, b->n_tiles);
     if (!rc) rc = dalloc(&b->d_tq_begin, b->nq + 1);
-    if (!rc) rc = dalloc(&b->d_counters, CNT_WORDS);
+    if (!rc) rc = dalloc(&b->d_counters, CNT_ALL);
     if (!rc) rc = dalloc(&b->d_tile_active, b->n_tiles);
     if (!rc) rc = dalloc(&b->d_tile_live, b->n_tiles);
     if (!rc) rc = dalloc(&b->d_tile_chunk0, b->n_tiles);
     if (!rc) rc = dalloc(&b->d_chunks, (size_t)b->chunk_cap);
     if (rc) return rc;
-    ATAC_HIP(hipMemset(b->d_counters, 0, sizeof(int32_t) * CNT_WORDS));   // no stale work-item count before the first evaluation
+    ATAC_HIP(hipMemset(b->d_counters, 0, sizeof(int32_t) * CNT_ALL));   // no stale work-item count before the first evaluation
     ATAC_HIP(hipMemcpy(b->d_tq_begin, tq.data(), sizeof(int32_t) * tq.size(), hipMemcpyHostToDevice));
     if (b->n_tiles > 0) {
         ATAC_HIP(hipMemcpy(b->d_tiles, b->tiles.data(), sizeof(TileDev) * b->n_tiles, hipMemcpyHostToDevice));
@@ -713,6 +748,7 @@ int atac_batch_create(const atac_grid* grids, int32_t n_grids, const atac_points
 
 int atac_batch_destroy(atac_batch b) {
     if (!b) return ATAC_OK;
+    if (b->cap_stream) (void)hipStreamSynchronize(b->cap_stream);   // a host call returns before its graph has ended
     release_plan(b);
     for (auto& u : b->ev_used) { (void)hipEventDestroy(u.second.first); (void)hipEventDestroy(u.second.second); }
     for (auto e : b->ev_pool) (void)hipEventDestroy(e);
@@ -739,10 +775,7 @@ int atac_batch_set_instances(atac_batch b, const atac_instance* inst, int32_t n_
     int rc = check_instances(b, inst, n_inst);
     if (rc) return rc;
     for (int i = 0; i < n_inst; ++i) {
-        const int32_t tb = b->inst_dev[i].tile_begin, tc = b->inst_dev[i].tile_count;
-        compose_for(b, inst[i], b->inst_dev[i]);
-        b->inst_dev[i].tile_begin = tb;
-        b->inst_dev[i].tile_count = tc;
+        recompose(b, i, inst[i]);
     }
     rc = ensure_cls(b);   // a new col_th needs its classification table
     if (rc) return rc;
@@ -791,12 +824,41 @@ static QueueDev tile_queues(atac_batch b) {
 
 static int32_t* counters(atac_batch b) { return b->d_counters; }
 
+// What an enqueued evaluation leaves for the adjoint.
+static int eval_done(atac_batch b, bool fused, bool precise, hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    ATAC_HIP(hipStreamIsCapturing(st, &cs));
+    if (fused) {
+        // the fast-path records were not written: nothing for atac_batch_vjp
+        b->rec_valid = false;
+        if (cs != hipStreamCaptureStatusNone) b->rec_captured = false;
+    } else if (cs == hipStreamCaptureStatusNone) {
+        b->rec_valid = true;
+        b->rec_precise = precise;
+    } else {
+        // recorded only: the records exist once the graph has run (atac_batch_graph_launch)
+        b->rec_valid = false;
+        b->rec_captured = true;
+        b->cap_precise = precise;
+    }
+    return ATAC_OK;
+}
+
+// Does an evaluation with these flags run one workgroup per instance?
+// A Km/Dm workgroup holds its CU alone (registers), so two rounds of instances take
+// twice as long: 512 instances of 500 points take 37 us against the pipeline's 39, of
+// 2,000 points 60 against 45; 256 of them 22 against 34 and 41 against 39.
+static bool takes_one_per_instance(atac_batch b, uint32_t flags) {
+    return b->one_per_instance && !(flags & ATAC_EVAL_ALL_ACTIVE) && b->n_tiles > 0 &&
+           b->most_points <= inst_points(mode_of(flags)) && (mode_of(flags) < 2 || b->inst.size() <= (size_t)b->n_cu);
+}
+
 // overflow_out (optional) receives the evaluation's overflow flag from the reduction.
 // g_fused != nullptr: the fused pass (ATAC_EVAL_FUSED_ADJOINT), the wrench and the
 // adjoint of g_fused into out and gg, no records kept.
 static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, hipStream_t st,
                         int32_t* overflow_out = nullptr, const double* g_fused = nullptr,
-                        const atac_gradients* gg = nullptr) {
+                        const atac_gradients* gg = nullptr, int32_t* done = nullptr) {
     if (flags & ~(ATAC_EVAL_DERIV | ATAC_EVAL_P6 | ATAC_EVAL_CHECKPOINT | ATAC_EVAL_PRECISE | ATAC_EVAL_ALL_ACTIVE |
                   (g_fused ? ATAC_EVAL_FUSED_ADJOINT : 0u)))
         return fail(ATAC_ERR_INVALID, "atac_batch_eval: unknown flag");
@@ -816,7 +878,20 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
     // groups whose boxes reach only cells where no point can be active are dropped
     // first; that pass also clears the counters (all points are contacts with
     // ATAC_EVAL_ALL_ACTIVE: nothing is dropped)
-    const bool cull = b->tune.group_cull > 0 && !(flags & ATAC_EVAL_ALL_ACTIVE) && b->n_tiles > 0;
+    const bool one = !fused && !b->timing && takes_one_per_instance(b, flags);   // (stage times need the stages)
+    const bool cull = !one && b->tune.group_cull > 0 && !(flags & ATAC_EVAL_ALL_ACTIVE) && b->n_tiles > 0;
+    b->last_culled = cull;
+    if (one) {
+        InstanceArgs ia{};
+        ia.inst = b->d_inst; ia.grids = b->d_grids; ia.tiles = b->d_tiles;
+        ia.chunk_total = b->chunk_total; ia.act = b->d_act; ia.rec = rec; ia.slow_diag = b->d_slow_diag;
+        ia.tile_active = b->d_tile_active; ia.tile_chunk0 = b->d_tile_chunk0; ia.chunks = b->d_chunks;
+        ia.counters = counters(b);
+        if (out) { ia.fm = out->fm; ia.p6 = out->dfm_dp6; ia.Km = out->Km; ia.Dm = out->Dm; ia.n_active = out->n_active; }
+        ia.overflow_out = overflow_out; ia.host_dst = overflow_out ? 1 : 0; ia.done = done;
+        ATAC_HIP(launch_instance(ia, mode, precise, (int)b->inst.size(), st));
+        return eval_done(b, false, precise, st);
+    }
     if (!cull) ATAC_HIP(launch_reset(b->d_counters, CNT_WORDS, st));
     if (b->n_tiles > 0) {
         DetectArgs da{};
@@ -828,7 +903,6 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
         da.tile_active = b->d_tile_active; da.tile_chunk0 = b->d_tile_chunk0; da.chunks = b->d_chunks;
         da.slow = b->d_slow; da.counters = counters(b);
         da.tile_live = cull ? b->d_tile_live : nullptr;
-        b->last_culled = cull;
         hipEvent_t t0 = stage_begin(b, st);
         if (cull) {
             CullArgs cu{};
@@ -880,26 +954,12 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
     ra.n_active = out ? out->n_active : nullptr;
     ra.counters = counters(b);
     ra.overflow_out = overflow_out;
-    ra.host_dst = overflow_out ? 1 : 0;   // the small-batch graph's outputs are its pinned staging
+    ra.host_dst = overflow_out ? 1 : 0;   // the host call's outputs are its pinned staging
+    ra.done = done;
     hipEvent_t t3 = stage_begin(b, st);
     ATAC_HIP(mode == 2 ? launch_reduce_jacobian(ra, st) : launch_reduce(ra, st));
     stage_end(b, ST_REDUCE, t3, st);
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    ATAC_HIP(hipStreamIsCapturing(st, &cs));
-    if (fused) {
-        // the fast-path records were not written: nothing for atac_batch_vjp
-        b->rec_valid = false;
-        if (cs != hipStreamCaptureStatusNone) b->rec_captured = false;
-    } else if (cs == hipStreamCaptureStatusNone) {
-        b->rec_valid = true;
-        b->rec_precise = precise;
-    } else {
-        // recorded only: the records exist once the graph has run (atac_batch_graph_launch)
-        b->rec_valid = false;
-        b->rec_captured = true;
-        b->cap_precise = precise;
-    }
-    return ATAC_OK;
+    return eval_done(b, fused, precise, st);
 }
 
 // The adjoint of the last evaluation that has run (or, while capturing, of the
@@ -1174,7 +1234,14 @@ int atac_batch_workspace(atac_batch b, int64_t* capacity, int64_t* used, int32_t
     ATAC_HIP(hipDeviceSynchronize());
     ATAC_HIP(hipMemcpy(c, b->d_counters, sizeof c, hipMemcpyDeviceToHost));
     if (capacity) *capacity = b->rec_cap;
-    if (used) *used = c[CNT_RECS];
+    int64_t n = c[CNT_RECS];
+    if (n == 0) {   // no contacts, or instance_kernel, which leaves the counts per tile only
+        std::vector<int32_t> act(b->n_tiles);
+        if (b->n_tiles) ATAC_HIP(hipMemcpy(act.data(), b->d_tile_active, sizeof(int32_t) * act.size(), hipMemcpyDeviceToHost));
+        n = 0;
+        for (int32_t v : act) n += v;
+    }
+    if (used) *used = n;
     if (overflowed) *overflowed = c[CNT_OVERFLOW] != 0 ? 1 : 0;
     return ATAC_OK;
 }
@@ -1228,14 +1295,46 @@ static int ensure_staging(atac_batch b) {
     if (!rc && !b->h_gfm) rc = dalloc(&b->h_gfm, n * 12);
     if (!rc && !b->h_grad) rc = dalloc(&b->h_grad, n * kVjpOut);
     if (!rc && !b->pin) {
-        const hipError_t e = hipHostMalloc((void**)&b->pin, n * (312 * sizeof(double) + sizeof(int32_t)) + 16,
+        const hipError_t e = hipHostMalloc((void**)&b->pin, n * (312 * sizeof(double) + 2 * sizeof(int32_t)) + 16,
                                            hipHostMallocDefault);
         if (e != hipSuccess) {
             b->pin = nullptr;
             rc = fail(ATAC_ERR_NOMEM, std::string("pinned staging: ") + hipGetErrorString(e));
+        } else {
+            std::memset(b->pin, 0, n * (312 * sizeof(double) + 2 * sizeof(int32_t)) + 16);   // no call is 0
         }
     }
     return rc;
+}
+
+// Waits until every instance's word in `done` holds the call's number (the device
+// writes it behind the instance's results), or, after two milliseconds, for the stream.
+static int wait_done(atac_batch b, const volatile int32_t* done, int32_t call, hipStream_t st) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (size_t i = 0; i < b->inst.size(); ++i)
+        for (uint32_t spins = 1; done[i] != call; ++spins)
+            if ((spins & 1023u) == 0u && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+                ATAC_HIP(hipStreamSynchronize(st));
+                if (done[i] != call) return fail(ATAC_ERR_HIP, "atac_batch_eval_instances_host: no result");
+                break;
+            }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return ATAC_OK;
+}
+
+// The pinned staging's results (fm | p6 | Km | Dm; n_active | overflow flag) to the caller.
+static int host_results(atac_batch b, const double* P, const int32_t* Pn, double* fm, double* Km, double* Dm, double* dfm_dp6,
+                        int32_t* n_active, const char* who) {
+    const size_t n = b->inst.size();
+    if (fm) std::memcpy(fm, P, sizeof(double) * 12 * n);
+    if (dfm_dp6) std::memcpy(dfm_dp6, P + 12 * n, sizeof(double) * 12 * n);
+    if (Km) std::memcpy(Km, P + 24 * n, sizeof(double) * 144 * n);
+    if (Dm) std::memcpy(Dm, P + 168 * n, sizeof(double) * 144 * n);
+    if (n_active) std::memcpy(n_active, Pn, sizeof(int32_t) * n);
+    if (Pn[n])
+        return fail(ATAC_ERR_NOMEM, std::string(who) + ": more active contacts than the record pool holds (" +
+                                        std::to_string(b->rec_cap) + "); plan the batch with a larger max_active");
+    return ATAC_OK;
 }
 
 int atac_batch_eval_host(atac_batch b, uint32_t flags, double* fm, double* Km, double* Dm, double* dfm_dp6,
@@ -1264,16 +1363,7 @@ int atac_batch_eval_host(atac_batch b, uint32_t flags, double* fm, double* Km, d
     ATAC_HIP(hipMemcpyAsync(Pn, o.n_active, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st));
     ATAC_HIP(hipMemcpyAsync(Pn + n, b->d_counters + CNT_OVERFLOW, sizeof(int32_t), hipMemcpyDeviceToHost, st));
     ATAC_HIP(hipStreamSynchronize(st));
-    if (fm) std::memcpy(fm, P, sizeof(double) * 12 * n);
-    if (dfm_dp6) std::memcpy(dfm_dp6, P + 12 * n, sizeof(double) * 12 * n);
-    if (Km) std::memcpy(Km, P + 24 * n, sizeof(double) * 144 * n);
-    if (Dm) std::memcpy(Dm, P + 168 * n, sizeof(double) * 144 * n);
-    if (n_active) std::memcpy(n_active, Pn, sizeof(int32_t) * n);
-    const int32_t ovf = Pn[n];
-    if (ovf)
-        return fail(ATAC_ERR_NOMEM, "atac_batch_eval_host: more active contacts than the record pool holds (" +
-                                        std::to_string(b->rec_cap) + "); plan the batch with a larger max_active");
-    return ATAC_OK;
+    return host_results(b, P, Pn, fm, Km, Dm, dfm_dp6, n_active, "atac_batch_eval_host");
 }
 
 int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int32_t n_inst, uint32_t flags, double* fm,
@@ -1293,10 +1383,7 @@ int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int3
     int rc = check_instances(b, inst, n_inst);
     if (rc) return rc;
     for (int i = 0; i < n_inst; ++i) {
-        const int32_t tb = b->inst_dev[i].tile_begin, tc = b->inst_dev[i].tile_count;
-        compose_for(b, inst[i], b->inst_dev[i]);
-        b->inst_dev[i].tile_begin = tb;
-        b->inst_dev[i].tile_count = tc;
+        recompose(b, i, inst[i]);
     }
     rc = ensure_cls(b);
     if (rc) return rc;
@@ -1316,27 +1403,44 @@ int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int3
     }
     double* P = reinterpret_cast<double*>(b->pin);
     int32_t* Pn = reinterpret_cast<int32_t*>(b->pin + n * 312 * sizeof(double));
+    hipStream_t st = b->cap_stream;
+    atac_outputs o{};
+    o.fm = P;
+    o.dfm_dp6 = dfm_dp6 ? P + 12 * n : nullptr;
+    o.Km = (Km || Dm) ? P + 24 * n : nullptr;
+    o.Dm = (Km || Dm) ? P + 168 * n : nullptr;
+    o.n_active = Pn;
+    // the kernel that writes an instance's results into host memory writes the call's
+    // number behind them; the host watches for those numbers, which come several
+    // microseconds before the stream counts as idle
+    int32_t* done = Pn + n + 1;
+    int32_t* call = done + n;
+    std::memcpy(b->pin_inst, b->inst_dev.data(), sizeof(InstDev) * n);   // the previous call has finished with it
+    *call = ++b->host_call;
+    if (takes_one_per_instance(b, flags)) {   // two launches: no graph
+        const bool timing = b->timing;
+        b->timing = false;
+        ATAC_HIP(launch_upload(b->pin_inst, b->d_inst, (int)n, call, b->d_counters, st));
+        rc = enqueue_eval(b, flags, &o, st, Pn + n, nullptr, nullptr, done);
+        b->timing = timing;
+        if (rc) (void)hipStreamSynchronize(st);
+        else rc = wait_done(b, done, *call, st);
+        return rc ? rc : host_results(b, P, Pn, fm, Km, Dm, dfm_dp6, n_active, "atac_batch_eval_instances_host");
+    }
     const uint32_t key = flags | ((Km || Dm) ? 1u << 8 : 0u) | (dfm_dp6 ? 1u << 9 : 0u);
     atac_batch_s::HostGraph& hg = b->host_graphs[key];
-    hipStream_t st = b->cap_stream;
     if (!hg.e || hg.gen != b->buf_gen) {
         // capture: instance upload and evaluation, whose reduction writes the results
         // and the overflow flag straight into the pinned staging (no stage timing inside)
+        ATAC_HIP(hipStreamSynchronize(st));
         if (hg.e) (void)hipGraphExecDestroy(hg.e);
         if (hg.g) (void)hipGraphDestroy(hg.g);
         hg = atac_batch_s::HostGraph{};
-        ATAC_HIP(hipStreamSynchronize(st));
         const bool timing = b->timing, rc_cap = b->rec_captured, cp = b->cap_precise;
         b->timing = false;
-        atac_outputs o{};
-        o.fm = P;
-        o.dfm_dp6 = dfm_dp6 ? P + 12 * n : nullptr;
-        o.Km = (Km || Dm) ? P + 24 * n : nullptr;
-        o.Dm = (Km || Dm) ? P + 168 * n : nullptr;
-        o.n_active = Pn;
         ATAC_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        hipError_t e = hipMemcpyAsync(b->d_inst, b->pin_inst, sizeof(InstDev) * n, hipMemcpyHostToDevice, st);
-        if (e == hipSuccess) rc = enqueue_eval(b, flags, &o, st, Pn + n);
+        hipError_t e = launch_upload(b->pin_inst, b->d_inst, (int)n, call, b->d_counters, st);
+        if (e == hipSuccess) rc = enqueue_eval(b, flags, &o, st, Pn + n, nullptr, nullptr, done);
         hipGraph_t g = nullptr;
         const hipError_t e2 = hipStreamEndCapture(st, &g);
         b->timing = timing;
@@ -1351,20 +1455,12 @@ int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int3
         ATAC_HIP(hipGraphInstantiate(&hg.e, hg.g, nullptr, nullptr, 0));
         hg.gen = b->buf_gen;
     }
-    std::memcpy(b->pin_inst, b->inst_dev.data(), sizeof(InstDev) * n);   // the previous call has finished with it
     ATAC_HIP(hipGraphLaunch(hg.e, st));
-    ATAC_HIP(hipStreamSynchronize(st));
+    rc = wait_done(b, done, *call, st);
+    if (rc) return rc;
     b->rec_valid = true;   // the replay left its records for atac_batch_vjp
     b->rec_precise = (flags & ATAC_EVAL_PRECISE) != 0;
-    if (fm) std::memcpy(fm, P, sizeof(double) * 12 * n);
-    if (dfm_dp6) std::memcpy(dfm_dp6, P + 12 * n, sizeof(double) * 12 * n);
-    if (Km) std::memcpy(Km, P + 24 * n, sizeof(double) * 144 * n);
-    if (Dm) std::memcpy(Dm, P + 168 * n, sizeof(double) * 144 * n);
-    if (n_active) std::memcpy(n_active, Pn, sizeof(int32_t) * n);
-    if (Pn[n])
-        return fail(ATAC_ERR_NOMEM, "atac_batch_eval_instances_host: more active contacts than the record pool holds (" +
-                                        std::to_string(b->rec_cap) + "); plan the batch with a larger max_active");
-    return ATAC_OK;
+    return host_results(b, P, Pn, fm, Km, Dm, dfm_dp6, n_active, "atac_batch_eval_instances_host");
 }
 
 int atac_batch_vjp_host(atac_batch b, const double* g_fm, double* g_q1, double* g_q2, double* g_phi1, double* g_phi2,

@@ -64,7 +64,7 @@ inline void compose_instance(const atac_instance& s, const GridDev& G, const flo
     d.pz = pz;
     d.pt_count = n_points;
     d.grid = s.grid;
-    d.pad = 0;
+    d.chunk0 = 0;
     set_f32_copies(d);
     d.cls = nullptr;   // set by the batch (its table for this grid and col_th)
 }

@@ -110,6 +110,33 @@ struct ReduceArgs {
     int32_t* n_active;          // optional: active contacts per instance
     const int32_t* counters;    // CNT_OVERFLOW set: every output is NaN (the records were incomplete)
     int32_t* overflow_out;      // optional: receives counters[CNT_OVERFLOW] (host-visible memory allowed)
+    int32_t* done;              // optional, in host memory: receives counters[CNT_CALL] behind the instance's outputs
+};
+
+// One workgroup per instance (instance_kernel): instances of at most that many points
+// (mode 0: the wrench alone), one tile each.
+constexpr int kInstBlock = 512;
+constexpr int inst_points(int mode) { return mode == 0 ? 4096 : 2048; }
+struct InstanceArgs {
+    const InstDev* inst;
+    const GridDev* grids;
+    const TileDev* tiles;
+    int32_t chunk_total;        // work items if every point were a contact
+    int32_t host_dst;           // the outputs are in host memory
+    uint32_t* act;              // a record slot per point
+    void* rec;
+    float* slow_diag;           // 4 per record slot (FP32 records)
+    int32_t* tile_active;
+    int32_t* tile_chunk0;
+    ChunkDev* chunks;
+    int32_t* counters;
+    double* fm;                 // outputs, any may be null
+    double* p6;
+    double* Km;
+    double* Dm;
+    int32_t* n_active;
+    int32_t* overflow_out;
+    int32_t* done;              // optional, in host memory: receives counters[CNT_CALL] behind the instance's outputs
 };
 
 struct PlainArgs {
@@ -155,6 +182,10 @@ const void* vjp_kernel_ptr(bool precise);
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st);
 // the same after the Km/Dm pass: rows of kJacRow, dst = fm, dfm_dp6, Km, Dm
 hipError_t launch_reduce_jacobian(const ReduceArgs& a, hipStream_t st);
+hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, int n_inst, hipStream_t st);
+// instance records, and the number of the call (to counters[CNT_CALL]), from host
+// memory the device can read
+hipError_t launch_upload(const InstDev* src, InstDev* dst, int n, const int32_t* call, int32_t* counters, hipStream_t st);
 hipError_t launch_grid_setup(const GridDev& G, float4* cells, hipStream_t st);
 // the cell classification of a grid for one col_th (cls_bytes(G) bytes)
 hipError_t launch_cls_setup(const GridDev& G, double col_th, uint8_t* cls, hipStream_t st);

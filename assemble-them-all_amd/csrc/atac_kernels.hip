@@ -724,6 +724,8 @@ __global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
         if (lane == 0) a.n_active[i] = ovf ? -1 : n;
     }
     if (a.host_dst) __threadfence_system();   // the stores reach host memory before the launch completes
+    if (a.done && lane == 0)
+        __hip_atomic_store(a.done + i, a.counters[CNT_CALL], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The per-instance reduction of jacobian_kernel's rows, one workgroup per
@@ -735,7 +737,7 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
     constexpr int kRows = 64 * 32;   // a tile holds at most 8192 / kChunk items
     __shared__ int s_rows[kRows];
     __shared__ int s_nrows, s_nact;
-    __shared__ double s_sum[kJacRow], s_R[9], s_t[3];
+    __shared__ double s_sum[kJacRow], s_m[288], s_R[9], s_t[3];
     const int k = (int)threadIdx.x, i = (int)blockIdx.x;
     const bool ovf = a.counters[CNT_OVERFLOW] != 0;
     if (a.overflow_out && i == 0 && k == 0) *a.overflow_out = ovf ? 1 : 0;
@@ -791,13 +793,266 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
     if (k >= 12 && k < 24 && a.dst[1]) a.dst[1][(int64_t)i * 12 + k - 12] = s_sum[k];
     if (k == 0 && a.n_active) a.n_active[i] = ovf ? -1 : s_nact;
     if (a.dst[2] || a.dst[3]) {
+        for (int e = k; e < 288; e += 256) s_m[e] = jac_element(s_sum + 24, s_sum + 9, s_t, e / 24, e % 24);
+        __syncthreads();
         for (int e = k; e < 288; e += 256) {
-            const int row = e / 24, col = e % 24;
-            double* dst = col < 12 ? a.dst[2] : a.dst[3];
-            if (dst) dst[(int64_t)i * 144 + 12 * row + (col < 12 ? col : col - 12)] = jac_entry(s_sum + 24, s_sum + 9, s_R, s_t, row, col);
+            const int m = e / 144, row = (e % 144) / 12, col = e % 12;
+            double* dst = m ? a.dst[3] : a.dst[2];
+            if (dst) dst[(int64_t)i * 144 + e % 144] = jac_entry(s_m, s_R, row, 12 * m + col);
         }
     }
     if (a.host_dst) __threadfence_system();   // the stores reach host memory before the launch completes
+    if (a.done) {
+        __syncthreads();
+        if (k == 0) __hip_atomic_store(a.done + i, a.counters[CNT_CALL], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// ------------------------------------------------------------------ one workgroup per instance
+// The whole evaluation of an instance of at most inst_points(MODE) points by one workgroup
+// of 8 wavefronts: detection, the slow-path records, the wrench (p6 column, Km/Dm)
+// and the instance's sums, in LDS from step to step. For small batches: the five
+// launches of the pipeline above are each a chain of dependent reads, with a drain
+// and a launch between them; this is one chain. 64 instances of 500 points: 14 us
+// against 30 (wrench), 21 against 33 (Km/Dm); of 2,000 points 18 against 34 and 37
+// against 37; of 8,000 points 43 against 43 and 113 against 47. inst_points lies where
+// the Km/Dm rounds (some 20 us each, for 512 contacts) have used up the gain, and for
+// the wrench at the size of one tile.
+// Nothing is reserved with atomics: an instance's records start at its tile's slot
+// and its work items at InstDev::chunk0, so a batch needs a record per point. The
+// active list, records, work items and tile entries are left as the pipeline leaves
+// them (the slow index of an FP32 record is its slot), for the adjoint; the sums run
+// in the pipeline's order (per work item, then the items in turn), so that an
+// instance's results do not depend on which of the two evaluated it.
+template <int MODE, typename R>
+__global__ __launch_bounds__(kInstBlock) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 2 : 4)))
+void instance_kernel(InstanceArgs a) {
+    using Rec = typename RecOf<R>::type;
+    constexpr int NT = kInstBlock, NW = NT / 64, PPL = 4, SP = 64, ITEMS = NW / 4;
+    constexpr bool JAC = MODE == 2;
+    constexpr int NF = JAC ? kJacRow : MODE == 1 ? 24 : 12;
+    constexpr int GROUPS = 64 / kStencil;
+    __shared__ uint16_t s_q[inst_points(MODE)];      // the wavefronts' active offsets, bit 15 = slow path
+    __shared__ uint16_t s_list[inst_points(MODE)];   // all of them, in point order
+    __shared__ uint16_t s_slow[inst_points(MODE)];   // those on the slow path (places in s_list)
+    __shared__ double s_stencil[NW][GROUPS][kStencil];
+    __shared__ double s_val[NW][JAC ? JacColumns::SIZE : 64 * NF];
+    __shared__ double s_part[NW][JAC ? kJacRowPad : 1];
+    __shared__ double s_row[ITEMS][JAC ? 1 : NF];
+    __shared__ double s_sum[NF], s_m[JAC ? 288 : 1], s_R[9], s_t[3];
+    __shared__ int s_count[NW], s_nslow;
+    const int tid = (int)threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), i = (int)blockIdx.x;
+    const uint64_t lt_mask = (1ull << lane) - 1ull;
+    if (tid == 0) s_nslow = 0;
+    __syncthreads();
+    // detection: wavefront w takes a contiguous range of the steps of 64 points, PPL
+    // steps at a time: their point reads, then their table reads, then their cells are
+    // out together, so a pass over 2,048 points waits three times
+    int wcount = 0, st0;
+    {
+        const InstDev in = as_const(a.inst)[i];
+        const GridDev G = as_const(a.grids)[in.grid];
+        const int np = (int)in.pt_count, ns = (np + SP - 1) / SP, st1 = (w + 1) * ns / NW;
+        st0 = w * ns / NW;
+        const auto px = as_global(in.px), py = as_global(in.py), pz = as_global(in.pz);
+        const ClsConsts kc = cls_consts_vgpr(G, in);
+        const auto cells = ATAC_GLOBAL(G.cells);
+        const float cth = (float)in.col_th;
+        for (int st = st0; st < st1; st += PPL) {
+            const int end = min(np, st1 * SP);
+            float x[PPL], y[PPL], z[PPL];
+            load_points<PPL>(px, py, pz, st * SP, lane, end, x, y, z);
+            unsigned valid = 0, open;
+#pragma unroll
+            for (int k = 0; k < PPL; ++k)
+                if ((st + k) * SP + lane < end) valid |= 1u << k;
+            const unsigned cand = detect_candidates<PPL>(G, in, kc, x, y, z, valid, false, open, [] {}, [] {});
+            if (!__any(cand != 0u)) continue;
+            CandRead r[PPL];
+#pragma unroll
+            for (int k = 0; k < PPL; ++k) {
+                uint32_t off = 0;
+                if ((cand >> k) & 1u) off = candidate_locate(G, in, x[k], y[k], z[k], ((open >> k) & 1u) != 0u, r[k]);
+                r[k].lo = load_f4_at(cells, off);
+                r[k].hi = load_f4_at(cells, off + 16u);
+            }
+#pragma unroll
+            for (int k = 0; k < PPL; ++k) {
+                bool act = false, slow = false;
+                if ((cand >> k) & 1u) act = candidate_finish(r[k], cth, slow);
+                const uint64_t bal = __ballot(act);
+                if (act)
+                    s_q[st0 * SP + wcount + __popcll(bal & lt_mask)] =
+                        (uint16_t)((unsigned)((st + k) * SP + lane) | (slow ? 0x8000u : 0u));
+                wcount += __popcll(bal);
+            }
+        }
+    }
+    if (lane == 0) s_count[w] = wcount;
+    __syncthreads();
+    // the record again, behind an opaque pointer: kept from the detection on, its 700
+    // bytes would go through register spills
+    const InstDev* again = a.inst;
+    asm volatile("" : "+s"(again));
+    const InstDev in = as_const(again)[i];
+    const GridDev G = as_const(a.grids)[in.grid];
+    const int np = (int)in.pt_count;
+    const auto px = as_global(in.px), py = as_global(in.py), pz = as_global(in.pz);
+    // the active list in point order, for the adjoint too, and the slow-path contacts
+    int before = 0, cnt = 0;
+    for (int k = 0; k < NW; ++k) {
+        if (k < w) before += s_count[k];
+        cnt += s_count[k];
+    }
+    const int64_t slot0 = in.tile_count ? as_const(a.tiles)[in.tile_begin].slot : 0;
+    for (int k = lane; k < wcount; k += 64) {
+        const uint32_t e = s_q[st0 * SP + k];
+        const int j = before + k;
+        s_list[j] = (uint16_t)e;
+        a.act[slot0 + j] = (e & 0x7fffu) | (e >> 15 ? kActSlow : 0u);
+        if (e >> 15) s_slow[atomicAdd(&s_nslow, 1)] = (uint16_t)j;
+    }
+    // work items: kChunk contacts each
+    const int items = (cnt + kChunk - 1) / kChunk;
+    if (tid == 0 && in.tile_count) {
+        a.tile_active[in.tile_begin] = cnt;
+        a.tile_chunk0[in.tile_begin] = in.chunk0;
+    }
+    if (tid < (np + kChunk - 1) / kChunk)
+        a.chunks[in.chunk0 + tid] = tid < items ? ChunkDev{i, min(kChunk, cnt - tid * kChunk), slot0 + tid * kChunk}
+                                                : ChunkDev{i, 0, 0};
+    if (i == 0 && tid == 0) {
+        a.counters[CNT_RECS] = 0;   // counted by the tiles' entries
+        a.counters[CNT_CHUNKS] = a.chunk_total;
+        a.counters[CNT_SLOW] = 0;
+        a.counters[CNT_OVERFLOW] = 0;
+        if (a.overflow_out) *a.overflow_out = 0;
+    }
+    __syncthreads();
+    // slow-path records: the 20 stencil evaluations of a contact on 20 lanes, as slow_kernel
+    Rec* rec = static_cast<Rec*>(a.rec) + slot0;
+    for (int base = w * GROUPS; base < s_nslow; base += NW * GROUPS) {
+        const int grp = lane / kStencil, st = lane % kStencil, k = base + grp;
+        const bool mine = grp < GROUPS && k < s_nslow;
+        const int j = mine ? s_slow[k] : 0;
+        Rec r;
+        if (mine) {
+            const uint32_t off = s_list[j] & 0x7fffu;
+            r.a[0] = px[off]; r.a[1] = py[off]; r.a[2] = pz[off]; r.a[3] = __uint_as_float(off);
+            double x[3], q[3];
+            bool accurate;
+            body2_point(in, (double)r.a[0], (double)r.a[1], (double)r.a[2], x);
+            stencil_point(x, st, q, accurate);
+            s_stencil[w][grp][st] = query_sdf64(G, q[0], q[1], q[2], accurate);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (mine && st == 0) {
+            double v[kStencil], val, g[3], H[6];
+#pragma unroll
+            for (int q = 0; q < kStencil; ++q) v[q] = s_stencil[w][grp][q];
+            stencil_combine(v, val, g, H);
+            float* diag = a.slow_diag ? a.slow_diag + 4 * (slot0 + j) : nullptr;
+            record_slow_fill(in, val, g, H, r, diag);
+            mark_slow_index(r, (int)(slot0 + j));
+            store_rec(rec + j, r);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    __syncthreads();
+    // ITEMS work items at a time, a wavefront per 64 contacts
+    double total = 0.0;   // thread k < NF: component k of the instance's sums
+    const InstR<R> I = make_inst<R>(in);
+    for (int m0 = 0; m0 < items; m0 += ITEMS) {
+        const int start = (m0 + (w >> 2)) * kChunk, n = max(0, min(kChunk, cnt - start));
+        const int p0 = 64 * (w & 3), nw = n - p0;
+        if (nw > 0) {
+            const int j = start + p0 + min(lane, nw - 1);   // lanes past the end repeat the last record, not summed
+            const uint32_t e = s_list[j], off = e & 0x7fffu;
+            const Rec r = item_record(G, in, off | (e >> 15 ? kActSlow : 0u), px[off], py[off], pz[off], rec + j);
+            ContactFwd<R> s;
+            R p6[12];
+            record_decode(r, a.slow_diag, in, s);
+            contact_forward<R>(I, s, MODE >= 1 ? p6 : nullptr);
+            if constexpr (JAC) {
+                put_jac_row<R>(JacColumns{&s_val[w][0], &s_part[w][0], lane, nw}, jac_inst(in), s, p6);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 12; ++k) s_val[w][lane * NF + k] = (double)s.f[k];
+                if constexpr (MODE == 1) {
+#pragma unroll
+                    for (int k = 0; k < 12; ++k) s_val[w][lane * NF + 12 + k] = (double)p6[k];
+                }
+            }
+        }
+        __syncthreads();
+        if constexpr (!JAC) {
+            if ((w & 3) == 0 && n > 0) {   // a lane's records 64 apart in turn, then the lanes
+                double lv[NF];
+#pragma unroll
+                for (int k = 0; k < NF; ++k) lv[k] = lane < n ? s_val[w][lane * NF + k] : 0.0;
+                for (int u = 1; u < 4; ++u)
+                    if (64 * u + lane < n) {
+#pragma unroll
+                        for (int k = 0; k < NF; ++k) lv[k] += s_val[w + u][lane * NF + k];
+                    }
+                const double col = lds_column_sums<NF>(&s_val[w][0], lv);
+                if (lane < NF) s_row[w >> 2][lane] = col;
+            }
+            __syncthreads();
+            if (tid < NF) {
+                for (int h = 0; h < ITEMS && m0 + h < items; ++h) total += s_row[h][tid];
+            }
+        } else if (tid < NF) {
+            for (int h = 0; h < ITEMS && m0 + h < items; ++h) {
+                const int nh = min(kChunk, cnt - (m0 + h) * kChunk);
+                double v = s_part[4 * h][tid];
+                for (int u = 1; u < 4; ++u)
+                    if (nh > 64 * u) v += s_part[4 * h + u][tid];
+                total += v;
+            }
+        }
+        __syncthreads();
+    }
+    if (tid < NF) s_sum[tid] = total;
+    if constexpr (JAC) {
+        if (tid == NT - 1) {
+            const JacInst J = jac_inst(in);
+#pragma unroll
+            for (int q = 0; q < 9; ++q) s_R[q] = J.R.a[q];
+            s_t[0] = J.t.x; s_t[1] = J.t.y; s_t[2] = J.t.z;
+        }
+    }
+    __syncthreads();
+    if (tid < 12 && a.fm) a.fm[(int64_t)i * 12 + tid] = s_sum[tid];
+    if (MODE >= 1 && tid >= 12 && tid < 24 && a.p6) a.p6[(int64_t)i * 12 + tid - 12] = s_sum[MODE >= 1 ? tid : 0];
+    if (tid == 0 && a.n_active) a.n_active[i] = cnt;
+    if constexpr (JAC) {
+        if (tid < 288) s_m[JAC ? tid : 0] = jac_element(s_sum + 24, s_sum + 9, s_t, tid / 24, tid % 24);
+        __syncthreads();
+        if (tid < 288) {
+            const int m = tid / 144, row = (tid % 144) / 12, col = tid % 12;
+            double* dst = m ? a.Dm : a.Km;
+            if (dst) dst[(int64_t)i * 144 + tid % 144] = jac_entry(s_m, s_R, row, 12 * m + col);
+        }
+    }
+    if (a.host_dst) __threadfence_system();   // the stores reach host memory before the launch completes
+    if (a.done) {
+        __syncthreads();
+        if (tid == 0) __hip_atomic_store(a.done + i, a.counters[CNT_CALL], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// The instances' records from (pinned) host memory to the device: a kernel rather
+// than a copy, which starts and ends several microseconds later in a stream.
+__global__ __launch_bounds__(256) void upload_kernel(const uint4* src, uint4* dst, int64_t n, const int32_t* call,
+                                                     int32_t* counters) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k < n) dst[k] = src[k];
+    if (k == 0) counters[CNT_CALL] = *call;
 }
 
 // ------------------------------------------------------------------ grid set-up
@@ -1149,6 +1404,29 @@ hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st) {
 hipError_t launch_reduce_jacobian(const ReduceArgs& a, hipStream_t st) {
     if (a.n_inst <= 0) return hipSuccess;
     hipLaunchKernelGGL(reduce_jacobian_kernel, dim3(a.n_inst), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+template <int MODE>
+static void launch_instance_m(const InstanceArgs& a, bool precise, int n_inst, hipStream_t st) {
+    if (precise) hipLaunchKernelGGL((instance_kernel<MODE, double>), dim3(n_inst), dim3(kInstBlock), 0, st, a);
+    else hipLaunchKernelGGL((instance_kernel<MODE, float>), dim3(n_inst), dim3(kInstBlock), 0, st, a);
+}
+
+hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, int n_inst, hipStream_t st) {
+    if (n_inst <= 0) return hipSuccess;
+    if (mode == 0) launch_instance_m<0>(a, precise, n_inst, st);
+    else if (mode == 1) launch_instance_m<1>(a, precise, n_inst, st);
+    else launch_instance_m<2>(a, precise, n_inst, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_upload(const InstDev* src, InstDev* dst, int n, const int32_t* call, int32_t* counters, hipStream_t st) {
+    static_assert(sizeof(InstDev) % sizeof(uint4) == 0, "copied 16 bytes at a time");
+    if (n <= 0) return hipSuccess;
+    const int64_t words = (int64_t)n * (sizeof(InstDev) / sizeof(uint4));
+    hipLaunchKernelGGL(upload_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
+                       reinterpret_cast<const uint4*>(src), reinterpret_cast<uint4*>(dst), words, call, counters);
     return hipGetLastError();
 }
 

@@ -46,7 +46,7 @@ struct InstDev {
     const float* pz;
     int64_t pt_count;
     int32_t grid;
-    int32_t pad;
+    int32_t chunk0;     // first work item of this instance when they are not pushed (instance_kernel)
     int32_t tile_begin; // first tile of this instance (tiles are contiguous per instance)
     int32_t tile_count;
     // the same poses, twists and parameters rounded to FP32 for the FP32 contact
@@ -132,7 +132,10 @@ enum {
     CNT_CHUNKS = 1,
     CNT_SLOW = 2,                   // contacts in the slow list (also past its capacity)
     CNT_OVERFLOW = 3,               // non-zero: the record pool or the slow list was too small
-    CNT_WORDS = 4
+    CNT_WORDS = 4,
+    // not reset: the number of the host call the evaluation belongs to
+    CNT_CALL = CNT_WORDS,
+    CNT_ALL
 };
 
 constexpr int kFmOut = 12;          // wrench of both bodies

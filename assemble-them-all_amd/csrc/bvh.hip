@@ -395,7 +395,7 @@ __global__ __launch_bounds__(512) void bvh_force_kernel(BvhForceArgs a) {
 __global__ __launch_bounds__(1024) void bvh_reduce_kernel(BvhForceArgs a, int nb) {
     constexpr int W = 160, G = 6;
     static_assert(kJacRow <= W && G * W <= 1024, "six rows at a time");
-    __shared__ double s_sum[G][W], s_R[9], s_t[3];
+    __shared__ double s_sum[G][W], s_m[288], s_R[9], s_t[3];
     __shared__ int64_t s_cnt[64];
     const int tid = (int)threadIdx.x, g = tid / W, k = tid % W;
     if (g < G && k < kJacRow) {
@@ -432,9 +432,11 @@ __global__ __launch_bounds__(1024) void bvh_reduce_kernel(BvhForceArgs a, int nb
     __syncthreads();
     if (tid < 24) a.out[tid] = s_sum[0][tid];
     const bool deriv = (a.flags & ATAC_EVAL_DERIV) != 0u;
+    if (tid < 288) s_m[tid] = jac_element(&s_sum[0][24], &s_sum[0][9], s_t, tid / 24, tid % 24);
+    __syncthreads();
     if (tid < 288) {
         const int m = tid / 144, row = (tid % 144) / 12, col = 12 * m + tid % 12;
-        a.out[24 + tid] = deriv ? jac_entry(&s_sum[0][24], &s_sum[0][9], s_R, s_t, row, col) : 0.0;
+        a.out[24 + tid] = deriv ? jac_entry(s_m, s_R, row, col) : 0.0;
     }
     if (tid == 0 && a.n_active) {
         int64_t c = 0;

@@ -111,7 +111,11 @@ constexpr double kFdEps = 1e-5;        // BodySDFObj.cpp:178,191
 constexpr double kCellMargin = 1e-9;   // cell units kept clear of the stencil edge
 
 ATAC_HD float lerpf(float a, float b, float t) { return (1.0f - t) * a + t * b; }
-ATAC_HD double lerpd(double a, double b, double t) { return (1.0 - t) * a + t * b; }
+// The FP64 products that end in a finite difference of step 1e-5 are fused
+// explicitly: the second differences magnify a last-bit difference 1e10 times, so
+// every kernel rounds the slow path's samples alike (left to the compiler, kernels
+// contract different products).
+ATAC_HD double lerpd(double a, double b, double t) { return fma(t, b, (1.0 - t) * a); }
 
 ATAC_HD int64_t grid_index(const GridDev& G, int i, int j, int k) {
     return (int64_t)i + (int64_t)G.n[0] * ((int64_t)j + (int64_t)G.n[1] * (int64_t)k);
@@ -148,7 +152,7 @@ ATAC_HD double query_sdf64(const GridDev& G, double x0, double x1, double x2, bo
     double b1 = fmin(fmax(x1, G.minb[1]), G.maxb[1]);
     double b2 = fmin(fmax(x2, G.minb[2]), G.maxb[2]);
     double e0 = x0 - b0, e1 = x1 - b1, e2 = x2 - b2;
-    return sqrt(e0 * e0 + e1 * e1 + e2 * e2) + trilinear64_inside(G, b0, b1, b2);
+    return sqrt(fma(e2, e2, fma(e1, e1, e0 * e0))) + trilinear64_inside(G, b0, b1, b2);
 }
 
 // The FD stencils of query_dSDF / query_ddSDF (BodySDFObj.cpp:176-205) as 20
@@ -970,9 +974,9 @@ struct ContactFwd {
 ATAC_HD void body2_point(const InstDev& in, double px, double py, double pz, double x[3]) {
     const double xi[3] = {px, py, pz};
     double xw[3];
-    for (int r = 0; r < 3; ++r) xw[r] = in.R1[3 * r] * xi[0] + in.R1[3 * r + 1] * xi[1] + in.R1[3 * r + 2] * xi[2] + in.p1[r];
+    for (int r = 0; r < 3; ++r) xw[r] = fma(in.R1[3 * r + 2], xi[2], fma(in.R1[3 * r + 1], xi[1], in.R1[3 * r] * xi[0])) + in.p1[r];
     const double q0 = xw[0] - in.p2[0], q1 = xw[1] - in.p2[1], q2 = xw[2] - in.p2[2];
-    for (int r = 0; r < 3; ++r) x[r] = in.R2[r] * q0 + in.R2[3 + r] * q1 + in.R2[6 + r] * q2;
+    for (int r = 0; r < 3; ++r) x[r] = fma(in.R2[6 + r], q2, fma(in.R2[3 + r], q1, in.R2[r] * q0));
 }
 
 // Sample phi at the contact point xi1 (FP32 as stored) of instance `in`.
@@ -1273,8 +1277,8 @@ ATAC_HD void contact_jvp(const InstR<R>& I, const ContactFwd<R>& s, const Tangen
 // every contact of an instance: so the contacts sum the 15 blocks
 //   A, [X]A, V = -[Y]A + [F]Z, W = [Y](C + [F]) - [F]Z[X], C = A[X] + B[U] + T r^T - [F], [X]C,
 //   B, [X]B, [Y]B, B[X], [X]B[X], [Y]B[X], B[Y], [X]B[Y], [Y]B[Y]
-// ([v] the cross-product matrix, U = R u1, Z = d xi2 / dx), and jac_entry forms the
-// 288 entries of Km and Dm from the sums, once per instance. In FP64 for both
+// ([v] the cross-product matrix, U = R u1, Z = d xi2 / dx), and jac_element
+// and jac_entry form the 288 entries of Km and Dm from the sums, once per instance. In FP64 for both
 // arithmetics (FP64 and unpacked FP32 issue at the same rate on gfx950); the
 // sample, the friction branch and, in the FP32 arithmetic, the wrench are the
 // forward pass's. The poses are rigid (R^T R = I), as everywhere in the wrench.
@@ -1433,51 +1437,41 @@ ATAC_HD void contact_jac(const JacInst& J, v3<double> xi1, double d, v3<double> 
     put(jac_block<JB_YBY>(), skew_left(Y, BY));
 }
 
-// Entry (row, col) of [Km | Dm] (col < 12: Km) from the summed blocks S (9 per
-// block, JB_* order), body 2's summed force f2 (= -F), R and t.
-ATAC_HD double jac_entry(const double* S, const double* f2, const double* R, const double* t, int row, int col) {
-    const int rb = row / 3, ri = row - 3 * rb, cb = col / 3, cj = col - 3 * cb;
-    auto blk = [&](int b, int i, int j) { return S[9 * b + 3 * i + j]; };
-    // columns om1 and v1 of the pose (in R-turned axes)
-    auto om1 = [&](int i, int j) {
-        if (rb == 0) return -blk(JB_XC, i, j);
-        if (rb == 1) return -blk(JB_C, i, j);
-        if (rb == 2) return blk(JB_W, i, j);
-        double v = blk(JB_C, i, j);   // C + [F]
-        if (i != j) {
-            const int k = 3 - i - j;
-            v += (j == (i + 1) % 3) ? f2[k] : -f2[k];
-        }
-        return v;
-    };
-    auto v1 = [&](int i, int j) {
-        return rb == 0 ? blk(JB_XA, i, j) : rb == 1 ? blk(JB_A, i, j) : rb == 2 ? blk(JB_V, i, j) : -blk(JB_A, i, j);
-    };
-    const int db = rb == 0 ? JB_XB : rb == 2 ? JB_YB : JB_B;   // its [X] and [Y] products 3 and 6 behind
-    const double ds = rb >= 2 ? -1.0 : 1.0;
-    auto el = [&](int i, int j) {
-        switch (cb) {
-            case 0: return om1(i, j);
-            case 1: return v1(i, j);
-            case 2: {
-                const int j1 = (j + 1) % 3, j2 = (j + 2) % 3;   // (M [t])_ij = M_ij1 t_j2 - M_ij2 t_j1
-                return v1(i, j1) * t[j2] - v1(i, j2) * t[j1] - om1(i, j);
-            }
-            case 3: return -v1(i, j);
-            case 4: return -ds * blk(db + (JB_BX - JB_B), i, j);
-            case 5: return ds * blk(db, i, j);
-            case 6: return ds * blk(db + (JB_BY - JB_B), i, j);
-            default: return -ds * blk(db, i, j);
-        }
-    };
-    const bool turn_c = (cb & 2) == 0;   // body 1 columns: the tangent in body 1's axes
+// Entry (row, col) of [Km | Dm] (col < 12: Km) in the SDF body's axes, from the summed
+// blocks S (9 per block, JB_* order), body 2's summed force f2 (= -F) and t.
+ATAC_HD double jac_element(const double* S, const double* f2, const double* t, int row, int col) {
+    const int rb = row / 3, i = row - 3 * rb, cb = col / 3, j = col - 3 * cb;
+    auto blk = [&](int b, int r, int c) { return S[9 * b + 3 * r + c]; };
+    if (cb >= 4) {   // twists: B and its [X] and [Y] products, for the force or its moments
+        const int b = rb == 0 ? JB_XB : rb == 2 ? JB_YB : JB_B;
+        const double v = blk(b + (cb == 4 ? JB_BX - JB_B : cb == 6 ? JB_BY - JB_B : 0), i, j);
+        return (rb >= 2) == (cb == 5 || cb == 6) ? -v : v;
+    }
+    // pose columns om1 and v1; om2 = v1 [t] - om1 and v2 = -v1
+    const int bv = rb == 0 ? JB_XA : rb == 2 ? JB_V : JB_A;
+    const double sv = rb == 3 ? -1.0 : 1.0;
+    if (cb & 1) return cb == 1 ? sv * blk(bv, i, j) : -sv * blk(bv, i, j);
+    double om1 = rb == 0 ? -blk(JB_XC, i, j) : rb == 2 ? blk(JB_W, i, j) : rb == 1 ? -blk(JB_C, i, j) : blk(JB_C, i, j);
+    const int j1 = j == 2 ? 0 : j + 1, j2 = j == 0 ? 2 : j - 1;
+    if (rb == 3 && i != j) om1 += i == j2 ? f2[j1] : -f2[j2];   // + [F]
+    if (cb == 0) return om1;
+    return sv * (blk(bv, i, j1) * t[j2] - blk(bv, i, j2) * t[j1]) - om1;
+}
+
+// Entry (row, col) with body 1's rows and columns turned into its own axes: M (12 x 24)
+// holds the jac_elements, R = R2^T R1.
+ATAC_HD double jac_entry(const double* M, const double* R, int row, int col) {
+    const int r0 = row / 3 * 3, c0 = col / 3 * 3, ri = row - r0, cj = col - c0;
+    const bool turn_r = row < 6, turn_c = (col / 6 & 1) == 0;
     double v = 0.0;
+#pragma unroll
     for (int i = 0; i < 3; ++i) {
-        if (rb >= 2 && i != ri) continue;
+        const int mr = turn_r ? r0 + i : row;
         double q = 0.0;
-        if (turn_c) for (int j = 0; j < 3; ++j) q += el(i, j) * R[3 * j + cj];
-        else q = el(i, cj);
-        v += rb < 2 ? R[3 * i + ri] * q : q;   // body 1 rows: R^T
+#pragma unroll
+        for (int j = 0; j < 3; ++j) q += M[24 * mr + c0 + j] * R[3 * j + cj];
+        q = turn_c ? q : M[24 * mr + col];
+        v = turn_r ? v + R[3 * i + ri] * q : q;
     }
     return v;
 }

@@ -42,15 +42,15 @@ __device__ __forceinline__ T wave_sum(T v) {
 }
 
 // Values a wavefront sums over its lanes, handed over one at a time (put<k>, in
-// order of k): 32 columns wait in LDS (64 rows of 33 doubles: conflict-free writes
-// by row and reads by column), then two lanes add each column, 32 rows each, and
+// order of k): 16 columns wait in LDS (64 rows of 17 doubles: conflict-free writes
+// by row and reads by column), then four lanes add each column, 16 rows each, and
 // the sums go to `out`. Rows at or past `n` (lanes without a contact) are left
-// out. One LDS write, one read and one add per value: the butterfly over the
-// lanes it replaces took about 25 VALU instructions.
+// out. One LDS write and, over four lanes, one read and one add per value and row:
+// the butterfly over the lanes it replaces took about 25 VALU instructions.
 template <int N>
 struct WaveColumns {
-    static constexpr int W = 32, STRIDE = 33, SIZE = 64 * STRIDE;
-    double* s;     // SIZE doubles of this wavefront
+    static constexpr int W = 16, STRIDE = 17, SIZE = 64 * STRIDE;
+    double* s;     // SIZE doubles of this wavefront (all its lanes take part)
     double* out;   // N rounded up to W
     int lane, n;
     template <int K>
@@ -66,22 +66,19 @@ struct WaveColumns {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int r0 = lane & 32;
-        const double* p = s + r0 * STRIDE + (lane & 31);
+        const int r0 = lane & 48;
+        const double* p = s + r0 * STRIDE + (lane & 15);
         double q[4] = {0.0, 0.0, 0.0, 0.0};
-        if (n >= 64) {
+        // every row is read (each lane wrote one); rows past n add nothing
 #pragma unroll
-            for (int i = 0; i < 32; i += 4)
+        for (int i = 0; i < 16; i += 4)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) q[j] += p[(i + j) * STRIDE];
-        } else {
-#pragma unroll 1
-            for (int i = 0; i < min(n, 32); ++i) {
-                const double v = p[i * STRIDE];
-                q[0] += r0 + i < n ? v : 0.0;
+            for (int j = 0; j < 4; ++j) {
+                const double v = p[(i + j) * STRIDE];
+                q[j] += r0 + i + j < n ? v : 0.0;
             }
-        }
         double v = (q[0] + q[1]) + (q[2] + q[3]);
+        v += __shfl_xor(v, 16, 64);
         v += __shfl_xor(v, 32, 64);
         if (lane < W) to[lane] = v;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

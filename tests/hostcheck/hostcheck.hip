@@ -247,9 +247,11 @@ int hc_jacobian_blocks(const float* vals, const int32_t n[3], const double minb[
         });
     }
     const double t[3] = {J.t.x, J.t.y, J.t.z};
+    double M[288];
+    for (int e = 0; e < 288; ++e) M[e] = jac_element(S, f2, t, e / 24, e % 24);
     for (int r = 0; r < 12; ++r)
         for (int c = 0; c < 24; ++c) {
-            const double v = jac_entry(S, f2, J.R.a, t, r, c);
+            const double v = jac_entry(M, J.R.a, r, c);
             if (c < 12) Km[12 * r + c] = v;
             else Dm[12 * r + c - 12] = v;
         }
