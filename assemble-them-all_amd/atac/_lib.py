@@ -27,7 +27,8 @@ EXPORTED = [
     "atac_last_error", "atac_version", "atac_device_init",
     "atac_grid_create", "atac_grid_destroy",
     "atac_points_create", "atac_points_destroy", "atac_points_permutation",
-    "atac_batch_create", "atac_batch_destroy", "atac_batch_set_instances", "atac_batch_retune", "atac_batch_info",
+    "atac_batch_create", "atac_batch_destroy", "atac_batch_set_instances", "atac_batch_set_poses",
+    "atac_batch_pose_gradients", "atac_batch_retune", "atac_batch_info",
     "atac_batch_eval", "atac_batch_vjp", "atac_batch_eval_vjp", "atac_batch_graph_capture", "atac_batch_graph_launch",
     "atac_batch_active_ids", "atac_batch_touched_values", "atac_eval_plain", "atac_eval_plain_vjp", "atac_batch_timing",
     "atac_batch_workspace",
@@ -99,6 +100,8 @@ def lib():
     L.atac_batch_create.argtypes = [vp, i32, vp, i32, vp, i32, vp, C.POINTER(vp)]
     L.atac_batch_destroy.argtypes = [vp]
     L.atac_batch_set_instances.argtypes = [vp, vp, i32, vp]
+    L.atac_batch_set_poses.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i32, vp]
+    L.atac_batch_pose_gradients.argtypes = [vp, vp, vp, vp, vp, vp, vp, C.POINTER(i32), vp]
     L.atac_batch_retune.argtypes = [vp, vp]
     L.atac_batch_info.argtypes = [vp, C.POINTER(i64), C.POINTER(i32), C.POINTER(i32), vp]
     L.atac_batch_eval.argtypes = [vp, u32, vp, vp]

@@ -14,13 +14,13 @@ hand-written adjoint kernel (atac_batch_vjp):
   satisfies <G, dE> = g . xi, which is what any loss of the form L(E exp(xi))
   sees. Components of G orthogonal to the tangent space are zero in that pairing.
 
-The forward pass uploads the poses (set_instances, a host copy) and evaluates; the
+The forward pass hands the poses to the batch (set_poses; set_instances for tensors
+elsewhere than on the device or in another layout) and evaluates; the
 backward pass needs the records of that evaluation, so evaluating the batch again
 between the two raises.
 """
 from __future__ import annotations
 
-import numpy as np
 import torch
 
 from . import _lib as L
@@ -63,25 +63,39 @@ def tangent_pairing_matrix(E: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     return torch.linalg.inv(E.to(torch.float64)).transpose(1, 2) @ M
 
 
+def _on_device(t, shape):
+    """Readable by the library's kernels as it is: FP64, in order, on the current device."""
+    return (t.is_cuda and t.dtype == torch.float64 and t.shape == shape and t.is_contiguous() and not t.is_neg()
+            and t.device.index == torch.cuda.current_device())
+
+
+def _instances(batch, host):
+    """Instance records with the poses, twists and stiffnesses of the host arrays (E1, E2, phi1, phi2, kn, kt)."""
+    insts = []
+    for i in range(batch.n):
+        s = L.Instance.from_buffer_copy(batch._inst[i])
+        s.E1[:] = host[0][i].ravel().tolist()
+        s.E2[:] = host[1][i].ravel().tolist()
+        s.phi1[:] = host[2][i].tolist()
+        s.phi2[:] = host[3][i].tolist()
+        s.kn = float(host[4][i])
+        s.kt = float(host[5][i])
+        insts.append(s)
+    return insts
+
+
 class ContactWrench(torch.autograd.Function):
     @staticmethod
     def forward(ctx, batch, E1, E2, phi1, phi2, kn, kt, precise):
         n = batch.n
-        host = [t.detach().to("cpu", torch.float64).contiguous().numpy() for t in (E1, E2, phi1, phi2, kn, kt)]
-        insts = []
-        for i in range(n):
-            s = L.Instance()
-            C_copy = batch._inst[i]
-            for name, _ in L.Instance._fields_:
-                setattr(s, name, getattr(C_copy, name))
-            s.E1[:] = host[0][i].ravel().tolist()
-            s.E2[:] = host[1][i].ravel().tolist()
-            s.phi1[:] = host[2][i].tolist()
-            s.phi2[:] = host[3][i].tolist()
-            s.kn = float(host[4][i])
-            s.kt = float(host[5][i])
-            insts.append(s)
-        batch.set_instances(insts)
+        # device tensors go to the host in one kernel's stores; anything else by copies
+        args = (E1, E2, phi1, phi2, kn, kt)
+        shapes = ((n, 4, 4), (n, 4, 4), (n, 6), (n, 6), (n,), (n,))
+        if all(_on_device(t, s) for t, s in zip(args, shapes)):
+            batch.set_poses(*args)
+        else:
+            host = [t.detach().to("cpu", torch.float64).contiguous().numpy() for t in args]
+            batch.set_instances(_instances(batch, host))
         out = batch.eval(precise=bool(precise))
         ctx.batch = batch
         ctx.generation = batch.generation
@@ -94,10 +108,18 @@ class ContactWrench(torch.autograd.Function):
         if batch.generation != ctx.generation:
             raise RuntimeError("contact_wrench: the batch was evaluated again or given new instances after this forward pass; "
                                "its adjoint records are gone")
-        E1, E2 = ctx.saved_tensors
+        E1, E2 = (E if need else None for E, need in zip(ctx.saved_tensors, ctx.needs_input_grad[1:3]))
         g = batch.vjp(g_fm.contiguous())
-        gE1 = tangent_pairing_matrix(E1, g["g_q1"]) if ctx.needs_input_grad[1] else None
-        gE2 = tangent_pairing_matrix(E2, g["g_q2"]) if ctx.needs_input_grad[2] else None
+        gE1 = gE2 = None
+        # (with the grad mode on, a second derivative is asked for: torch's operations, which have one)
+        if not torch.is_grad_enabled() and all(E is None or _on_device(E, (batch.n, 4, 4)) for E in (E1, E2)):
+            if E1 is not None or E2 is not None:
+                gE1, gE2, singular = batch.pose_gradients(E1, g["g_q1"], E2, g["g_q2"])
+                if singular:   # torch's error
+                    gE1, gE2 = (None if E is None else tangent_pairing_matrix(E, g[k]) for E, k in ((E1, "g_q1"), (E2, "g_q2")))
+        else:
+            gE1 = None if E1 is None else tangent_pairing_matrix(E1, g["g_q1"])
+            gE2 = None if E2 is None else tangent_pairing_matrix(E2, g["g_q2"])
         return (None, gE1, gE2, g["g_phi1"], g["g_phi2"], g["g_kn"], g["g_kt"], None)
 
 

@@ -204,6 +204,15 @@ class ContactBatch:
         self.generation += 1   # the adjoint records of the last evaluation belong to the old instances
         check(lib().atac_batch_set_instances(self.handle, arr, self.n, _stream()))
 
+    def set_poses(self, E1, E2, phi1, phi2, kn, kt):
+        """set_instances with new poses, twists and stiffnesses from contiguous FP64 tensors on
+        the device (n x 4 x 4, n x 4 x 4, n x 6, n x 6, n, n)."""
+        arr = (L.Instance * self.n).from_buffer_copy(self._inst)
+        self.generation += 1
+        check(lib().atac_batch_set_poses(self.handle, E1.data_ptr(), E2.data_ptr(), phi1.data_ptr(), phi2.data_ptr(),
+                                         kn.data_ptr(), kt.data_ptr(), arr, self.n, _stream()))
+        self._inst = arr
+
     def alloc_outputs(self, deriv=False, p6=False, device="cuda"):
         f64 = dict(dtype=torch.float64, device=device)
         out = {"fm": torch.empty((self.n, 12), **f64),
@@ -288,6 +297,15 @@ class ContactBatch:
         s = self._grad_struct(out)
         check(lib().atac_batch_vjp(self.handle, _ptr(g_fm), C.byref(s), _stream()))
         return out
+
+    def pose_gradients(self, E1, g_q1, E2, g_q2):
+        """The matrix gradients of atac.autograd for contiguous FP64 poses on the device (None: left out),
+        and the number of poses that have no inverse."""
+        gE1, gE2 = (None if E is None else torch.empty_like(E) for E in (E1, E2))
+        bad = C.c_int32()
+        p = [None if t is None else t.data_ptr() for t in (E1, g_q1, gE1, E2, g_q2, gE2)]
+        check(lib().atac_batch_pose_gradients(self.handle, *p, C.byref(bad), _stream()))
+        return gE1, gE2, bad.value
 
     def graph_capture(self, out, deriv=False, p6=False, checkpoint=False, precise=False, g_fm=None, grads=None,
                       fused=False):

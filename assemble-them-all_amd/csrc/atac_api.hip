@@ -108,7 +108,9 @@ struct atac_batch_s {
     bool last_culled = false;         // the last evaluation enqueued ran the culling pass
     bool one_per_instance = false;    // the plan allows instance_kernel
     int64_t most_points = 0;          // of an instance
-    int32_t host_call = 0;            // calls of atac_batch_eval_instances_host so far
+    int32_t host_call = 0;            // number of the last host call that waits for the device's words
+    InstDev* pin_pose = nullptr;      // pinned: the records atac_batch_set_poses uploads
+    hipEvent_t pose_read = nullptr;   // ... read
     int32_t chunk_total = 0;          // work items if every point were a contact
     int32_t* d_tile_chunk0 = nullptr;
     ChunkDev* d_chunks = nullptr;
@@ -141,7 +143,8 @@ struct atac_batch_s {
     // pinned host staging of the host-buffer entry points' results: the device-to-host
     // copies run as DMA without the runtime's pageable staging, then one wait
     char* pin = nullptr;          // 312 doubles per instance | n_active per instance | overflow flag | number of
-                                  // the finished call per instance | number of the call
+                                  // the finished call per instance | number of the call |
+                                  // finished call per pose gradient (two per instance)
     InstDev* pin_inst = nullptr;  // pinned instance records for atac_batch_eval_instances_host
     // graphs of atac_batch_eval_instances_host per flag combination, valid while no device
     // buffer has been (re)allocated since their capture (buf_gen)
@@ -757,6 +760,8 @@ int atac_batch_destroy(atac_batch b) {
     dfree(b->h_out); dfree(b->h_nact); dfree(b->h_gfm); dfree(b->h_grad);
     if (b->pin) (void)hipHostFree(b->pin);
     if (b->pin_inst) (void)hipHostFree(b->pin_inst);
+    if (b->pose_read) { (void)hipEventSynchronize(b->pose_read); (void)hipEventDestroy(b->pose_read); }
+    if (b->pin_pose) (void)hipHostFree(b->pin_pose);
     for (auto& kv : b->host_graphs) {
         if (kv.second.e) (void)hipGraphExecDestroy(kv.second.e);
         if (kv.second.g) (void)hipGraphDestroy(kv.second.g);
@@ -766,23 +771,30 @@ int atac_batch_destroy(atac_batch b) {
     return ATAC_OK;
 }
 
-int atac_batch_set_instances(atac_batch b, const atac_instance* inst, int32_t n_inst, void* stream) {
-    if (!b || (n_inst && !inst)) return fail(ATAC_ERR_INVALID, "atac_batch_set_instances: null argument");
-    if (n_inst != (int32_t)b->inst.size()) return fail(ATAC_ERR_INVALID, "atac_batch_set_instances: instance count differs");
+// The checks and the composed records of new instances; the device's are uploaded by
+// the caller.
+static int compose_instances(atac_batch b, const atac_instance* inst, int32_t n_inst, const char* who) {
+    if (n_inst != (int32_t)b->inst.size()) return fail(ATAC_ERR_INVALID, std::string(who) + ": instance count differs");
     for (int i = 0; i < n_inst; ++i)
         if (inst[i].grid != b->inst[i].grid || inst[i].points != b->inst[i].points || inst[i].segment != b->inst[i].segment)
-            return fail(ATAC_ERR_INVALID, "atac_batch_set_instances: instance " + std::to_string(i) + " changes its grid/points/segment");
+            return fail(ATAC_ERR_INVALID, std::string(who) + ": instance " + std::to_string(i) +
+                                              " changes its grid/points/segment");
     int rc = check_instances(b, inst, n_inst);
     if (rc) return rc;
-    for (int i = 0; i < n_inst; ++i) {
-        recompose(b, i, inst[i]);
-    }
+    for (int i = 0; i < n_inst; ++i) recompose(b, i, inst[i]);
     rc = ensure_cls(b);   // a new col_th needs its classification table
     if (rc) return rc;
     b->inst.assign(inst, inst + n_inst);
     // the records of the last evaluation belong to the old poses: the adjoint
     // must not combine them with the new instance records
     b->rec_valid = false;
+    return ATAC_OK;
+}
+
+int atac_batch_set_instances(atac_batch b, const atac_instance* inst, int32_t n_inst, void* stream) {
+    if (!b || (n_inst && !inst)) return fail(ATAC_ERR_INVALID, "atac_batch_set_instances: null argument");
+    const int rc = compose_instances(b, inst, n_inst, "atac_batch_set_instances");
+    if (rc) return rc;
     if (n_inst) {
         if (stream) {
             ATAC_HIP(hipMemcpyAsync(b->d_inst, b->inst_dev.data(), sizeof(InstDev) * n_inst, hipMemcpyHostToDevice,
@@ -1295,27 +1307,28 @@ static int ensure_staging(atac_batch b) {
     if (!rc && !b->h_gfm) rc = dalloc(&b->h_gfm, n * 12);
     if (!rc && !b->h_grad) rc = dalloc(&b->h_grad, n * kVjpOut);
     if (!rc && !b->pin) {
-        const hipError_t e = hipHostMalloc((void**)&b->pin, n * (312 * sizeof(double) + 2 * sizeof(int32_t)) + 16,
+        const hipError_t e = hipHostMalloc((void**)&b->pin, n * (312 * sizeof(double) + 4 * sizeof(int32_t)) + 16,
                                            hipHostMallocDefault);
         if (e != hipSuccess) {
             b->pin = nullptr;
             rc = fail(ATAC_ERR_NOMEM, std::string("pinned staging: ") + hipGetErrorString(e));
         } else {
-            std::memset(b->pin, 0, n * (312 * sizeof(double) + 2 * sizeof(int32_t)) + 16);   // no call is 0
+            std::memset(b->pin, 0, n * (312 * sizeof(double) + 4 * sizeof(int32_t)) + 16);   // no call is 0
         }
     }
     return rc;
 }
 
-// Waits until every instance's word in `done` holds the call's number (the device
-// writes it behind the instance's results), or, after two milliseconds, for the stream.
-static int wait_done(atac_batch b, const volatile int32_t* done, int32_t call, hipStream_t st) {
+// Waits until the n words of `done` hold the call's number, or its negative (the device
+// writes it behind the results it stands for), or, after two milliseconds, for the stream.
+static int wait_done(const volatile int32_t* done, size_t n, int32_t call, hipStream_t st) {
     const auto t0 = std::chrono::steady_clock::now();
-    for (size_t i = 0; i < b->inst.size(); ++i)
-        for (uint32_t spins = 1; done[i] != call; ++spins)
+    const auto arrived = [&](size_t i) { const int32_t v = done[i]; return v == call || v == -call; };
+    for (size_t i = 0; i < n; ++i)
+        for (uint32_t spins = 1; !arrived(i); ++spins)
             if ((spins & 1023u) == 0u && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
                 ATAC_HIP(hipStreamSynchronize(st));
-                if (done[i] != call) return fail(ATAC_ERR_HIP, "atac_batch_eval_instances_host: no result");
+                if (!arrived(i)) return fail(ATAC_ERR_HIP, "the device wrote no result");
                 break;
             }
     std::atomic_thread_fence(std::memory_order_acquire);
@@ -1366,29 +1379,89 @@ int atac_batch_eval_host(atac_batch b, uint32_t flags, double* fm, double* Km, d
     return host_results(b, P, Pn, fm, Km, Dm, dfm_dp6, n_active, "atac_batch_eval_host");
 }
 
+static int next_call(atac_batch b) {   // 1, 2, ... (never 0 or its own negative)
+    b->host_call = b->host_call == INT32_MAX ? 1 : b->host_call + 1;
+    return b->host_call;
+}
+
+static int refuse_capture(hipStream_t st, const char* who) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    ATAC_HIP(hipStreamIsCapturing(st, &cs));
+    return cs == hipStreamCaptureStatusNone ? ATAC_OK : fail(ATAC_ERR_STATE, std::string(who) + ": the stream is being captured");
+}
+
+int atac_batch_set_poses(atac_batch b, const double* E1, const double* E2, const double* phi1, const double* phi2,
+                         const double* kn, const double* kt, atac_instance* inst, int32_t n_inst, void* stream) {
+    if (!b || (n_inst && (!inst || !E1 || !E2 || !phi1 || !phi2 || !kn || !kt)))
+        return fail(ATAC_ERR_INVALID, "atac_batch_set_poses: null argument");
+    if (n_inst != (int32_t)b->inst.size()) return fail(ATAC_ERR_INVALID, "atac_batch_set_poses: instance count differs");
+    hipStream_t st = (hipStream_t)stream;
+    int rc = refuse_capture(st, "atac_batch_set_poses");
+    if (rc || n_inst == 0) return rc;
+    rc = ensure_staging(b);
+    if (rc) return rc;
+    const size_t n = (size_t)n_inst;
+    double* rows = reinterpret_cast<double*>(b->pin);
+    int32_t* done = reinterpret_cast<int32_t*>(b->pin + n * 312 * sizeof(double)) + n + 1;
+    const int32_t call = next_call(b);
+    ATAC_HIP(launch_pose_rows(E1, E2, phi1, phi2, kn, kt, rows, done, call, n_inst, st));
+    rc = wait_done(done, n, call, st);
+    if (rc) return rc;
+    for (size_t i = 0; i < n; ++i) {
+        const double* r = rows + kPoseRow * i;
+        std::memcpy(inst[i].E1, r, 44 * sizeof(double));   // E1, phi1, E2, phi2 lie in a row
+        inst[i].kn = r[44];
+        inst[i].kt = r[45];
+    }
+    rc = compose_instances(b, inst, n_inst, "atac_batch_set_poses");
+    if (rc) return rc;
+    if (!b->pin_pose) {
+        hipError_t e = hipHostMalloc((void**)&b->pin_pose, sizeof(InstDev) * n, hipHostMallocDefault);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&b->pose_read, hipEventDisableTiming);
+        if (e != hipSuccess) {
+            if (b->pin_pose) (void)hipHostFree(b->pin_pose);
+            b->pin_pose = nullptr;
+            return fail(ATAC_ERR_NOMEM, std::string("pinned staging: ") + hipGetErrorString(e));
+        }
+    } else {
+        ATAC_HIP(hipEventSynchronize(b->pose_read));   // the last upload, on whatever stream it was
+    }
+    std::memcpy(b->pin_pose, b->inst_dev.data(), sizeof(InstDev) * n);
+    ATAC_HIP(launch_upload(b->pin_pose, b->d_inst, n_inst, nullptr, nullptr, st));
+    ATAC_HIP(hipEventRecord(b->pose_read, st));
+    return ATAC_OK;
+}
+
+int atac_batch_pose_gradients(atac_batch b, const double* E1, const double* g_q1, double* g_E1, const double* E2,
+                              const double* g_q2, double* g_E2, int32_t* singular, void* stream) {
+    if (!b || !singular || (g_E1 && (!E1 || !g_q1)) || (g_E2 && (!E2 || !g_q2)))
+        return fail(ATAC_ERR_INVALID, "atac_batch_pose_gradients: null argument");
+    *singular = 0;
+    const size_t n = b->inst.size();
+    hipStream_t st = (hipStream_t)stream;
+    int rc = refuse_capture(st, "atac_batch_pose_gradients");
+    if (rc || n == 0) return rc;
+    rc = ensure_staging(b);
+    if (rc) return rc;
+    int32_t* done = reinterpret_cast<int32_t*>(b->pin + n * 312 * sizeof(double)) + 2 * n + 2;
+    const int32_t call = next_call(b);
+    ATAC_HIP(launch_pose_gradients(E1, g_q1, g_E1, E2, g_q2, g_E2, done, call, (int)n, st));
+    rc = wait_done(done, 2 * n, call, st);
+    if (rc) return rc;
+    for (size_t i = 0; i < 2 * n; ++i) *singular += done[i] < 0;
+    return ATAC_OK;
+}
+
 int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int32_t n_inst, uint32_t flags, double* fm,
                                    double* Km, double* Dm, double* dfm_dp6, int32_t* n_active) {
     if (!b || (n_inst && !inst)) return fail(ATAC_ERR_INVALID, "atac_batch_eval_instances_host: null argument");
-    if (n_inst != (int32_t)b->inst.size())
-        return fail(ATAC_ERR_INVALID, "atac_batch_eval_instances_host: instance count differs");
-    for (int i = 0; i < n_inst; ++i)
-        if (inst[i].grid != b->inst[i].grid || inst[i].points != b->inst[i].points || inst[i].segment != b->inst[i].segment)
-            return fail(ATAC_ERR_INVALID, "atac_batch_eval_instances_host: instance " + std::to_string(i) +
-                                              " changes its grid/points/segment");
     if (flags & ~(ATAC_EVAL_DERIV | ATAC_EVAL_P6 | ATAC_EVAL_CHECKPOINT | ATAC_EVAL_PRECISE | ATAC_EVAL_ALL_ACTIVE))
         return fail(ATAC_ERR_INVALID, "atac_batch_eval_instances_host: unknown flag");
     const int mode = mode_of(flags);
     if (dfm_dp6 && mode < 1) return fail(ATAC_ERR_INVALID, "dfm_dp6 requested without ATAC_EVAL_P6 or ATAC_EVAL_DERIV");
     if ((Km || Dm) && mode < 2) return fail(ATAC_ERR_INVALID, "Km/Dm requested without ATAC_EVAL_DERIV");
-    int rc = check_instances(b, inst, n_inst);
+    int rc = compose_instances(b, inst, n_inst, "atac_batch_eval_instances_host");
     if (rc) return rc;
-    for (int i = 0; i < n_inst; ++i) {
-        recompose(b, i, inst[i]);
-    }
-    rc = ensure_cls(b);
-    if (rc) return rc;
-    b->inst.assign(inst, inst + n_inst);
-    b->rec_valid = false;
     if (n_inst == 0) return ATAC_OK;
     rc = ensure_staging(b);
     if (!rc) rc = ensure_buffers(b, mode, (flags & ATAC_EVAL_PRECISE) != 0);
@@ -1416,7 +1489,7 @@ int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int3
     int32_t* done = Pn + n + 1;
     int32_t* call = done + n;
     std::memcpy(b->pin_inst, b->inst_dev.data(), sizeof(InstDev) * n);   // the previous call has finished with it
-    *call = ++b->host_call;
+    *call = next_call(b);
     if (takes_one_per_instance(b, flags)) {   // two launches: no graph
         const bool timing = b->timing;
         b->timing = false;
@@ -1424,7 +1497,7 @@ int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int3
         rc = enqueue_eval(b, flags, &o, st, Pn + n, nullptr, nullptr, done);
         b->timing = timing;
         if (rc) (void)hipStreamSynchronize(st);
-        else rc = wait_done(b, done, *call, st);
+        else rc = wait_done(done, n, *call, st);
         return rc ? rc : host_results(b, P, Pn, fm, Km, Dm, dfm_dp6, n_active, "atac_batch_eval_instances_host");
     }
     const uint32_t key = flags | ((Km || Dm) ? 1u << 8 : 0u) | (dfm_dp6 ? 1u << 9 : 0u);
@@ -1456,7 +1529,7 @@ int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int3
         hg.gen = b->buf_gen;
     }
     ATAC_HIP(hipGraphLaunch(hg.e, st));
-    rc = wait_done(b, done, *call, st);
+    rc = wait_done(done, n, *call, st);
     if (rc) return rc;
     b->rec_valid = true;   // the replay left its records for atac_batch_vjp
     b->rec_precise = (flags & ATAC_EVAL_PRECISE) != 0;

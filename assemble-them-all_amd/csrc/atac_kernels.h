@@ -183,9 +183,20 @@ hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st);
 // the same after the Km/Dm pass: rows of kJacRow, dst = fm, dfm_dp6, Km, Dm
 hipError_t launch_reduce_jacobian(const ReduceArgs& a, hipStream_t st);
 hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, int n_inst, hipStream_t st);
-// instance records, and the number of the call (to counters[CNT_CALL]), from host
-// memory the device can read
+// instance records, and (call != nullptr) the number of the call to counters[CNT_CALL],
+// from host memory the device can read
 hipError_t launch_upload(const InstDev* src, InstDev* dst, int n, const int32_t* call, int32_t* counters, hipStream_t st);
+
+// Poses, twists and stiffnesses of n instances (the device arrays of
+// atac_batch_set_poses) as rows of kPoseRow doubles in host memory, in the order of
+// atac_instance's members; done[i] = call behind row i.
+constexpr int kPoseRow = 46;
+hipError_t launch_pose_rows(const double* E1, const double* E2, const double* phi1, const double* phi2, const double* kn,
+                            const double* kt, double* rows, int32_t* done, int32_t call, int n, hipStream_t st);
+// gE = E^-T M(g) of two lists of n poses (either may be null); done[2 i + body] = call
+// (-call: E is singular)
+hipError_t launch_pose_gradients(const double* E1, const double* g1, double* gE1, const double* E2, const double* g2,
+                                 double* gE2, int32_t* done, int32_t call, int n, hipStream_t st);
 hipError_t launch_grid_setup(const GridDev& G, float4* cells, hipStream_t st);
 // the cell classification of a grid for one col_th (cls_bytes(G) bytes)
 hipError_t launch_cls_setup(const GridDev& G, double col_th, uint8_t* cls, hipStream_t st);

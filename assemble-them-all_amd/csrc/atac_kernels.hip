@@ -1052,7 +1052,81 @@ __global__ __launch_bounds__(256) void upload_kernel(const uint4* src, uint4* ds
                                                      int32_t* counters) {
     const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (k < n) dst[k] = src[k];
-    if (k == 0) counters[CNT_CALL] = *call;
+    if (k == 0 && call) counters[CNT_CALL] = *call;
+}
+
+__global__ __launch_bounds__(64) void pose_rows_kernel(const double* E1, const double* E2, const double* phi1,
+                                                       const double* phi2, const double* kn, const double* kt, double* rows,
+                                                       int32_t* done, int32_t call) {
+    const int k = (int)threadIdx.x;
+    const int64_t i = blockIdx.x;
+    if (k < kPoseRow)
+        rows[i * kPoseRow + k] = k < 16 ? E1[16 * i + k] : k < 22 ? phi1[6 * i + k - 16] : k < 38 ? E2[16 * i + k - 22]
+                               : k < 44 ? phi2[6 * i + k - 38] : k == 44 ? kn[i] : kt[i];
+    __threadfence_system();   // one wavefront: every lane's store is out before lane 0's
+    if (k == 0) __hip_atomic_store(done + i, call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A lane per pose: E^T X = M by elimination with row exchanges, in registers.
+__global__ __launch_bounds__(64) void pose_gradients_kernel(const double* E1, const double* g1, double* gE1,
+                                                            const double* E2, const double* g2, double* gE2,
+                                                            int32_t* done, int32_t call, int n) {
+    const int64_t t = (int64_t)blockIdx.x * 64 + threadIdx.x, i = t >> 1;
+    if (i >= n) return;
+    const double* E = (t & 1) ? E2 : E1;
+    const double* g = (t & 1) ? g2 : g1;
+    double* out = (t & 1) ? gE2 : gE1;
+    bool singular = false;
+    if (out) {
+        double m[4][8];   // [E^T | M]
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                m[r][c] = E[16 * i + 4 * c + r];
+                m[r][4 + c] = 0.0;
+            }
+        const double w0 = 0.5 * g[6 * i], w1 = 0.5 * g[6 * i + 1], w2 = 0.5 * g[6 * i + 2];
+        m[0][5] = -w2; m[0][6] = w1;
+        m[1][4] = w2;  m[1][6] = -w0;
+        m[2][4] = -w1; m[2][5] = w0;
+        m[0][7] = g[6 * i + 3]; m[1][7] = g[6 * i + 4]; m[2][7] = g[6 * i + 5];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+#pragma unroll
+            for (int r = k + 1; r < 4; ++r) {
+                const bool swap = fabs(m[r][k]) > fabs(m[k][k]);
+#pragma unroll
+                for (int c = k; c < 8; ++c) {
+                    const double a = m[k][c], b = m[r][c];
+                    m[k][c] = swap ? b : a;
+                    m[r][c] = swap ? a : b;
+                }
+            }
+            singular = singular || m[k][k] == 0.0;
+#pragma unroll
+            for (int r = k + 1; r < 4; ++r) {
+                const double f = m[r][k] / m[k][k];
+#pragma unroll
+                for (int c = k + 1; c < 8; ++c) m[r][c] -= f * m[k][c];
+            }
+        }
+#pragma unroll
+        for (int c = 4; c < 8; ++c) {
+#pragma unroll
+            for (int k = 3; k >= 0; --k) {
+                double v = m[k][c];
+#pragma unroll
+                for (int j = k + 1; j < 4; ++j) v -= m[k][j] * m[j][c];
+                m[k][c] = v / m[k][k];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) out[16 * i + 4 * r + c] = m[r][4 + c];
+    }
+    __hip_atomic_store(done + t, singular ? -call : call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ------------------------------------------------------------------ grid set-up
@@ -1418,6 +1492,18 @@ hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, int n_
     if (mode == 0) launch_instance_m<0>(a, precise, n_inst, st);
     else if (mode == 1) launch_instance_m<1>(a, precise, n_inst, st);
     else launch_instance_m<2>(a, precise, n_inst, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_pose_rows(const double* E1, const double* E2, const double* phi1, const double* phi2, const double* kn,
+                            const double* kt, double* rows, int32_t* done, int32_t call, int n, hipStream_t st) {
+    hipLaunchKernelGGL(pose_rows_kernel, dim3(n), dim3(64), 0, st, E1, E2, phi1, phi2, kn, kt, rows, done, call);
+    return hipGetLastError();
+}
+
+hipError_t launch_pose_gradients(const double* E1, const double* g1, double* gE1, const double* E2, const double* g2,
+                                 double* gE2, int32_t* done, int32_t call, int n, hipStream_t st) {
+    hipLaunchKernelGGL(pose_gradients_kernel, dim3((n + 31) / 32), dim3(64), 0, st, E1, g1, gE1, E2, g2, gE2, done, call, n);
     return hipGetLastError();
 }
 

@@ -141,6 +141,16 @@ int atac_batch_destroy(atac_batch b);
  * ATAC_ERR_STATE until the next evaluation). stream NULL: a synchronous upload
  * ordered after the work already queued on the batch's own stream. */
 int atac_batch_set_instances(atac_batch b, const atac_instance* inst, int32_t n_inst, void* stream);
+/* The same with the poses, twists and stiffnesses in device memory (FP64, in the
+ * stream's order: E1, E2 n x 16, phi1, phi2 n x 6, kn, kt n); inst holds the other
+ * members and receives these. Waits for those arrays, not for the upload. */
+int atac_batch_set_poses(atac_batch b, const double* E1, const double* E2, const double* phi1, const double* phi2,
+                         const double* kn, const double* kt, atac_instance* inst, int32_t n_inst, void* stream);
+/* Matrix gradients of poses from twist gradients g = (g_w, g_v): g_E = E^-T M(g),
+ * M(g) = [[skew(g_w) / 2, g_v], [0, 0]] (n x 16; a null g_E is left out). singular:
+ * the number of poses without an inverse. Device pointers; waits for the result. */
+int atac_batch_pose_gradients(atac_batch b, const double* E1, const double* g_q1, double* g_E1, const double* E2,
+                              const double* g_q2, double* g_E2, int32_t* singular, void* stream);
 /* Re-plans tiles and launch shape (used by the autotuner). */
 int atac_batch_retune(atac_batch b, const atac_tuning* tuning);
 int atac_batch_info(atac_batch b, int64_t* n_points, int32_t* n_tiles, int32_t* persistent_blocks,
