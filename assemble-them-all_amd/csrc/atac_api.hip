@@ -609,11 +609,11 @@ static int plan(atac_batch b, const atac_tuning* t) {
     // one workgroup per instance (instance_kernel): default plans of small instances, as
     // many as the GPU holds at once (two per CU); with 1,024 instances of 500 points the
     // pipeline's finer pieces fill it better (37 us against 42; 512: 34 against 25)
-    b->one_per_instance = (!t || default_tuning(*t)) && b->rec_cap == slot && b->inst_dev.size() <= (size_t)(2 * b->n_cu) &&
-                          T >= inst_points(0);
+    static_assert(kGroup % kChunk == 0, "an instance's items are as many over its tiles as over its points");
     b->most_points = 0;
     for (const InstDev& d : b->inst_dev) b->most_points = std::max(b->most_points, (int64_t)d.pt_count);
-    b->one_per_instance = b->one_per_instance && b->most_points <= inst_points(0);
+    b->one_per_instance = (!t || default_tuning(*t)) && b->rec_cap == slot &&
+                          b->inst_dev.size() <= (size_t)(2 * b->n_cu) && b->most_points <= inst_points(0);
     // tile queues: 1 = one queue in instance order; 2 = one queue grouped by grid;
     // 3 = grouped by grid and cut into one queue per XCD with balanced point counts;
     // 4 = one queue per XCD by the tile's place in its instance's point order: a
@@ -866,11 +866,13 @@ static bool takes_one_per_instance(atac_batch b, uint32_t flags) {
 }
 
 // overflow_out (optional) receives the evaluation's overflow flag from the reduction.
+// call != 0: the host call of that number by one workgroup per instance, its records
+// in the pinned staging.
 // g_fused != nullptr: the fused pass (ATAC_EVAL_FUSED_ADJOINT), the wrench and the
 // adjoint of g_fused into out and gg, no records kept.
 static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, hipStream_t st,
                         int32_t* overflow_out = nullptr, const double* g_fused = nullptr,
-                        const atac_gradients* gg = nullptr, int32_t* done = nullptr) {
+                        const atac_gradients* gg = nullptr, int32_t* done = nullptr, int32_t call = 0) {
     if (flags & ~(ATAC_EVAL_DERIV | ATAC_EVAL_P6 | ATAC_EVAL_CHECKPOINT | ATAC_EVAL_PRECISE | ATAC_EVAL_ALL_ACTIVE |
                   (g_fused ? ATAC_EVAL_FUSED_ADJOINT : 0u)))
         return fail(ATAC_ERR_INVALID, "atac_batch_eval: unknown flag");
@@ -901,6 +903,7 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
         ia.counters = counters(b);
         if (out) { ia.fm = out->fm; ia.p6 = out->dfm_dp6; ia.Km = out->Km; ia.Dm = out->Dm; ia.n_active = out->n_active; }
         ia.overflow_out = overflow_out; ia.host_dst = overflow_out ? 1 : 0; ia.done = done;
+        ia.call = call; ia.src = call ? b->pin_inst : nullptr;
         ATAC_HIP(launch_instance(ia, mode, precise, (int)b->inst.size(), st));
         return eval_done(b, false, precise, st);
     }
@@ -1490,11 +1493,10 @@ int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int3
     int32_t* call = done + n;
     std::memcpy(b->pin_inst, b->inst_dev.data(), sizeof(InstDev) * n);   // the previous call has finished with it
     *call = next_call(b);
-    if (takes_one_per_instance(b, flags)) {   // two launches: no graph
+    if (takes_one_per_instance(b, flags)) {   // one launch: no graph
         const bool timing = b->timing;
         b->timing = false;
-        ATAC_HIP(launch_upload(b->pin_inst, b->d_inst, (int)n, call, b->d_counters, st));
-        rc = enqueue_eval(b, flags, &o, st, Pn + n, nullptr, nullptr, done);
+        rc = enqueue_eval(b, flags, &o, st, Pn + n, nullptr, nullptr, done, *call);
         b->timing = timing;
         if (rc) (void)hipStreamSynchronize(st);
         else rc = wait_done(done, n, *call, st);

@@ -110,15 +110,17 @@ struct ReduceArgs {
     int32_t* n_active;          // optional: active contacts per instance
     const int32_t* counters;    // CNT_OVERFLOW set: every output is NaN (the records were incomplete)
     int32_t* overflow_out;      // optional: receives counters[CNT_OVERFLOW] (host-visible memory allowed)
-    int32_t* done;              // optional, in host memory: receives counters[CNT_CALL] behind the instance's outputs
+    int32_t* done;              // optional, in host memory: receives `call` behind the instance's outputs
+    int32_t call;
+    const InstDev* src;         // optional, in host memory: the instances, copied to inst first
 };
 
 // One workgroup per instance (instance_kernel): instances of at most that many points
-// (mode 0: the wrench alone), one tile each.
+// (mode 0: the wrench alone).
 constexpr int kInstBlock = 512;
-constexpr int inst_points(int mode) { return mode == 0 ? 4096 : 2048; }
+constexpr int inst_points(int mode) { return mode == 0 ? 8192 : 2048; }
 struct InstanceArgs {
-    const InstDev* inst;
+    InstDev* inst;
     const GridDev* grids;
     const TileDev* tiles;
     int32_t chunk_total;        // work items if every point were a contact
@@ -136,7 +138,10 @@ struct InstanceArgs {
     double* Dm;
     int32_t* n_active;
     int32_t* overflow_out;
-    int32_t* done;              // optional, in host memory: receives counters[CNT_CALL] behind the instance's outputs
+    int32_t* done;              // optional, in host memory: receives `call` behind the instance's outputs
+    const InstDev* src;         // optional, in host memory: the instances, copied to inst first
+    int32_t call;
+    int32_t pad;
 };
 
 struct PlainArgs {

@@ -815,15 +815,16 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
 // launches of the pipeline above are each a chain of dependent reads, with a drain
 // and a launch between them; this is one chain. 64 instances of 500 points: 14 us
 // against 30 (wrench), 21 against 33 (Km/Dm); of 2,000 points 18 against 34 and 37
-// against 37; of 8,000 points 43 against 43 and 113 against 47. inst_points lies where
-// the Km/Dm rounds (some 20 us each, for 512 contacts) have used up the gain, and for
-// the wrench at the size of one tile.
+// against 37; of 8,000 points 43 against 43 and 113 against 47 (8 instances: 37
+// against 41): inst_points lies where the steps in turn have used up the gain (a round
+// of 512 contacts takes some 20 us for Km/Dm).
 // Nothing is reserved with atomics: an instance's records start at its tile's slot
 // and its work items at InstDev::chunk0, so a batch needs a record per point. The
 // active list, records, work items and tile entries are left as the pipeline leaves
-// them (the slow index of an FP32 record is its slot), for the adjoint; the sums run
-// in the pipeline's order (per work item, then the items in turn), so that an
-// instance's results do not depend on which of the two evaluated it.
+// them, all under the instance's first tile (the slow index of an FP32 record is its
+// slot), for the adjoint; the sums run in the pipeline's order, per work item, then the
+// items in turn. A host call's instances are read from its pinned copy: an upload of
+// its own costs 4 us.
 template <int MODE, typename R>
 __global__ __launch_bounds__(kInstBlock) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 2 : 4)))
 void instance_kernel(InstanceArgs a) {
@@ -832,11 +833,13 @@ void instance_kernel(InstanceArgs a) {
     constexpr bool JAC = MODE == 2;
     constexpr int NF = JAC ? kJacRow : MODE == 1 ? 24 : 12;
     constexpr int GROUPS = 64 / kStencil;
-    __shared__ uint16_t s_q[inst_points(MODE)];      // the wavefronts' active offsets, bit 15 = slow path
-    __shared__ uint16_t s_list[inst_points(MODE)];   // all of them, in point order
-    __shared__ uint16_t s_slow[inst_points(MODE)];   // those on the slow path (places in s_list)
+    __shared__ uint16_t s_list[inst_points(MODE)];   // the active offsets in point order, bit 15 = slow path
     __shared__ double s_stencil[NW][GROUPS][kStencil];
     __shared__ double s_val[NW][JAC ? JacColumns::SIZE : 64 * NF];
+    // until the contacts: the wavefronts' own active offsets, and the slow ones' places in s_list
+    static_assert(sizeof s_val >= 4 * inst_points(MODE), "both lists lie in s_val");
+    uint16_t* const s_q = reinterpret_cast<uint16_t*>(s_val);
+    uint16_t* const s_slow = s_q + inst_points(MODE);
     __shared__ double s_part[NW][JAC ? kJacRowPad : 1];
     __shared__ double s_row[ITEMS][JAC ? 1 : NF];
     __shared__ double s_sum[NF], s_m[JAC ? 288 : 1], s_R[9], s_t[3];
@@ -844,13 +847,20 @@ void instance_kernel(InstanceArgs a) {
     const int tid = (int)threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), i = (int)blockIdx.x;
     const uint64_t lt_mask = (1ull << lane) - 1ull;
     if (tid == 0) s_nslow = 0;
+    if (a.src) {
+        constexpr int WORDS = sizeof(InstDev) / sizeof(uint4);
+        if (tid < WORDS) reinterpret_cast<uint4*>(a.inst + i)[tid] = reinterpret_cast<const uint4*>(a.src + i)[tid];
+        __threadfence();
+    }
     __syncthreads();
+    const InstDev* inst = a.inst;
+    asm volatile("" : "+s"(inst));   // its reads stay behind the copy
     // detection: wavefront w takes a contiguous range of the steps of 64 points, PPL
     // steps at a time: their point reads, then their table reads, then their cells are
     // out together, so a pass over 2,048 points waits three times
     int wcount = 0, st0;
     {
-        const InstDev in = as_const(a.inst)[i];
+        const InstDev in = as_const(inst)[i];
         const GridDev G = as_const(a.grids)[in.grid];
         const int np = (int)in.pt_count, ns = (np + SP - 1) / SP, st1 = (w + 1) * ns / NW;
         st0 = w * ns / NW;
@@ -915,7 +925,7 @@ void instance_kernel(InstanceArgs a) {
     // work items: kChunk contacts each
     const int items = (cnt + kChunk - 1) / kChunk;
     if (tid == 0 && in.tile_count) {
-        a.tile_active[in.tile_begin] = cnt;
+        for (int t = 0; t < in.tile_count; ++t) a.tile_active[in.tile_begin + t] = t ? 0 : cnt;
         a.tile_chunk0[in.tile_begin] = in.chunk0;
     }
     if (tid < (np + kChunk - 1) / kChunk)
@@ -1042,7 +1052,7 @@ void instance_kernel(InstanceArgs a) {
     if (a.host_dst) __threadfence_system();   // the stores reach host memory before the launch completes
     if (a.done) {
         __syncthreads();
-        if (tid == 0) __hip_atomic_store(a.done + i, a.counters[CNT_CALL], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (tid == 0) __hip_atomic_store(a.done + i, a.call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 

@@ -251,7 +251,7 @@ int atac_batch_eval_host(atac_batch b, uint32_t flags, double* fm, double* Km, d
  * evaluations, Simulation.cpp:1081-1117; the reference calls computeForce* per force
  * object each time). The evaluation writes the results straight into pinned host memory
  * and a number behind them that the host waits for. Small batches of small instances are
- * two launches; others replay the upload and the evaluation as one HIP graph (captured
+ * one launch; others replay the upload and the evaluation as one HIP graph (captured
  * on first use per flag combination and again after the batch's buffers change). Same
  * instance rules, meaning and layout as those two; not for use while the batch's own
  * stream is being captured. */

@@ -10,7 +10,7 @@ from atac.batch import batch_from_workload
 pytestmark = pytest.mark.gpu
 
 SIZES = [0, 1, 63, 64, 65, 255, 256, 257, 1023, 1025, 2047, 2048]
-SIZES_WRENCH = SIZES + [2049, 4095, 4096]
+SIZES_WRENCH = SIZES + [2049, 4095, 4096, 4097, 8191, 8192]
 # the sums run in one order; a contact's terms are rounded alike up to the compiler's
 # choice of fused multiply-adds: a few ulp of the largest term (FP32 2^-24, FP64 2^-53,
 # times some 10 operations and a cancellation of up to 100 between the terms)
@@ -61,7 +61,7 @@ def test_equals_the_pipeline(gpu, kw, precise):
     _compare(_workload(SIZES if kw else SIZES_WRENCH, 0.05), dict(kw, precise=precise))
 
 
-@pytest.mark.parametrize("sizes", [[2049], [4097], [40] * 129, [40] * 257], ids=["2049", "4097", "258", "514"])
+@pytest.mark.parametrize("sizes", [[2049], [8193], [40] * 129, [40] * 257], ids=["2049", "8193", "258", "514"])
 def test_around_the_rule(gpu, sizes):
     """One point more than the range, and batches on either side of an instance (two) per CU."""
     _compare(_workload(sizes, 0.05), {"deriv": True, "p6": True})
