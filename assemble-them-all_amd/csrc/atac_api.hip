@@ -123,6 +123,7 @@ struct atac_batch_s {
     float* d_slow_diag = nullptr;     // 4 x slow_cap
     double* d_part = nullptr;         // chunk_cap x part_width
     int64_t part_width = 0;
+    bool split_items = false;         // a workgroup per work item in the contact and adjoint kernels
     int grid_detect = 0, grid_contact[2][3] = {{0, 0, 0}, {0, 0, 0}}, grid_vjp[2] = {0, 0};
     int grid_slow = 0;
     size_t lds_detect = 0;
@@ -696,11 +697,14 @@ static int plan(atac_batch b, const atac_tuning* t) {
         b->grid_detect = std::max(b->nq, std::min(b->n_tiles, nb * b->n_cu));
     else
         b->grid_detect = std::max(b->nq, b->nq * max_q);
-    const int64_t items = std::max<int64_t>(1, (b->chunk_cap + 3) / 4);
+    // about an item per tile: up to eight tiles per CU, a workgroup per item (ItemWalk)
+    b->split_items = b->n_tiles <= 8 * b->n_cu;
+    const int64_t items = b->split_items ? std::min<int64_t>(std::max<int64_t>(1, b->chunk_cap), 8 * (int64_t)b->n_cu)
+                                         : std::max<int64_t>(1, (b->chunk_cap + 3) / 4);
     for (int pr = 0; pr < 2; ++pr) {
         for (int m = 0; m < 3; ++m) {
             int nc = 0;
-            ATAC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nc, contact_kernel_ptr(m, pr == 1), 256, 0));
+            ATAC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nc, contact_kernel_ptr(m, pr == 1, false), 256, 0));
             // the Km/Dm mode: a work item per workgroup, as many workgroups as are
             // resident. The others: a wavefront per work item (of the most the
             // evaluation can push; those past its count return at once), so that the
@@ -951,8 +955,8 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
         ca.counters = counters(b); ca.chunk_cap = (int32_t)b->chunk_cap; ca.partial = b->d_part;
         ca.g_fm = g_fused;
         hipEvent_t t3 = stage_begin(b, st);
-        if (fused) ATAC_HIP(launch_fused(ca, precise, b->grid_vjp[precise ? 1 : 0], st));
-        else ATAC_HIP(launch_contact(ca, mode, precise, b->grid_contact[precise ? 1 : 0][mode], st));
+        if (fused) ATAC_HIP(launch_fused(ca, precise, b->split_items, b->grid_vjp[precise ? 1 : 0], st));
+        else ATAC_HIP(launch_contact(ca, mode, precise, b->split_items, b->grid_contact[precise ? 1 : 0][mode], st));
         stage_end(b, ST_CONTACT, t3, st);
     }
     ReduceArgs ra{};
@@ -1005,7 +1009,7 @@ static int enqueue_vjp(atac_batch b, const double* g_fm, const atac_gradients* g
         va.rec = precise ? (const void*)b->d_rec64 : (const void*)b->d_rec32; va.slow_diag = b->d_slow_diag;
         va.counters = counters(b); va.chunk_cap = (int32_t)b->chunk_cap; va.g_fm = g_fm; va.partial = b->d_part;
         hipEvent_t t0 = stage_begin(b, st);
-        ATAC_HIP(launch_vjp(va, precise, b->grid_vjp[precise ? 1 : 0], st));
+        ATAC_HIP(launch_vjp(va, precise, b->split_items, b->grid_vjp[precise ? 1 : 0], st));
         stage_end(b, ST_VJP, t0, st);
     }
     ReduceArgs ra{};

@@ -178,12 +178,12 @@ struct TouchedArgs {
 hipError_t launch_detect(const DetectArgs& a, int block, int ppl, int grid, size_t lds, hipStream_t st);
 const void* detect_kernel_ptr(int block, int ppl);
 hipError_t launch_slow(const SlowArgs& a, bool precise, int grid, hipStream_t st);
-hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, int grid, hipStream_t st);
-const void* contact_kernel_ptr(int mode, bool precise);
-hipError_t launch_vjp(const VjpArgs& a, bool precise, int grid, hipStream_t st);
+// split: a workgroup per work item instead of a wavefront (the Km/Dm mode has always one)
+hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, bool split, int grid, hipStream_t st);
+const void* contact_kernel_ptr(int mode, bool precise, bool split);
+hipError_t launch_vjp(const VjpArgs& a, bool precise, bool split, int grid, hipStream_t st);
 // the wrench and the adjoint of a known cotangent in one pass (no records kept)
-hipError_t launch_fused(const ContactArgs& a, bool precise, int grid, hipStream_t st);
-const void* vjp_kernel_ptr(bool precise);
+hipError_t launch_fused(const ContactArgs& a, bool precise, bool split, int grid, hipStream_t st);
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st);
 // the same after the Km/Dm pass: rows of kJacRow, dst = fm, dfm_dp6, Km, Dm
 hipError_t launch_reduce_jacobian(const ReduceArgs& a, hipStream_t st);

@@ -16,7 +16,7 @@
 //                  record slots and work items of the bounded record pool.
 //   slow_kernel    the FP64 FD-stencil samples of the few active points whose
 //                  stencil leaves their cell.
-//   contact_kernel work items of kChunk active points, one wavefront each: builds
+//   contact_kernel work items of kChunk active points (ItemWalk): builds
 //                  the records (sample of phi, grad phi, Hessian) and sums the
 //                  wrench (optionally the p6 column) into the item's partial row.
 //   jacobian_kernel the same with Km/Dm, one workgroup per item: sums the wrench,
@@ -431,24 +431,56 @@ __device__ __forceinline__ Rec item_record(const GridDev& G, const InstDev& in, 
     return r;
 }
 
-// Work items of kChunk records, one wavefront each: the wrench (and p6 column) of
-// every record, summed per lane, then over the wave in a fixed order into the
-// item's partial row.
-template <bool P6, typename R>
+// Work items of kChunk records: how the contact and adjoint kernels deal them out.
+// SPLIT: a workgroup per item, a wavefront per 64 records, whose sums are added in LDS;
+// otherwise a wavefront per item, its lanes taking the records 64 apart in turn. With
+// few items (about one per tile) the second leaves the SIMDs with one or two wavefronts
+// and four dependent steps each; with many, the first only adds sums. 96 FP64 instances
+// (244 tiles), an evaluation and its adjoint: 57 us by wavefront, 46 by workgroup; the
+// fused pass over 300 instances (1,500 tiles) 76.8 and 75.5.
+template <bool SPLIT>
+struct ItemWalk {
+    static constexpr int U = SPLIT ? 1 : kChunk / 64;   // records per lane
+    static __device__ __forceinline__ int begin() { return SPLIT ? (int)blockIdx.x : wave_id(); }
+    static __device__ __forceinline__ int step() { return SPLIT ? (int)gridDim.x : wave_count(); }
+    static __device__ __forceinline__ int first() { return SPLIT ? (int)(threadIdx.x & ~63u) : 0; }   // of the wavefront's records
+    // the item's row from its wavefronts' column sums (lane k: component k)
+    template <int NF>
+    static __device__ __forceinline__ void store(double (*s_row)[NF], double col, double* dst) {
+        const int lane = threadIdx.x & 63;
+        if constexpr (SPLIT) {
+            if (lane < NF) s_row[threadIdx.x >> 6][lane] = col;
+            __syncthreads();
+            if (threadIdx.x < NF) {
+                const int k = threadIdx.x;
+                dst[k] = s_row[0][k] + s_row[1][k] + s_row[2][k] + s_row[3][k];
+            }
+            __syncthreads();
+        } else if (lane < NF) {
+            dst[lane] = col;
+        }
+    }
+};
+
+// The wrench (and p6 column) of every record, summed per lane, then over the wave in a
+// fixed order into the item's partial row.
+template <bool P6, typename R, bool SPLIT>
 __global__ __launch_bounds__(256) void contact_kernel(ContactArgs a) {
     using Rec = typename RecOf<R>::type;
     constexpr int NF = P6 ? 24 : 12;
-    constexpr int U = kChunk / 64;   // records per lane
-    __shared__ double s_red[4][64 * NF];
+    using Walk = ItemWalk<SPLIT>;
+    constexpr int U = Walk::U;
+    __shared__ double s_red[4][64 * NF], s_row[4][NF];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int total = min(a.counters[CNT_CHUNKS], a.chunk_cap);
-    for (int c = wave_id(); c < total; c += wave_count()) {
+    for (int c = Walk::begin(); c < total; c += Walk::step()) {
         const ChunkDev ch = as_const(a.chunks)[c];
         const InstDev in = as_const(a.inst)[ch.inst];
         const GridDev G = as_const(a.grids)[in.grid];
-        const int n = ch.n;
-        Rec* rec = static_cast<Rec*>(a.rec) + ch.rec0;
-        const auto act = as_global(a.act) + ch.rec0;
+        const int64_t rec0 = ch.rec0 + Walk::first();
+        const int n = ch.n - Walk::first();
+        Rec* rec = static_cast<Rec*>(a.rec) + rec0;
+        const auto act = as_global(a.act) + rec0;
         const InstR<R> I = make_inst<R>(in);
         LaneAcc<R> acc[NF];
 #pragma unroll
@@ -486,8 +518,7 @@ __global__ __launch_bounds__(256) void contact_kernel(ContactArgs a) {
         double lv[NF];
 #pragma unroll
         for (int k = 0; k < NF; ++k) lv[k] = acc[k].value();
-        const double col = lds_column_sums<NF>(&s_red[w][0], lv);
-        if (lane < NF) dst[lane] = col;
+        Walk::template store<NF>(s_row, n > 0 ? lds_column_sums<NF>(&s_red[w][0], lv) : 0.0, dst);
     }
 }
 
@@ -543,19 +574,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // wrench summed as contact_kernel's mode 0 sums it and its adjoint as
 // vjp_kernel does, per lane over the records 64 apart in turn, then over the
 // lanes: the partial row is fm 12 | kVjpOut. No record is written.
-template <typename R>
+template <typename R, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 3 : 1))) void fused_kernel(ContactArgs a) {
     using Rec = typename RecOf<R>::type;
-    __shared__ double s_red[4][64 * kVjpOut];
+    using Walk = ItemWalk<SPLIT>;
+    __shared__ double s_red[4][64 * kVjpOut], s_row[4][kFmOut], s_vrow[4][kVjpOut];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int total = min(a.counters[CNT_CHUNKS], a.chunk_cap);
-    for (int c = wave_id(); c < total; c += wave_count()) {
+    for (int c = Walk::begin(); c < total; c += Walk::step()) {
         const ChunkDev ch = as_const(a.chunks)[c];
         const InstDev in = as_const(a.inst)[ch.inst];
         const GridDev G = as_const(a.grids)[in.grid];
-        const int n = ch.n;
-        const Rec* rec = static_cast<const Rec*>(a.rec) + ch.rec0;
-        const auto act = as_global(a.act) + ch.rec0;
+        const int64_t rec0 = ch.rec0 + Walk::first();
+        const int n = min(64 * Walk::U, ch.n - Walk::first());
+        const Rec* rec = static_cast<const Rec*>(a.rec) + rec0;
+        const auto act = as_global(a.act) + rec0;
         const InstR<R> I = make_inst<R>(in);
         R gb[12];
 #pragma unroll
@@ -593,31 +626,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
         double lf[kFmOut];
 #pragma unroll
         for (int k = 0; k < kFmOut; ++k) lf[k] = acc[k].value();
-        const double colf = lds_column_sums<kFmOut>(&s_red[w][0], lf);
-        if (lane < kFmOut) dst[lane] = colf;
+        Walk::template store<kFmOut>(s_row, n > 0 ? lds_column_sums<kFmOut>(&s_red[w][0], lf) : 0.0, dst);
         double lv[kVjpOut];
 #pragma unroll
         for (int k = 0; k < kVjpOut; ++k) lv[k] = (double)vacc[k];
-        double col = lds_column_sums<kVjpOut>(&s_red[w][0], lv);
+        double col = n > 0 ? lds_column_sums<kVjpOut>(&s_red[w][0], lv) : 0.0;
         if (lane == 24 || lane == 25) col *= in.kn_chain;   // d/d kn = kn_chain * d/d kn_eff (ForceGeneralSDFContact.cpp:155-156)
-        if (lane < kVjpOut) dst[kFmOut + lane] = col;
+        Walk::template store<kVjpOut>(s_vrow, col, dst + kFmOut);
     }
 }
 
 // ------------------------------------------------------------------ batched adjoint
 // The adjoint of every record of a work item, with d(loss)/d(wrench) of its
 // instance, summed into the item's partial row (kVjpOut).
-template <typename R>
+template <typename R, bool SPLIT>
 __global__ __launch_bounds__(256) void vjp_kernel(VjpArgs a) {
     using Rec = typename RecOf<R>::type;
-    __shared__ double s_red[4][64 * kVjpOut];
+    using Walk = ItemWalk<SPLIT>;
+    __shared__ double s_red[4][64 * kVjpOut], s_row[4][kVjpOut];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int total = min(a.counters[CNT_CHUNKS], a.chunk_cap);
-    for (int c = wave_id(); c < total; c += wave_count()) {
+    for (int c = Walk::begin(); c < total; c += Walk::step()) {
         const ChunkDev ch = as_const(a.chunks)[c];
+        if (ch.n == 0) continue;   // its row is not read
         const InstDev in = as_const(a.inst)[ch.inst];
-        const int n = ch.n;
-        const Rec* rec = static_cast<const Rec*>(a.rec) + ch.rec0;
+        const int n = min(64 * Walk::U, ch.n - Walk::first());
+        const Rec* rec = static_cast<const Rec*>(a.rec) + ch.rec0 + Walk::first();
         const InstR<R> I = make_inst<R>(in);
         R gb[12];
 #pragma unroll
@@ -625,25 +659,32 @@ __global__ __launch_bounds__(256) void vjp_kernel(VjpArgs a) {
         R acc[kVjpOut];
 #pragma unroll
         for (int k = 0; k < kVjpOut; ++k) acc[k] = (R)0;
-        // the next iteration's record is loaded while this one is computed
-        Rec cur;
-        if (lane < n) cur = load_rec(rec + lane);
-        for (int j = lane; j < n; j += 64) {
-            Rec nxt;
-            if (j + 64 < n) nxt = load_rec(rec + j + 64);
+        const auto add = [&](const Rec& r) {
             ContactFwd<R> s;
-            record_decode(cur, a.slow_diag, in, s);
+            record_decode(r, a.slow_diag, in, s);
             contact_forward<R>(I, s, nullptr);
             contact_vjp<R, true>(I, s, gb, acc);
-            cur = nxt;
+        };
+        if constexpr (SPLIT) {
+            if (lane < n) add(load_rec(rec + lane));
+        } else {
+            // the next iteration's record is loaded while this one is computed
+            Rec cur;
+            if (lane < n) cur = load_rec(rec + lane);
+            for (int j = lane; j < n; j += 64) {
+                Rec nxt = cur;
+                if (j + 64 < n) nxt = load_rec(rec + j + 64);
+                add(cur);
+                cur = nxt;
+            }
         }
         double* dst = a.partial + (int64_t)c * kVjpOut;
         double lv[kVjpOut];
 #pragma unroll
         for (int k = 0; k < kVjpOut; ++k) lv[k] = (double)acc[k];
-        double col = lds_column_sums<kVjpOut>(&s_red[w][0], lv);
+        double col = n > 0 ? lds_column_sums<kVjpOut>(&s_red[w][0], lv) : 0.0;
         if (lane == 24 || lane == 25) col *= in.kn_chain;   // d/d kn = kn_chain * d/d kn_eff (ForceGeneralSDFContact.cpp:155-156)
-        if (lane < kVjpOut) dst[lane] = col;
+        Walk::template store<kVjpOut>(s_row, col, dst);
     }
 }
 
@@ -1444,36 +1485,37 @@ hipError_t launch_slow(const SlowArgs& a, bool precise, int grid, hipStream_t st
     return hipGetLastError();
 }
 
-template <typename R>
+template <typename R, bool SPLIT>
 static const void* contact_ptr_t(int mode) {
-    return mode == 0   ? (const void*)&contact_kernel<false, R>
-           : mode == 1 ? (const void*)&contact_kernel<true, R> : (const void*)&jacobian_kernel<R>;
+    return mode == 0   ? (const void*)&contact_kernel<false, R, SPLIT>
+           : mode == 1 ? (const void*)&contact_kernel<true, R, SPLIT> : (const void*)&jacobian_kernel<R>;
 }
 
-const void* contact_kernel_ptr(int mode, bool precise) {
-    return precise ? contact_ptr_t<double>(mode) : contact_ptr_t<float>(mode);
+const void* contact_kernel_ptr(int mode, bool precise, bool split) {
+    if (split) return precise ? contact_ptr_t<double, true>(mode) : contact_ptr_t<float, true>(mode);
+    return precise ? contact_ptr_t<double, false>(mode) : contact_ptr_t<float, false>(mode);
 }
 
-hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, int grid, hipStream_t st) {
+hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, bool split, int grid, hipStream_t st) {
     ContactArgs args = a;
     void* params[] = {&args};
-    return hipLaunchKernel(contact_kernel_ptr(mode, precise), dim3(grid), dim3(256), params, 0, st);
+    return hipLaunchKernel(contact_kernel_ptr(mode, precise, split), dim3(grid), dim3(256), params, 0, st);
 }
 
-hipError_t launch_vjp(const VjpArgs& a, bool precise, int grid, hipStream_t st) {
-    if (precise) hipLaunchKernelGGL(vjp_kernel<double>, dim3(grid), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(vjp_kernel<float>, dim3(grid), dim3(256), 0, st, a);
-    return hipGetLastError();
+hipError_t launch_vjp(const VjpArgs& a, bool precise, bool split, int grid, hipStream_t st) {
+    VjpArgs args = a;
+    void* params[] = {&args};
+    const void* k = split ? (precise ? (const void*)&vjp_kernel<double, true> : (const void*)&vjp_kernel<float, true>)
+                          : (precise ? (const void*)&vjp_kernel<double, false> : (const void*)&vjp_kernel<float, false>);
+    return hipLaunchKernel(k, dim3(grid), dim3(256), params, 0, st);
 }
 
-hipError_t launch_fused(const ContactArgs& a, bool precise, int grid, hipStream_t st) {
-    if (precise) hipLaunchKernelGGL(fused_kernel<double>, dim3(grid), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(fused_kernel<float>, dim3(grid), dim3(256), 0, st, a);
-    return hipGetLastError();
-}
-
-const void* vjp_kernel_ptr(bool precise) {
-    return precise ? (const void*)&vjp_kernel<double> : (const void*)&vjp_kernel<float>;
+hipError_t launch_fused(const ContactArgs& a, bool precise, bool split, int grid, hipStream_t st) {
+    ContactArgs args = a;
+    void* params[] = {&args};
+    const void* k = split ? (precise ? (const void*)&fused_kernel<double, true> : (const void*)&fused_kernel<float, true>)
+                          : (precise ? (const void*)&fused_kernel<double, false> : (const void*)&fused_kernel<float, false>);
+    return hipLaunchKernel(k, dim3(grid), dim3(256), params, 0, st);
 }
 
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st) {
