@@ -141,6 +141,21 @@ ATAC_HD int node_w(float v) {
 #endif
 }
 
+// Keys of the traversal's stack entries: the squared box distance e rounded toward
+// zero to FP32, with the child's lane (0 .. 7) in the last three bits, so the keys of a
+// node's children differ. The key only orders them: the lane bits can raise it above e.
+// bvh_key_bound, without them, never exceeds e, and is what an entry is dropped by.
+ATAC_HD uint32_t bvh_key(double e, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (__float_as_uint(__double2float_rz(e)) & ~7u) | (uint32_t)lane;
+#else
+    float f = (float)e;
+    if ((double)f > e) f = nextafterf(f, 0.0f);
+    return (__builtin_bit_cast(uint32_t, f) & ~7u) | (uint32_t)lane;
+#endif
+}
+ATAC_HD double bvh_key_bound(uint32_t key) { return (double)__builtin_bit_cast(float, key & ~7u); }
+
 // Pseudonormal of face f for a closest point with barycentric coordinates b
 // (libigl pseudonormal_test: two coordinates <= eps -> the remaining vertex's
 // normal; one -> the normal of the edge opposite that corner; none -> the face's).

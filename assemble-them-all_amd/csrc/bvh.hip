@@ -207,9 +207,9 @@ __device__ __forceinline__ double group_min(double v) {
 // p; gl = the lane's place in it): each lane tests one child box of a node, or one
 // triangle of a leaf, and keeps the best triangle it has tested; the group's bound
 // is the least of them. A node's children whose boxes can hold a closer point go on
-// the group's stack (LDS), the nearest on top: an entry is the child's code and a
-// key, the squared box distance rounded toward zero with the lane in its last three
-// bits, so keys differ and never exceed the distance. One lane per point is limited
+// the group's stack (LDS), the nearest on top: an entry is the child's code and its
+// key (bvh_key). Boxes as near as the best triangle are visited too: among equal
+// distances the smallest face wins, whatever the order. One lane per point is limited
 // by its chain of dependent reads (1.08 ms for 60,000 points, 4,224 triangles, under
 // one wavefront per SIMD, and a stack in scratch); eight lanes make eight times the
 // wavefronts and an eighth of the steps.
@@ -227,7 +227,7 @@ __device__ __forceinline__ MeshHit mesh_closest(const MeshDev& M, D3 p, int gl, 
     auto pop = [&]() {
         while (sp > 0) {
             const uint2 e = stack[--sp];
-            if ((double)__uint_as_float(e.y) <= best) { code = (int)e.x; return true; }
+            if (bvh_key_bound(e.y) <= best) { code = (int)e.x; return true; }
         }
         return false;
     };
@@ -236,7 +236,7 @@ __device__ __forceinline__ MeshHit mesh_closest(const MeshDev& M, D3 p, int gl, 
             const float4 lo = nodes[2 * (code + gl)], hi = nodes[2 * (code + gl) + 1];
             const double e = box_dist2(p, lo, hi);
             const bool push = node_w(lo.w) != kBvhEmpty && e <= best;
-            const uint32_t key = push ? (__float_as_uint(__double2float_rz(e)) & ~7u) | (uint32_t)gl : 0u;
+            const uint32_t key = push ? bvh_key(e, gl) : 0u;
             int rank = 0;   // children on top of this one are nearer, those below it farther
             rank += group_xor<1>(key) > key;
             rank += group_xor<2>(key) > key;

@@ -7,6 +7,7 @@
 #include <vector>
 #include "atac.h"
 #include "atac_compose.h"
+#include "bvh_host.h"
 #include "contact_math.h"
 
 using namespace atac;
@@ -255,6 +256,76 @@ int hc_jacobian_blocks(const float* vals, const int32_t n[3], const double minb[
             if (c < 12) Km[12 * r + c] = v;
             else Dm[12 * r + c - 12] = v;
         }
+    return 0;
+}
+
+// Closest triangles of n points: mesh_closest's traversal (the 8 lanes of a group in
+// turn, their votes taken as the kernel takes them) and, next to it, every triangle
+// tested. Returns 0, or 1 when the mesh is refused.
+int hc_mesh_closest(const double* V, int64_t nv, const int64_t* F, int64_t nf, const double* x, int64_t n, double* d2,
+                    int32_t* face, double* brute_d2, int32_t* brute_face, int32_t* deepest) {
+    MeshHost m;
+    if (!mesh_build(V, nv, F, nf, m).empty()) return 1;
+    *deepest = 0;
+    for (int64_t i = 0; i < n; ++i) {
+        const D3 p = d3(x[3 * i], x[3 * i + 1], x[3 * i + 2]);
+        MeshHit lane[kBvhWidth], all;
+        struct Entry { int code; uint32_t key; } stack[kBvhStack];
+        double best = INFINITY;
+        int code = 0, sp = 0;
+        auto pop = [&]() {
+            while (sp > 0) {
+                const Entry e = stack[--sp];
+                if (bvh_key_bound(e.key) <= best) { code = e.code; return true; }
+            }
+            return false;
+        };
+        for (bool more = true; more;) {
+            while (more && code >= 0) {
+                uint32_t key[kBvhWidth];
+                int at[kBvhWidth], n_push = 0;
+                bool push[kBvhWidth];
+                for (int g = 0; g < kBvhWidth; ++g) {
+                    const float4 lo = m.nodes[2 * (code + g)], hi = m.nodes[2 * (code + g) + 1];
+                    const double e = box_dist2(p, lo, hi);
+                    at[g] = node_w(lo.w);
+                    push[g] = at[g] != kBvhEmpty && e <= best;
+                    key[g] = push[g] ? bvh_key(e, g) : 0u;
+                    n_push += push[g] ? 1 : 0;
+                }
+                for (int g = 0; g < kBvhWidth; ++g) {
+                    int rank = 0;
+                    for (int o = 0; o < kBvhWidth; ++o) rank += o != g && key[o] > key[g] ? 1 : 0;
+                    if (push[g]) stack[sp + rank] = Entry{at[g], key[g]};
+                }
+                sp += n_push;
+                *deepest = std::max(*deepest, sp);
+                more = pop();
+            }
+            if (!more) break;
+            const int at = (-code - 1) * kBvhWidth;
+            for (int g = 0; g < kBvhWidth; ++g) {
+                const int t = m.tri[at + g];
+                if (t == kNoTriangle) continue;
+                const double* v = &m.tv[(int64_t)at * 9 + g];
+                lane[g].test(p, d3(v[0], v[8], v[16]), d3(v[24], v[32], v[40]), d3(v[48], v[56], v[64]), t < 0 ? ~t : t, t < 0);
+            }
+            for (const MeshHit& h : lane) best = std::min(best, h.d2);
+            more = pop();
+        }
+        d2[i] = best;
+        face[i] = -1;
+        for (const MeshHit& h : lane)
+            if (h.f >= 0 && h.d2 == best && (face[i] < 0 || h.f < face[i])) face[i] = h.f;
+        for (const int32_t t : m.tri) {
+            if (t == kNoTriangle) continue;
+            const int64_t f = t < 0 ? ~t : t;
+            const auto vert = [&](int c) { const double* q = V + 3 * F[3 * f + c]; return d3(q[0], q[1], q[2]); };
+            all.test(p, vert(0), vert(1), vert(2), (int)f, t < 0);
+        }
+        brute_d2[i] = all.d2;
+        brute_face[i] = all.f;
+    }
     return 0;
 }
 

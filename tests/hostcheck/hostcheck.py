@@ -15,7 +15,7 @@ def build():
     cmd = ["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O2", "-std=c++17", "-fPIC", "-shared",
            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
            "-I" + os.path.join(_REPO, "assemble-them-all_amd", "csrc"), "-I" + os.path.join(_REPO, "include"),
-           os.path.join(_HERE, "hostcheck.hip"), "-o", _LIB]
+           os.path.join(_HERE, "hostcheck.hip"), os.path.join(_REPO, "assemble-them-all_amd", "csrc", "bvh.hip"), "-o", _LIB]
     r = subprocess.run(cmd, stderr=subprocess.PIPE, text=True)
     if r.returncode != 0:
         errs = [ln for ln in r.stderr.splitlines() if "packed-fp32-ops" not in ln]
@@ -30,7 +30,7 @@ def _stale():
         return True
     csrc = os.path.join(_REPO, "assemble-them-all_amd", "csrc")
     srcs = [os.path.join(_HERE, "hostcheck.hip"), os.path.join(_REPO, "include", "atac.h")]
-    srcs += [os.path.join(csrc, f) for f in os.listdir(csrc) if f.endswith(".h")]
+    srcs += [os.path.join(csrc, f) for f in os.listdir(csrc) if f.endswith(".h") or f == "bvh.hip"]
     return max(os.path.getmtime(f) for f in srcs) > os.path.getmtime(_LIB)
 
 
@@ -150,3 +150,18 @@ def jacobian_blocks(grid, pts_f32, inst):
     lib().hc_jacobian_blocks(_vp(vals), _vp(n), _vp(mn), _vp(mx), _vp(d), _vp(px), _vp(py), _vp(pz),
                              C.c_int64(len(p)), C.byref(inst), _vp(Km), _vp(Dm), _vp(counts))
     return Km, Dm, counts
+
+
+def mesh_closest(V, F, x):
+    """The BVH traversal's (squared distance, face) per point, the same over all triangles, and the
+    most stack entries in use."""
+    V = np.ascontiguousarray(V, dtype=np.float64)
+    F = np.ascontiguousarray(F, dtype=np.int64)
+    x = np.ascontiguousarray(x, dtype=np.float64)
+    d2, bd2 = np.empty(len(x)), np.empty(len(x))
+    f, bf = np.empty(len(x), dtype=np.int32), np.empty(len(x), dtype=np.int32)
+    deepest = C.c_int32(0)
+    r = lib().hc_mesh_closest(_vp(V), C.c_int64(len(V)), _vp(F), C.c_int64(len(F)), _vp(x), C.c_int64(len(x)), _vp(d2),
+                              _vp(f), _vp(bd2), _vp(bf), C.byref(deepest))
+    assert r == 0, "mesh refused"
+    return d2, f, bd2, bf, deepest.value

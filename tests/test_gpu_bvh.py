@@ -8,6 +8,7 @@ import pytest
 from atac import _lib as L
 from atac.bvh import BVHMesh
 from atac.workloads import box_mesh, icosphere, torus
+from meshes import split_box
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -49,6 +50,25 @@ def test_distance_normal_matches_oracle(name):
     print(name, "faces equal", same.mean(), "normals equal", agree.mean(), flush=True)
     assert agree[same].all()
     assert agree.mean() > 0.999, agree.mean()
+
+
+@pytest.mark.parametrize("points", ["lattice", "vertices", "random"])
+def test_equally_near_triangles(points):
+    """A box of 3,072 triangles whose coordinates, and those of the lattice, are small powers of
+    two apart, so the distances are exact on both sides: equal faces and normals, the smallest face
+    among the equally near. At random points equal distances."""
+    V, F = split_box(0.5, 16)
+    rng = np.random.default_rng(23)
+    x = {"lattice": lambda: rng.integers(-16, 17, (6000, 3)) / 32.0, "vertices": lambda: V,
+         "random": lambda: rng.uniform(-0.5, 0.5, (20000, 3))}[points]()
+    d, n, f = BVHMesh(V, F).distance_normal(x)
+    od, on, of = O.mesh_distance_normal(V, F, x)
+    if points == "random":
+        # d of a few FP64 roundings; a dropped triangle changes d^2 by 1e-7 of itself
+        np.testing.assert_allclose(d, od, rtol=1e-14, atol=1e-15)
+    else:
+        assert np.array_equal(d, od) and np.array_equal(f, of)
+        np.testing.assert_allclose(n, on, rtol=0, atol=1e-15)
 
 
 def test_bad_meshes():
