@@ -135,6 +135,18 @@ struct atac_batch_s {
     bool cap_precise = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
+    // what graph records; recorded again, for poses that are not rotations, on the first
+    // launch with such poses after a capture that had none
+    struct Captured {
+        uint32_t flags = 0;
+        const double* g_fm = nullptr;
+        atac_outputs out{};
+        atac_gradients grads{};
+        bool has_out = false, has_grads = false, rigid = false;
+    } captured;
+    hipGraph_t graph_any = nullptr;
+    hipGraphExec_t graph_any_exec = nullptr;
+    bool all_rigid = true;        // every instance's poses are rotations (InstDev::rigid)
     hipStream_t cap_stream = nullptr;
     // device staging for the synchronous host-buffer entry points
     double* h_out = nullptr;      // fm 12 | p6 12 | Km 144 | Dm 144 per instance
@@ -415,6 +427,10 @@ static void compose_for(atac_batch b, const atac_instance& s, InstDev& d) {
     d.gbox = P.d_gbox ? P.d_gbox + 8 * P.gseg[s.segment] : nullptr;
 }
 
+static void note_rigid(atac_batch b) {
+    b->all_rigid = std::all_of(b->inst_dev.begin(), b->inst_dev.end(), [](const InstDev& d) { return d.rigid != 0; });
+}
+
 // The same for an instance of a planned batch: its place in the plan stays.
 static void recompose(atac_batch b, int i, const atac_instance& s) {
     InstDev& d = b->inst_dev[i];
@@ -477,6 +493,13 @@ static int check_instances(atac_batch b, const atac_instance* inst, int32_t n) {
 
 constexpr int kXcds = 8;   // MI355X: 8 XCDs, each with its own L2
 
+static void drop_graph(atac_batch b) {
+    if (b->graph_exec) { (void)hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
+    if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
+    if (b->graph_any_exec) { (void)hipGraphExecDestroy(b->graph_any_exec); b->graph_any_exec = nullptr; }
+    if (b->graph_any) { (void)hipGraphDestroy(b->graph_any); b->graph_any = nullptr; }
+}
+
 static void release_plan(atac_batch b) {
     dfree(b->d_tiles); dfree(b->d_order); dfree(b->d_tq_begin); dfree(b->d_counters);
     dfree(b->d_tile_active); dfree(b->d_tile_chunk0); dfree(b->d_chunks); dfree(b->d_tile_live);
@@ -485,8 +508,7 @@ static void release_plan(atac_batch b) {
     b->part_width = 0;
     b->rec_valid = false;
     b->rec_captured = false;
-    if (b->graph_exec) { (void)hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
-    if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
+    drop_graph(b);
 }
 
 // Width of a work item's partial row for an evaluation mode (0 wrench, 1 + p6,
@@ -494,7 +516,7 @@ static void release_plan(atac_batch b) {
 // partial row per work item: mode 0-2 the evaluation's, 3 the adjoint's, 4 the
 // fused pass's (wrench and adjoint)
 static int64_t part_width_of(int mode) {
-    return mode == 4 ? kFmOut + kVjpOut : mode == 3 ? kVjpOut : (mode == 2 ? kJacRow : (mode == 1 ? 24 : 12));
+    return mode == 4 ? kFmOut + kVjpOut : mode == 3 ? kVjpOut : (mode == 2 ? kJvpRow : (mode == 1 ? 24 : 12));
 }
 
 // Allocates what an evaluation of this mode and precision (or the adjoint,
@@ -517,8 +539,7 @@ static int ensure_buffers(atac_batch b, int mode, bool precise) {
     const int64_t w = std::max<int64_t>(part_width_of(mode), part_width_of(3));
     if (!rc && b->chunk_cap > 0 && w > b->part_width) {
         // a captured graph holds the old buffer: it is dropped with it
-        if (b->graph_exec) { (void)hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
-        if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
+        drop_graph(b);
         (void)hipDeviceSynchronize();
         dfree(b->d_part);
         rc = dalloc(&b->d_part, (size_t)(b->chunk_cap * w));
@@ -704,7 +725,7 @@ static int plan(atac_batch b, const atac_tuning* t) {
     for (int pr = 0; pr < 2; ++pr) {
         for (int m = 0; m < 3; ++m) {
             int nc = 0;
-            ATAC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nc, contact_kernel_ptr(m, pr == 1, false), 256, 0));
+            ATAC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nc, contact_kernel_ptr(m, pr == 1, false, true), 256, 0));
             // the Km/Dm mode: a work item per workgroup, as many workgroups as are
             // resident. The others: a wavefront per work item (of the most the
             // evaluation can push; those past its count return at once), so that the
@@ -742,6 +763,7 @@ int atac_batch_create(const atac_grid* grids, int32_t n_grids, const atac_points
     b->inst_dev.resize(n_inst);
     for (int i = 0; i < n_inst; ++i)
         compose_for(b, inst[i], b->inst_dev[i]);
+    note_rigid(b);
     rc = ensure_cls(b);
     if (rc) { atac_batch_destroy(b); return rc; }
     std::vector<GridDev> gd(n_grids);
@@ -795,6 +817,7 @@ static int compose_instances(atac_batch b, const atac_instance* inst, int32_t n_
     int rc = check_instances(b, inst, n_inst);
     if (rc) return rc;
     for (int i = 0; i < n_inst; ++i) recompose(b, i, inst[i]);
+    note_rigid(b);
     rc = ensure_cls(b);   // a new col_th needs its classification table
     if (rc) return rc;
     b->inst.assign(inst, inst + n_inst);
@@ -901,6 +924,14 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
     int rc = ensure_buffers(b, mode, precise);
     if (rc) return rc;
     if (b->inst.empty()) return ATAC_OK;
+    bool rigid = b->all_rigid;
+    if (mode == 2 && rigid && st != b->cap_stream) {
+        // another program's graph may be replayed with other poses (the batch's own are
+        // recorded for both)
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        ATAC_HIP(hipStreamIsCapturing(st, &cs));
+        rigid = cs == hipStreamCaptureStatusNone;
+    }
     void* rec = precise ? (void*)b->d_rec64 : (void*)b->d_rec32;
     // groups whose boxes reach only cells where no point can be active are dropped
     // first; that pass also clears the counters (all points are contacts with
@@ -917,7 +948,7 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
         if (out) { ia.fm = out->fm; ia.p6 = out->dfm_dp6; ia.Km = out->Km; ia.Dm = out->Dm; ia.n_active = out->n_active; }
         ia.overflow_out = overflow_out; ia.host_dst = overflow_out ? 1 : 0; ia.done = done;
         ia.call = call; ia.src = call ? b->pin_inst : nullptr;
-        ATAC_HIP(launch_instance(ia, mode, precise, (int)b->inst.size(), st));
+        ATAC_HIP(launch_instance(ia, mode, precise, rigid, (int)b->inst.size(), st));
         return eval_done(b, false, precise, st);
     }
     if (!cull) ATAC_HIP(launch_reset(b->d_counters, CNT_WORDS, st));
@@ -956,7 +987,7 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
         ca.g_fm = g_fused;
         hipEvent_t t3 = stage_begin(b, st);
         if (fused) ATAC_HIP(launch_fused(ca, precise, b->split_items, b->grid_vjp[precise ? 1 : 0], st));
-        else ATAC_HIP(launch_contact(ca, mode, precise, b->split_items, b->grid_contact[precise ? 1 : 0][mode], st));
+        else ATAC_HIP(launch_contact(ca, mode, precise, b->split_items, rigid, b->grid_contact[precise ? 1 : 0][mode], st));
         stage_end(b, ST_CONTACT, t3, st);
     }
     ReduceArgs ra{};
@@ -985,7 +1016,7 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
     ra.host_dst = overflow_out ? 1 : 0;   // the host call's outputs are its pinned staging
     ra.done = done;
     hipEvent_t t3 = stage_begin(b, st);
-    ATAC_HIP(mode == 2 ? launch_reduce_jacobian(ra, st) : launch_reduce(ra, st));
+    ATAC_HIP(mode == 2 ? launch_reduce_jacobian(ra, rigid, st) : launch_reduce(ra, st));
     stage_end(b, ST_REDUCE, t3, st);
     return eval_done(b, fused, precise, st);
 }
@@ -1046,6 +1077,33 @@ int atac_batch_vjp(atac_batch b, const double* g_fm, const atac_gradients* out, 
     return enqueue_vjp(b, g_fm, out, (hipStream_t)stream);
 }
 
+// Records b->captured on the batch's own stream, for the poses the batch holds.
+static int record_graph(atac_batch b, hipGraph_t* graph, hipGraphExec_t* exec) {
+    const atac_batch_s::Captured& c = b->captured;
+    const atac_outputs* out = c.has_out ? &c.out : nullptr;
+    const atac_gradients* grads = c.has_grads ? &c.grads : nullptr;
+    ATAC_HIP(hipStreamSynchronize(b->cap_stream));
+    const bool timing = b->timing;
+    b->timing = false;
+    ATAC_HIP(hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal));
+    b->rec_captured = false;
+    int rc;
+    if (b->graph_fused) {
+        rc = enqueue_eval(b, c.flags, out, b->cap_stream, nullptr, c.g_fm, grads);
+    } else {
+        rc = enqueue_eval(b, c.flags, out, b->cap_stream);
+        if (!rc && c.g_fm) rc = enqueue_vjp(b, c.g_fm, grads, b->cap_stream);
+    }
+    b->timing = timing;
+    hipGraph_t g = nullptr;
+    hipError_t e = hipStreamEndCapture(b->cap_stream, &g);
+    if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
+    if (e != hipSuccess) return fail(ATAC_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+    *graph = g;
+    ATAC_HIP(hipGraphInstantiate(exec, g, nullptr, nullptr, 0));
+    return ATAC_OK;
+}
+
 int atac_batch_graph_capture(atac_batch b, uint32_t flags, const atac_outputs* out, const double* g_fm,
                              const atac_gradients* grads) {
     if (!b) return fail(ATAC_ERR_INVALID, "atac_batch_graph_capture: null batch");
@@ -1055,33 +1113,25 @@ int atac_batch_graph_capture(atac_batch b, uint32_t flags, const atac_outputs* o
     int rc = ensure_buffers(b, fused ? 4 : mode_of(flags), (flags & ATAC_EVAL_PRECISE) != 0);
     if (!rc && g_fm) rc = ensure_buffers(b, 3, (flags & ATAC_EVAL_PRECISE) != 0);
     if (rc) return rc;
-    if (b->graph_exec) { (void)hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
-    if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
-    ATAC_HIP(hipStreamSynchronize(b->cap_stream));
-    const bool timing = b->timing;
-    b->timing = false;
-    ATAC_HIP(hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal));
-    b->rec_captured = false;
+    drop_graph(b);
     b->graph_fused = fused;
-    if (fused) {
-        rc = enqueue_eval(b, flags, out, b->cap_stream, nullptr, g_fm, grads);
-    } else {
-        rc = enqueue_eval(b, flags, out, b->cap_stream);
-        if (!rc && g_fm) rc = enqueue_vjp(b, g_fm, grads, b->cap_stream);
-    }
-    b->timing = timing;
-    hipGraph_t g = nullptr;
-    hipError_t e = hipStreamEndCapture(b->cap_stream, &g);
-    if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
-    if (e != hipSuccess) return fail(ATAC_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-    b->graph = g;
-    ATAC_HIP(hipGraphInstantiate(&b->graph_exec, b->graph, nullptr, nullptr, 0));
-    return ATAC_OK;
+    atac_batch_s::Captured& c = b->captured;
+    c = {flags, g_fm, out ? *out : atac_outputs{}, grads ? *grads : atac_gradients{}, out != nullptr, grads != nullptr,
+         b->all_rigid};
+    return record_graph(b, &b->graph, &b->graph_exec);
 }
 
 int atac_batch_graph_launch(atac_batch b, void* stream) {
     if (!b || !b->graph_exec) return fail(ATAC_ERR_STATE, "atac_batch_graph_launch: no captured graph");
-    ATAC_HIP(hipGraphLaunch(b->graph_exec, (hipStream_t)stream));
+    hipGraphExec_t exec = b->graph_exec;
+    if (b->captured.rigid && !b->all_rigid && mode_of(b->captured.flags) == 2) {
+        if (!b->graph_any_exec) {
+            const int rc = record_graph(b, &b->graph_any, &b->graph_any_exec);
+            if (rc) return rc;
+        }
+        exec = b->graph_any_exec;
+    }
+    ATAC_HIP(hipGraphLaunch(exec, (hipStream_t)stream));
     if (b->graph_fused) {
         b->rec_valid = false;   // its pass overwrote the work lists and kept no records
     } else if (b->rec_captured) {   // the graph's evaluation leaves its records for atac_batch_vjp
@@ -1515,7 +1565,8 @@ int atac_batch_eval_instances_host(atac_batch b, const atac_instance* inst, int3
         else rc = wait_done(done, n, *call, st);
         return rc ? rc : host_results(b, P, Pn, fm, Km, Dm, dfm_dp6, n_active, "atac_batch_eval_instances_host");
     }
-    const uint32_t key = flags | ((Km || Dm) ? 1u << 8 : 0u) | (dfm_dp6 ? 1u << 9 : 0u);
+    const uint32_t key = flags | ((Km || Dm) ? 1u << 8 : 0u) | (dfm_dp6 ? 1u << 9 : 0u) |
+                         (mode == 2 && !b->all_rigid ? 1u << 10 : 0u);
     atac_batch_s::HostGraph& hg = b->host_graphs[key];
     if (!hg.e || hg.gen != b->buf_gen) {
         // capture: instance upload and evaluation, whose reduction writes the results
@@ -1825,7 +1876,7 @@ int atac_bvh_force_host(atac_mesh m, const atac_instance* inst, const double* xi
     int rc = dalloc(&dx, (size_t)std::max<int64_t>(3 * n, 1));
     if (!rc) rc = dalloc(&dout, (size_t)kBvhOut);
     if (!rc) rc = dalloc(&dna, 1);
-    if (!rc) rc = dalloc(&dpart, (size_t)(nb * kJacRow));
+    if (!rc) rc = dalloc(&dpart, (size_t)(nb * kJvpRow));
     if (!rc) rc = dalloc(&dcnt, (size_t)nb);
     hipError_t e = hipSuccess;
     std::vector<double> h(kBvhOut);
@@ -1876,7 +1927,7 @@ int atac_bvh_force_noalloc(atac_mesh m, const atac_instance* inst, const double*
     // every workgroup writes its whole row and count, and the reduction reads
     // only the rows of this launch: nothing needs clearing between calls
     a.part = part;
-    a.part_cnt = reinterpret_cast<int64_t*>(part + kBvhMaxBlocks * kJacRow);
+    a.part_cnt = reinterpret_cast<int64_t*>(part + kBvhMaxBlocks * kJvpRow);
     ATAC_HIP(launch_bvh_force(a, (hipStream_t)stream));
     return ATAC_OK;
 }

@@ -19,8 +19,19 @@ inline void set_f32_copies(InstDev& d) {
     }
     d.fkn = (float)d.kn; d.fkt = (float)d.kt; d.fmu = (float)d.mu;
     d.fdamping = (float)d.damping; d.fcontact_scale = (float)d.contact_scale;
-    d.fpad0 = 0.0f;
     for (float& f : d.fpad) f = 0.0f;
+}
+
+// R^T R = I to kRigidTol (a NaN is none).
+constexpr double kRigidTol = 0x1p-46;
+inline bool is_rotation(const double R[9]) {
+    bool ok = true;
+    for (int i = 0; i < 3; ++i)
+        for (int j = 0; j <= i; ++j) {
+            const double q = R[i] * R[j] + R[3 + i] * R[3 + j] + R[6 + i] * R[6 + j];
+            ok = ok && std::fabs(q - (i == j ? 1.0 : 0.0)) <= kRigidTol;
+        }
+    return ok;
 }
 
 inline void compose_instance(const atac_instance& s, const GridDev& G, const float* px, const float* py, const float* pz,
@@ -63,6 +74,7 @@ inline void compose_instance(const atac_instance& s, const GridDev& G, const flo
     d.py = py;
     d.pz = pz;
     d.pt_count = n_points;
+    d.rigid = is_rotation(R1) && is_rotation(R2) ? 1 : 0;
     d.grid = s.grid;
     d.chunk0 = 0;
     set_f32_copies(d);

@@ -75,7 +75,7 @@ struct ContactArgs {
     int32_t* counters;
     int32_t chunk_cap;
     int32_t pad;
-    double* partial;            // per work item: fm 12 | p6 12 | Km/Dm block sums 135 (as the mode has them);
+    double* partial;            // per work item: fm 12 | p6 12 | Km/Dm block sums 135 or columns 288 (as the mode has them);
                                 // the fused pass: fm 12 | kVjpOut
     const double* g_fm;         // the fused pass: d(loss)/d(wrench) per instance (n_inst x 12)
 };
@@ -179,15 +179,16 @@ hipError_t launch_detect(const DetectArgs& a, int block, int ppl, int grid, size
 const void* detect_kernel_ptr(int block, int ppl);
 hipError_t launch_slow(const SlowArgs& a, bool precise, int grid, hipStream_t st);
 // split: a workgroup per work item instead of a wavefront (the Km/Dm mode has always one)
-hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, bool split, int grid, hipStream_t st);
-const void* contact_kernel_ptr(int mode, bool precise, bool split);
+// rigid (Km/Dm): every instance's poses are rotations, in this and each later run of a captured launch
+hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, bool split, bool rigid, int grid, hipStream_t st);
+const void* contact_kernel_ptr(int mode, bool precise, bool split, bool rigid);
 hipError_t launch_vjp(const VjpArgs& a, bool precise, bool split, int grid, hipStream_t st);
 // the wrench and the adjoint of a known cotangent in one pass (no records kept)
 hipError_t launch_fused(const ContactArgs& a, bool precise, bool split, int grid, hipStream_t st);
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st);
-// the same after the Km/Dm pass: rows of kJacRow, dst = fm, dfm_dp6, Km, Dm
-hipError_t launch_reduce_jacobian(const ReduceArgs& a, hipStream_t st);
-hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, int n_inst, hipStream_t st);
+// the same after the Km/Dm pass: rows of kJvpRow, dst = fm, dfm_dp6, Km, Dm
+hipError_t launch_reduce_jacobian(const ReduceArgs& a, bool rigid, hipStream_t st);
+hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, bool rigid, int n_inst, hipStream_t st);
 // instance records, and (call != nullptr) the number of the call to counters[CNT_CALL],
 // from host memory the device can read
 hipError_t launch_upload(const InstDev* src, InstDev* dst, int n, const int32_t* call, int32_t* counters, hipStream_t st);

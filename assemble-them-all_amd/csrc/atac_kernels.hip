@@ -526,42 +526,55 @@ __global__ __launch_bounds__(256) void contact_kernel(ContactArgs a) {
 // Work items of kChunk records, one workgroup each, wavefront w taking records
 // [64 w, 64 w + 64), one per lane: the wrench, the p6 column and the blocks Km and
 // Dm are made of (contact_jac), summed over the item into its partial row
-// (kJacRow values). Bound by instruction issue: about 1,700 instructions per 64
+// (kJacRow of its kJvpRow values; poses that are not rotations fill it). Bound by instruction issue: about 1,700 instructions per 64
 // contacts, where 24 tangents per contact and their 288 wave sums took about 13,000
 // (an evaluation of 256 poses x 5,000 points with Km/Dm: 149 -> 57 us; of 26 poses
 // from host memory: 132 -> 80 us). 64 contacts per wavefront rather than 256:
-// small batches have few items and need the waves.
-template <typename R>
+// small batches have few items and need the waves. RIGID: every instance's poses are
+// rotations. Otherwise each item takes the form of its instance (InstDev::rigid), which
+// costs the blocks 4 % (FP32) and 25 % (FP64, spilled registers) of an evaluation.
+template <typename R, bool RIGID>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void jacobian_kernel(ContactArgs a) {
     using Rec = typename RecOf<R>::type;
     __shared__ double s_col[4][JacColumns::SIZE];
-    __shared__ double s_part[4][kJacRowPad];
+    __shared__ double s_part[4][RIGID ? kJacRowPad : kJvpRowPad];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int total = min(a.counters[CNT_CHUNKS], a.chunk_cap);
     for (int c = (int)blockIdx.x; c < total; c += (int)gridDim.x) {
         const ChunkDev ch = as_const(a.chunks)[c];
         const int n = ch.n - 64 * w;   // this wavefront's records
-        if (n > 0) {
-            const InstDev in = as_const(a.inst)[ch.inst];
+        const bool rigid = RIGID || as_const(a.inst)[ch.inst].rigid != 0;
+        // lanes past the end repeat the last record; their rows are not summed
+        const int64_t j = ch.rec0 + 64 * w + min(lane, n - 1);
+        const auto forward = [&](const InstDev& in, ContactFwd<R>& s, R p6[12]) {
             const GridDev G = as_const(a.grids)[in.grid];
-            // lanes past the end repeat the last record; their rows are not summed
-            const int j = 64 * w + min(lane, n - 1);
-            Rec* rec = static_cast<Rec*>(a.rec) + ch.rec0 + j;
-            const uint32_t e = (as_global(a.act) + ch.rec0)[j], off = e & ~kActSlow;
-            const Rec r = item_record(G, in, e, as_global(in.px)[off], as_global(in.py)[off], as_global(in.pz)[off], rec);
-            ContactFwd<R> s;
-            R p6[12];
+            const uint32_t e = as_global(a.act)[j], off = e & ~kActSlow;
+            const Rec r = item_record(G, in, e, as_global(in.px)[off], as_global(in.py)[off], as_global(in.pz)[off],
+                                      static_cast<Rec*>(a.rec) + j);
             record_decode(r, a.slow_diag, in, s);
             contact_forward<R>(make_inst<R>(in), s, p6);
+        };
+        ContactFwd<R> s;
+        R p6[12];
+        if (n > 0 && rigid) {
+            const InstDev in = as_const(a.inst)[ch.inst];
+            forward(in, s, p6);
             put_jac_row<R>(JacColumns{&s_col[w][0], &s_part[w][0], lane, n}, jac_inst(in), s, p6);
+        } else if (!RIGID && n > 0) {
+            // the record again, behind an opaque pointer: nothing of this rare branch is formed
+            // (and kept in registers) ahead of the other
+            const InstDev* again = a.inst;
+            asm volatile("" : "+s"(again));
+            const InstDev in = as_const(again)[ch.inst];
+            forward(in, s, p6);
+            put_jvp_row<R>(JvpColumns{&s_col[w][0], &s_part[w][0], lane, n}, make_inst<R>(in), s, p6);
         }
         __syncthreads();
-        const int k = (int)threadIdx.x;
-        if (k < kJacRow && ch.n > 0) {
+        for (int k = (int)threadIdx.x; k < (rigid ? kJacRow : kJvpRow) && ch.n > 0; k += 256) {
             double v = s_part[0][k];
             for (int i = 1; i < 4; ++i)
                 if (ch.n > 64 * i) v += s_part[i][k];
-            a.partial[(int64_t)c * kJacRow + k] = v;
+            a.partial[(int64_t)c * kJvpRow + k] = v;
         }
         __syncthreads();
     }
@@ -770,18 +783,21 @@ __global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
 // instance: thread k sums component k of the instance's rows, in tile order and
 // each tile's items in order (the rows of 64 tiles listed in LDS first, so that
 // their reads go out together); the wrench and p6 sums are outputs, and the
-// threads form the 288 entries of Km and Dm from the block sums (jac_entry).
+// threads form the 288 entries of Km and Dm from the block sums (jac_entry). Rows
+// of tangent columns (InstDev::rigid 0) have two components a thread.
+template <bool RIGID>
 __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
     constexpr int kRows = 64 * 32;   // a tile holds at most 8192 / kChunk items
     __shared__ int s_rows[kRows];
     __shared__ int s_nrows, s_nact;
-    __shared__ double s_sum[kJacRow], s_m[288], s_R[9], s_t[3];
+    __shared__ double s_sum[RIGID ? kJacRow : kJvpRow], s_m[288], s_R[9], s_t[3];
     const int k = (int)threadIdx.x, i = (int)blockIdx.x;
     const bool ovf = a.counters[CNT_OVERFLOW] != 0;
     if (a.overflow_out && i == 0 && k == 0) *a.overflow_out = ovf ? 1 : 0;
     const InstDev in = as_const(a.inst)[i];
     const auto part = as_global(a.partial);
-    double sum = 0.0;
+    const bool rigid = RIGID || in.rigid != 0;
+    double sum = 0.0, sum2 = 0.0;
     int nact = 0;
     for (int g0 = 0; g0 < in.tile_count; g0 += 64) {
         if (k < 64) {
@@ -802,20 +818,23 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
         }
         __syncthreads();
         const int nr = s_nrows;
-        if (k < kJacRow) {
+        const auto add_rows = [&](double& to, int comp) {
             int j = 0;
             for (; j + 8 <= nr; j += 8) {
                 double v[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = part[(int64_t)s_rows[j + u] * kJacRow + k];
+                for (int u = 0; u < 8; ++u) v[u] = part[(int64_t)s_rows[j + u] * kJvpRow + comp];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) sum += v[u];
+                for (int u = 0; u < 8; ++u) to += v[u];
             }
-            for (; j < nr; ++j) sum += part[(int64_t)s_rows[j] * kJacRow + k];
-        }
+            for (; j < nr; ++j) to += part[(int64_t)s_rows[j] * kJvpRow + comp];
+        };
+        if (k < kJacRow || !rigid) add_rows(sum, k);
+        if (!rigid && k < kJvpRow - 256) add_rows(sum2, k + 256);
         __syncthreads();
     }
-    if (k < kJacRow) s_sum[k] = ovf ? __builtin_nan("") : sum;
+    if (k < kJacRow || !rigid) s_sum[k] = ovf ? __builtin_nan("") : sum;
+    if (!rigid && k < kJvpRow - 256) s_sum[k + 256] = ovf ? __builtin_nan("") : sum2;
     if (k < 64) {
         nact = (int)wave_sum((double)nact);
         if (k == 0) s_nact = nact;
@@ -831,12 +850,14 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
     if (k >= 12 && k < 24 && a.dst[1]) a.dst[1][(int64_t)i * 12 + k - 12] = s_sum[k];
     if (k == 0 && a.n_active) a.n_active[i] = ovf ? -1 : s_nact;
     if (a.dst[2] || a.dst[3]) {
-        for (int e = k; e < 288; e += 256) s_m[e] = jac_element(s_sum + 24, s_sum + 9, s_t, e / 24, e % 24);
+        if (rigid)
+            for (int e = k; e < 288; e += 256) s_m[e] = jac_element(s_sum + 24, s_sum + 9, s_t, e / 24, e % 24);
         __syncthreads();
         for (int e = k; e < 288; e += 256) {
             const int m = e / 144, row = (e % 144) / 12, col = e % 12;
             double* dst = m ? a.dst[3] : a.dst[2];
-            if (dst) dst[(int64_t)i * 144 + e % 144] = jac_entry(s_m, s_R, row, 12 * m + col);
+            if (dst)
+                dst[(int64_t)i * 144 + e % 144] = rigid ? jac_entry(s_m, s_R, row, 12 * m + col) : jvp_entry(s_sum, m, row, col);
         }
     }
     if (a.host_dst) __threadfence_system();   // the stores reach host memory before the launch completes
@@ -863,13 +884,14 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
 // slot), for the adjoint; the sums run in the pipeline's order, per work item, then the
 // items in turn. A host call's instances are read from its pinned copy: an upload of
 // its own costs 4 us.
-template <int MODE, typename R>
+// RIGID: as for jacobian_kernel (MODE 2).
+template <int MODE, typename R, bool RIGID>
 __global__ __launch_bounds__(kInstBlock) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 2 : 4)))
 void instance_kernel(InstanceArgs a) {
     using Rec = typename RecOf<R>::type;
     constexpr int NT = kInstBlock, NW = NT / 64, PPL = 4, SP = 64, ITEMS = NW / 4;
     constexpr bool JAC = MODE == 2;
-    constexpr int NF = JAC ? kJacRow : MODE == 1 ? 24 : 12;
+    constexpr int NF = JAC ? (RIGID ? kJacRow : kJvpRow) : MODE == 1 ? 24 : 12;
     constexpr int GROUPS = 64 / kStencil;
     __shared__ uint16_t s_list[inst_points(MODE)];   // the active offsets in point order, bit 15 = slow path
     __shared__ double s_stencil[NW][GROUPS][kStencil];
@@ -878,7 +900,7 @@ void instance_kernel(InstanceArgs a) {
     static_assert(sizeof s_val >= 4 * inst_points(MODE), "both lists lie in s_val");
     uint16_t* const s_q = reinterpret_cast<uint16_t*>(s_val);
     uint16_t* const s_slow = s_q + inst_points(MODE);
-    __shared__ double s_part[NW][JAC ? kJacRowPad : 1];
+    __shared__ double s_part[NW][JAC ? (RIGID ? kJacRowPad : kJvpRowPad) : 1];
     __shared__ double s_row[ITEMS][JAC ? 1 : NF];
     __shared__ double s_sum[NF], s_m[JAC ? 288 : 1], s_R[9], s_t[3];
     __shared__ int s_count[NW], s_nslow;
@@ -1012,7 +1034,9 @@ void instance_kernel(InstanceArgs a) {
     }
     __syncthreads();
     // ITEMS work items at a time, a wavefront per 64 contacts
-    double total = 0.0;   // thread k < NF: component k of the instance's sums
+    const bool rigid = RIGID || in.rigid != 0;
+    const int nf = JAC && rigid ? kJacRow : NF;
+    double total = 0.0;   // thread k < nf: component k of the instance's sums
     const InstR<R> I = make_inst<R>(in);
     for (int m0 = 0; m0 < items; m0 += ITEMS) {
         const int start = (m0 + (w >> 2)) * kChunk, n = max(0, min(kChunk, cnt - start));
@@ -1020,14 +1044,27 @@ void instance_kernel(InstanceArgs a) {
         if (nw > 0) {
             const int j = start + p0 + min(lane, nw - 1);   // lanes past the end repeat the last record, not summed
             const uint32_t e = s_list[j], off = e & 0x7fffu;
-            const Rec r = item_record(G, in, off | (e >> 15 ? kActSlow : 0u), px[off], py[off], pz[off], rec + j);
             ContactFwd<R> s;
             R p6[12];
-            record_decode(r, a.slow_diag, in, s);
-            contact_forward<R>(I, s, MODE >= 1 ? p6 : nullptr);
+            const auto forward = [&](const InstDev& in, const InstR<R>& I) {
+                const Rec r = item_record(G, in, off | (e >> 15 ? kActSlow : 0u), px[off], py[off], pz[off], rec + j);
+                record_decode(r, a.slow_diag, in, s);
+                contact_forward<R>(I, s, MODE >= 1 ? p6 : nullptr);
+            };
             if constexpr (JAC) {
-                put_jac_row<R>(JacColumns{&s_val[w][0], &s_part[w][0], lane, nw}, jac_inst(in), s, p6);
+                if (RIGID || rigid) {
+                    forward(in, I);
+                    put_jac_row<R>(JacColumns{&s_val[w][0], &s_part[w][0], lane, nw}, jac_inst(in), s, p6);
+                } else {   // a branch of its own, as in jacobian_kernel
+                    const InstDev* third = a.inst;
+                    asm volatile("" : "+s"(third));
+                    const InstDev in3 = as_const(third)[i];
+                    const InstR<R> I3 = make_inst<R>(in3);
+                    forward(in3, I3);
+                    put_jvp_row<R>(JvpColumns{&s_val[w][0], &s_part[w][0], lane, nw}, I3, s, p6);
+                }
             } else {
+                forward(in, I);
 #pragma unroll
                 for (int k = 0; k < 12; ++k) s_val[w][lane * NF + k] = (double)s.f[k];
                 if constexpr (MODE == 1) {
@@ -1054,7 +1091,7 @@ void instance_kernel(InstanceArgs a) {
             if (tid < NF) {
                 for (int h = 0; h < ITEMS && m0 + h < items; ++h) total += s_row[h][tid];
             }
-        } else if (tid < NF) {
+        } else if (tid < nf) {
             for (int h = 0; h < ITEMS && m0 + h < items; ++h) {
                 const int nh = min(kChunk, cnt - (m0 + h) * kChunk);
                 double v = s_part[4 * h][tid];
@@ -1065,7 +1102,7 @@ void instance_kernel(InstanceArgs a) {
         }
         __syncthreads();
     }
-    if (tid < NF) s_sum[tid] = total;
+    if (tid < nf) s_sum[tid] = total;
     if constexpr (JAC) {
         if (tid == NT - 1) {
             const JacInst J = jac_inst(in);
@@ -1079,12 +1116,13 @@ void instance_kernel(InstanceArgs a) {
     if (MODE >= 1 && tid >= 12 && tid < 24 && a.p6) a.p6[(int64_t)i * 12 + tid - 12] = s_sum[MODE >= 1 ? tid : 0];
     if (tid == 0 && a.n_active) a.n_active[i] = cnt;
     if constexpr (JAC) {
-        if (tid < 288) s_m[JAC ? tid : 0] = jac_element(s_sum + 24, s_sum + 9, s_t, tid / 24, tid % 24);
+        if (tid < 288 && rigid) s_m[JAC ? tid : 0] = jac_element(s_sum + 24, s_sum + 9, s_t, tid / 24, tid % 24);
         __syncthreads();
         if (tid < 288) {
             const int m = tid / 144, row = (tid % 144) / 12, col = tid % 12;
             double* dst = m ? a.Dm : a.Km;
-            if (dst) dst[(int64_t)i * 144 + tid % 144] = jac_entry(s_m, s_R, row, 12 * m + col);
+            if (dst)
+                dst[(int64_t)i * 144 + tid % 144] = rigid ? jac_entry(s_m, s_R, row, 12 * m + col) : jvp_entry(s_sum, m, row, col);
         }
     }
     if (a.host_dst) __threadfence_system();   // the stores reach host memory before the launch completes
@@ -1486,20 +1524,21 @@ hipError_t launch_slow(const SlowArgs& a, bool precise, int grid, hipStream_t st
 }
 
 template <typename R, bool SPLIT>
-static const void* contact_ptr_t(int mode) {
+static const void* contact_ptr_t(int mode, bool rigid) {
     return mode == 0   ? (const void*)&contact_kernel<false, R, SPLIT>
-           : mode == 1 ? (const void*)&contact_kernel<true, R, SPLIT> : (const void*)&jacobian_kernel<R>;
+           : mode == 1 ? (const void*)&contact_kernel<true, R, SPLIT>
+           : rigid     ? (const void*)&jacobian_kernel<R, true> : (const void*)&jacobian_kernel<R, false>;
 }
 
-const void* contact_kernel_ptr(int mode, bool precise, bool split) {
-    if (split) return precise ? contact_ptr_t<double, true>(mode) : contact_ptr_t<float, true>(mode);
-    return precise ? contact_ptr_t<double, false>(mode) : contact_ptr_t<float, false>(mode);
+const void* contact_kernel_ptr(int mode, bool precise, bool split, bool rigid) {
+    if (split) return precise ? contact_ptr_t<double, true>(mode, rigid) : contact_ptr_t<float, true>(mode, rigid);
+    return precise ? contact_ptr_t<double, false>(mode, rigid) : contact_ptr_t<float, false>(mode, rigid);
 }
 
-hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, bool split, int grid, hipStream_t st) {
+hipError_t launch_contact(const ContactArgs& a, int mode, bool precise, bool split, bool rigid, int grid, hipStream_t st) {
     ContactArgs args = a;
     void* params[] = {&args};
-    return hipLaunchKernel(contact_kernel_ptr(mode, precise, split), dim3(grid), dim3(256), params, 0, st);
+    return hipLaunchKernel(contact_kernel_ptr(mode, precise, split, rigid), dim3(grid), dim3(256), params, 0, st);
 }
 
 hipError_t launch_vjp(const VjpArgs& a, bool precise, bool split, int grid, hipStream_t st) {
@@ -1527,23 +1566,25 @@ hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_jacobian(const ReduceArgs& a, hipStream_t st) {
+hipError_t launch_reduce_jacobian(const ReduceArgs& a, bool rigid, hipStream_t st) {
     if (a.n_inst <= 0) return hipSuccess;
-    hipLaunchKernelGGL(reduce_jacobian_kernel, dim3(a.n_inst), dim3(256), 0, st, a);
+    if (rigid) hipLaunchKernelGGL(reduce_jacobian_kernel<true>, dim3(a.n_inst), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(reduce_jacobian_kernel<false>, dim3(a.n_inst), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
-template <int MODE>
+template <int MODE, bool RIGID>
 static void launch_instance_m(const InstanceArgs& a, bool precise, int n_inst, hipStream_t st) {
-    if (precise) hipLaunchKernelGGL((instance_kernel<MODE, double>), dim3(n_inst), dim3(kInstBlock), 0, st, a);
-    else hipLaunchKernelGGL((instance_kernel<MODE, float>), dim3(n_inst), dim3(kInstBlock), 0, st, a);
+    if (precise) hipLaunchKernelGGL((instance_kernel<MODE, double, RIGID>), dim3(n_inst), dim3(kInstBlock), 0, st, a);
+    else hipLaunchKernelGGL((instance_kernel<MODE, float, RIGID>), dim3(n_inst), dim3(kInstBlock), 0, st, a);
 }
 
-hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, int n_inst, hipStream_t st) {
+hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, bool rigid, int n_inst, hipStream_t st) {
     if (n_inst <= 0) return hipSuccess;
-    if (mode == 0) launch_instance_m<0>(a, precise, n_inst, st);
-    else if (mode == 1) launch_instance_m<1>(a, precise, n_inst, st);
-    else launch_instance_m<2>(a, precise, n_inst, st);
+    if (mode == 0) launch_instance_m<0, true>(a, precise, n_inst, st);
+    else if (mode == 1) launch_instance_m<1, true>(a, precise, n_inst, st);
+    else if (rigid) launch_instance_m<2, true>(a, precise, n_inst, st);
+    else launch_instance_m<2, false>(a, precise, n_inst, st);
     return hipGetLastError();
 }
 

@@ -53,7 +53,7 @@ struct InstDev {
     // arithmetic (read as wave-uniform scalars)
     float fR1[9], fR2[9], fw1[3], fv1[3], fw2[3], fv2[3];
     float fkn, fkt, fmu, fdamping, fcontact_scale;
-    float fpad0;
+    int32_t rigid;      // R1 and R2 are rotations to kRigidTol: Km and Dm from the block sums (contact_jac)
     // per-cell classification of the instance's grid for its col_th (cls_fill;
     // bricked, cls_offset): 0 no active point, 1 only active points, 2 open
     const uint8_t* cls;
@@ -141,6 +141,7 @@ enum {
 constexpr int kFmOut = 12;          // wrench of both bodies
 constexpr int kP6Out = 12;          // d fm / d contact_scale (reference p6 column)
 constexpr int kJacRow = 12 + 12 + 135;   // with Km/Dm: wrench, p6 column and the Jacobian's block sums
+constexpr int kJvpRow = 12 + 12 + 288;   // the same with the 24 tangent columns instead of the blocks (InstDev::rigid 0)
 constexpr int kVjpOut = 26;         // q1(6) q2(6) phi1(6) phi2(6) kn(1) kt(1)
 
 }  // namespace atac

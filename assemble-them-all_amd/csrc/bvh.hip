@@ -316,20 +316,24 @@ __global__ __launch_bounds__(256) void mesh_distance_kernel(MeshQueryArgs a) {
 // Small steps rather than many points per workgroup: a body has a few thousand
 // points, and the traversal needs every CU (10,242 points in 6 workgroups of one
 // lane per point: 2.46 ms).
+// RIGID: the poses are rotations (InstDev::rigid); a kernel of its own, as the tangent
+// columns of others would cost this one 63 spilled registers and 8 us.
+template <bool RIGID>
 __global__ __launch_bounds__(512) void bvh_force_kernel(BvhForceArgs a) {
     __shared__ union {
         uint2 stack[kBvhStep][kBvhStackStride];
         double col[JacColumns::SIZE];
     } s;
-    __shared__ double s_part[kJacRowPad];
+    __shared__ double s_part[RIGID ? kJacRowPad : kJvpRowPad];
     __shared__ double s_hit[4][kBvhStep];   // d, normal
     __shared__ int s_idx[kBvhStep], s_m;
     const int tid = (int)threadIdx.x, gl = tid & 7, g = tid >> 3, lane = tid & 63;
     const bool p6on = (a.flags & ATAC_EVAL_P6) != 0u, deriv = (a.flags & ATAC_EVAL_DERIV) != 0u;
-    const int nrow = deriv ? kJacRow : 24;
+    constexpr int NJ = RIGID ? kJacRow : kJvpRow;
+    const int nrow = deriv ? NJ : 24;
     const int64_t b0 = (int64_t)blockIdx.x * a.block_points;
     const int64_t b1 = b0 + a.block_points < a.n ? b0 + a.block_points : a.n;
-    double acc = 0.0;   // thread k < kJacRow: component k of the row
+    double acc = 0.0;   // thread k < nrow: component k of the row
     int64_t cnt = 0;
     for (int64_t base = b0; base < b1; base += kBvhStep) {
         const int64_t i = base + g;
@@ -375,7 +379,8 @@ __global__ __launch_bounds__(512) void bvh_force_kernel(BvhForceArgs a) {
 #pragma unroll
                     for (int k = 0; k < 12; ++k) p6[k] = 0.0;
                 }
-                if (deriv) put_jac_row<double>(JacColumns{s.col, s_part, lane, m}, jac_inst(a.in), c, p6);
+                if (deriv && RIGID) put_jac_row<double>(JacColumns{s.col, s_part, lane, m}, jac_inst(a.in), c, p6);
+                else if (deriv) put_jvp_row<double>(JvpColumns{s.col, s_part, lane, m}, make_inst<double>(a.in), c, p6);
                 else put_wrench_row<double>(WaveColumns<24>{s.col, s_part, lane, m}, c, p6);
             }
         }
@@ -386,33 +391,36 @@ __global__ __launch_bounds__(512) void bvh_force_kernel(BvhForceArgs a) {
         }
         __syncthreads();
     }
-    if (tid < kJacRow) a.part[(int64_t)blockIdx.x * kJacRow + tid] = acc;
+    if (tid < NJ) a.part[(int64_t)blockIdx.x * kJvpRow + tid] = acc;
     if (tid == 0) a.part_cnt[blockIdx.x] = cnt;
 }
 
 // The workgroups' partial rows, added six rows apart in order and the six sums in
-// order; then Km and Dm from the block sums (zeros when not asked for).
+// order (three of tangent columns); then Km and Dm from the sums (zeros when not
+// asked for).
+template <bool RIGID>
 __global__ __launch_bounds__(1024) void bvh_reduce_kernel(BvhForceArgs a, int nb) {
-    constexpr int W = 160, G = 6;
-    static_assert(kJacRow <= W && G * W <= 1024, "six rows at a time");
-    __shared__ double s_sum[G][W], s_m[288], s_R[9], s_t[3];
+    constexpr int S = 960;   // threads that add rows; the last wavefront adds the counts
+    constexpr int G = RIGID ? 6 : 3, W = S / G, NJ = RIGID ? kJacRow : kJvpRow;
+    static_assert(NJ <= W, "G rows at a time");
+    __shared__ double s_sum[S], s_m[288], s_R[9], s_t[3];
     __shared__ int64_t s_cnt[64];
     const int tid = (int)threadIdx.x, g = tid / W, k = tid % W;
-    if (g < G && k < kJacRow) {
+    if (g < G && k < NJ) {
         double v = 0.0;
         int b = g;
         for (; b + 7 * G < nb; b += 8 * G) {
             double q[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) q[u] = a.part[(int64_t)(b + u * G) * kJacRow + k];
+            for (int u = 0; u < 8; ++u) q[u] = a.part[(int64_t)(b + u * G) * kJvpRow + k];
 #pragma unroll
             for (int u = 0; u < 8; ++u) v += q[u];
         }
-        for (; b < nb; b += G) v += a.part[(int64_t)b * kJacRow + k];
-        s_sum[g][k] = v;
+        for (; b < nb; b += G) v += a.part[(int64_t)b * kJvpRow + k];
+        s_sum[tid] = v;
     }
-    if (tid >= G * W) {   // the last wavefront
-        const int l = tid - G * W;
+    if (tid >= S) {
+        const int l = tid - S;
         int64_t c = 0;
         for (int b = l; b < nb; b += 64) c += a.part_cnt[b];
         s_cnt[l] = c;
@@ -424,19 +432,19 @@ __global__ __launch_bounds__(1024) void bvh_reduce_kernel(BvhForceArgs a, int nb
         }
     }
     __syncthreads();
-    if (tid < kJacRow) {
-        double v = s_sum[0][tid];
-        for (int q = 1; q < G; ++q) v += s_sum[q][tid];
-        s_sum[0][tid] = v;
+    if (tid < NJ) {
+        double v = s_sum[tid];
+        for (int q = 1; q < G; ++q) v += s_sum[q * W + tid];
+        s_sum[tid] = v;
     }
     __syncthreads();
-    if (tid < 24) a.out[tid] = s_sum[0][tid];
+    if (tid < 24) a.out[tid] = s_sum[tid];
     const bool deriv = (a.flags & ATAC_EVAL_DERIV) != 0u;
-    if (tid < 288) s_m[tid] = jac_element(&s_sum[0][24], &s_sum[0][9], s_t, tid / 24, tid % 24);
+    if (RIGID && tid < 288) s_m[tid] = jac_element(s_sum + 24, s_sum + 9, s_t, tid / 24, tid % 24);
     __syncthreads();
     if (tid < 288) {
-        const int m = tid / 144, row = (tid % 144) / 12, col = 12 * m + tid % 12;
-        a.out[24 + tid] = deriv ? jac_entry(s_m, s_R, row, col) : 0.0;
+        const int m = tid / 144, row = (tid % 144) / 12, col = tid % 12;
+        a.out[24 + tid] = !deriv ? 0.0 : RIGID ? jac_entry(s_m, s_R, row, 12 * m + col) : jvp_entry(s_sum, m, row, col);
     }
     if (tid == 0 && a.n_active) {
         int64_t c = 0;
@@ -453,12 +461,12 @@ hipError_t launch_mesh_distance(const MeshQueryArgs& a, hipStream_t st) {
 
 // ------------------------------------------------------------------ fixed scratch
 // The partial rows and contact counts of the force launches of
-// atac_bvh_force_noalloc: kBvhMaxBlocks workgroups' rows (kJacRow doubles
+// atac_bvh_force_noalloc: kBvhMaxBlocks workgroups' rows (kJvpRow doubles
 // each), then their counts (one 8-byte word each). One copy per device, held
 // until the process ends. Host code never passes `scratch` itself to a kernel
 // (on the host it names a stand-in, not device memory): it uses the address
 // hipGetSymbolAddress gave for the device, kept in g_scratch_addr.
-static __device__ __align__(256) double scratch[kBvhMaxBlocks * (kJacRow + 1)];
+static __device__ __align__(256) double scratch[kBvhMaxBlocks * (kJvpRow + 1)];
 
 namespace {
 constexpr int kScratchDevices = 64;
@@ -491,10 +499,12 @@ void* bvh_scratch_address(int device) {
 hipError_t launch_bvh_force(BvhForceArgs a, hipStream_t st) {
     a.block_points = bvh_block_points(a.n);
     const int nb = (int)bvh_force_blocks(a.n);
-    hipLaunchKernelGGL(bvh_force_kernel, dim3(nb), dim3(512), 0, st, a);
+    if (a.in.rigid) hipLaunchKernelGGL(bvh_force_kernel<true>, dim3(nb), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL(bvh_force_kernel<false>, dim3(nb), dim3(512), 0, st, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(bvh_reduce_kernel, dim3(1), dim3(1024), 0, st, a, nb);
+    if (a.in.rigid) hipLaunchKernelGGL(bvh_reduce_kernel<true>, dim3(1), dim3(1024), 0, st, a, nb);
+    else hipLaunchKernelGGL(bvh_reduce_kernel<false>, dim3(1), dim3(1024), 0, st, a, nb);
     return hipGetLastError();
 }
 

@@ -42,7 +42,7 @@ struct BvhForceArgs {
     uint32_t flags;       // ATAC_EVAL_* (DERIV, P6)
     double* out;          // 12 fm, 12 p6, 144 Km, 144 Dm
     int64_t* n_active;
-    double* part;         // per workgroup: kJacRow partial sums
+    double* part;         // per workgroup: kJvpRow partial sums (kJacRow of them for rotations)
     int64_t* part_cnt;    // per workgroup: contacts
     int64_t block_points; // points per workgroup, a multiple of kBvhStep
 };

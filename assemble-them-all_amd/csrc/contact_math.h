@@ -1188,14 +1188,9 @@ struct Tangent {
 // Column j of [Km | Dm] (j < 12: q1 then q2; 12 <= j < 24: phi1 then phi2).
 template <typename R>
 ATAC_HD Tangent<R> unit_tangent(int j) {
-    Tangent<R> t;
-    t.om1 = t.v1 = t.om2 = t.v2 = t.w1p = t.v1p = t.w2p = t.v2p = zero3<R>();
-    t.kn = 0;
-    v3<R>* slots[8] = {&t.om1, &t.v1, &t.om2, &t.v2, &t.w1p, &t.v1p, &t.w2p, &t.v2p};
-    v3<R>& s = *slots[j / 3];
-    int c = j % 3;
-    if (c == 0) s.x = 1; else if (c == 1) s.y = 1; else s.z = 1;
-    return t;
+    // selects, not a store through an index: the tangent stays in registers
+    const auto slot = [j](int k) { return mk3<R>((R)(j == 3 * k), (R)(j == 3 * k + 1), (R)(j == 3 * k + 2)); };
+    return {slot(0), slot(1), slot(2), slot(3), slot(4), slot(5), slot(6), slot(7), (R)0};
 }
 
 // Tangents of the collision values (the 14 derivative blocks of
@@ -1281,7 +1276,12 @@ ATAC_HD void contact_jvp(const InstR<R>& I, const ContactFwd<R>& s, const Tangen
 // and jac_entry form the 288 entries of Km and Dm from the sums, once per instance. In FP64 for both
 // arithmetics (FP64 and unpacked FP32 issue at the same rate on gfx950); the
 // sample, the friction branch and, in the FP32 arithmetic, the wrench are the
-// forward pass's. The poses are rigid (R^T R = I), as everywhere in the wrench.
+// forward pass's. All of this takes R1 and R2 for rotations, which the wrench itself
+// does not: where R^T R differs from I by r, Km and Dm differ from the derivative of
+// the wrench by up to 3 r of their largest entry (r 1e-7, as from FP32 poses: 5e-8 and
+// 1.4e-7). So instances with r above 2^-46 = 1.4e-14 (InstDev::rigid) sum the 24
+// tangents of contact_jvp instead: 64 roundings of an entry, which products of many
+// FP64 rotations stay below and whose effect is below the sums' own rounding.
 constexpr int kJacBlocks = 15, kJacSums = 9 * kJacBlocks;
 enum { JB_A, JB_XA, JB_V, JB_W, JB_C, JB_XC, JB_B, JB_XB, JB_YB, JB_BX, JB_XBX, JB_YBX, JB_BY, JB_XBY, JB_YBY };
 

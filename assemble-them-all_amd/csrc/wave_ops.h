@@ -109,4 +109,25 @@ __device__ __forceinline__ void put_jac_row(const JacColumns& col, const JacInst
                 });
 }
 
+// The same with the 24 tangent columns in place of the blocks, for poses that are not
+// rotations (kJvpRow values, column by column; `col` hands over one of 12 at a time and
+// writes W): the derivative of the wrench with the pose matrices as they are given.
+using JvpColumns = WaveColumns<24>;
+constexpr int kJvpRowPad = kJvpRow + JvpColumns::W;
+template <typename R>
+__device__ __forceinline__ void put_jvp_row(const JvpColumns& col, const InstR<R>& I, const ContactFwd<R>& s, const R p6[12]) {
+    put_wrench_row<R>(col, s, p6);
+    for (int j = 0; j < 24; ++j) {
+        R df[12];
+        contact_jvp<R>(I, s, unit_tangent<R>(j), df);
+        double v[12];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) v[k] = (double)df[k];
+        WaveColumns<12>{col.s, col.out + 24 + 12 * j, col.lane, col.n}.template put_all<0>(v, std::make_integer_sequence<int, 12>());
+    }
+}
+
+// Km (m = 0) or Dm (m = 1), entry (row, c), from a row summed that way.
+__device__ __forceinline__ double jvp_entry(const double* sum, int m, int row, int c) { return sum[24 + 12 * (12 * m + c) + row]; }
+
 }  // namespace atac

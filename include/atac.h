@@ -319,7 +319,7 @@ int atac_bvh_force_host(atac_mesh m, const atac_instance* inst, const double* xi
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): it calls no allocating routine. The partial
  * rows of its force workgroups live in a fixed scratch array of each device
- * (0.7 MB, held until the process ends), so n is at most
+ * (1.3 MB, held until the process ends), so n is at most
  * ATAC_BVH_NOALLOC_MAX_POINTS; larger n is refused with ATAC_ERR_INVALID.
  * Every call on a device shares that device's array: calls that overlap on one
  * GPU (other streams, other threads) race and must be serialised by the caller.

@@ -223,10 +223,11 @@ int hc_eval(const float* vals, const int32_t n[3], const double minb[3], const d
 }
 
 // Km and Dm of one force object (FP64 arithmetic) as the batched path forms them:
-// contact_jac's blocks summed over the contacts, then jac_entry.
+// contact_jac's blocks summed over the contacts, then jac_entry; for poses that are not
+// rotations (rigid[0] = 0) the tangent columns.
 int hc_jacobian_blocks(const float* vals, const int32_t n[3], const double minb[3], const double maxb[3],
                        const double d[3], const float* px, const float* py, const float* pz, int64_t npts,
-                       const atac_instance* inst, double* Km, double* Dm, int64_t counts[3]) {
+                       const atac_instance* inst, double* Km, double* Dm, int64_t counts[3], int32_t* rigid) {
     HostGrid hg;
     host_grid(vals, n, minb, maxb, d, hg);
     InstDev in;
@@ -235,13 +236,22 @@ int hc_jacobian_blocks(const float* vals, const int32_t n[3], const double minb[
     host_cls(hg, in);
     const InstR<double> I = make_inst<double>(in);
     const JacInst J = jac_inst(in);
-    double S[kJacSums] = {}, f2[3] = {};
+    double S[kJacSums] = {}, f2[3] = {}, T[288] = {};
+    *rigid = in.rigid;
     for (int64_t o = 0; o < npts; ++o) {
         if (!detect_active(hg.G, in, px[o], py[o], pz[o])) continue;
         ContactFwd<double> s;
         const bool slow = sample_via_record<double>(hg.G, in, o, s);
         contact_forward<double>(I, s, nullptr);
         ++counts[slow ? 2 : (s.fric && !s.stat ? 1 : 0)];
+        if (!in.rigid) {
+            for (int j = 0; j < 24; ++j) {
+                double col[12];
+                contact_jvp<double>(I, s, unit_tangent<double>(j), col);
+                for (int r = 0; r < 12; ++r) T[24 * r + j] += col[r];
+            }
+            continue;
+        }
         for (int k = 0; k < 3; ++k) f2[k] += s.f[9 + k];
         contact_jac(J, s.xi1, s.d, s.g, s.H, s.fric, s.stat, [&](auto b, const m3<double>& M) {
             for (int k = 0; k < 9; ++k) S[9 * decltype(b)::value + k] += M.a[k];
@@ -252,7 +262,7 @@ int hc_jacobian_blocks(const float* vals, const int32_t n[3], const double minb[
     for (int e = 0; e < 288; ++e) M[e] = jac_element(S, f2, t, e / 24, e % 24);
     for (int r = 0; r < 12; ++r)
         for (int c = 0; c < 24; ++c) {
-            const double v = jac_entry(M, J.R.a, r, c);
+            const double v = in.rigid ? jac_entry(M, J.R.a, r, c) : T[24 * r + c];
             if (c < 12) Km[12 * r + c] = v;
             else Dm[12 * r + c - 12] = v;
         }

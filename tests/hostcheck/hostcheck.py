@@ -141,15 +141,17 @@ def group_cull(grid, pts_f32, inst, gsize=256):
 
 
 def jacobian_blocks(grid, pts_f32, inst):
-    """(Km, Dm, contacts by branch [static or frictionless, dynamic, slow path]) of one force
-    object in FP64 from the summed 3x3 blocks."""
+    """(Km, Dm, contacts by branch [static or frictionless, dynamic, slow path], poses taken for
+    rotations) of one force object in FP64 as the batched path sums them."""
     vals, n, mn, mx, d = _grid_args(grid)
     p = np.ascontiguousarray(pts_f32, dtype=np.float32).reshape(-1, 3)
     px, py, pz = [np.ascontiguousarray(p[:, k]) for k in range(3)]
     Km, Dm, counts = np.zeros((12, 12)), np.zeros((12, 12)), np.zeros(3, dtype=np.int64)
+    rigid = C.c_int32(-1)
     lib().hc_jacobian_blocks(_vp(vals), _vp(n), _vp(mn), _vp(mx), _vp(d), _vp(px), _vp(py), _vp(pz),
-                             C.c_int64(len(p)), C.byref(inst), _vp(Km), _vp(Dm), _vp(counts))
-    return Km, Dm, counts
+                             C.c_int64(len(p)), C.byref(inst), _vp(Km), _vp(Dm), _vp(counts),
+                             C.byref(rigid))
+    return Km, Dm, counts, bool(rigid.value)
 
 
 def mesh_closest(V, F, x):
