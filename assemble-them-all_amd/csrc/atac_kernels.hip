@@ -312,20 +312,23 @@ __global__ __launch_bounds__(BLOCK) void detect_kernel(DetectArgs a) {
         if (base >= 0) {
             // the tile's active offsets, in ascending point order, at its pool range;
             // the contact pass builds their records (the slow pass those of the
-            // contacts whose FD stencil leaves the cell)
+            // contacts whose FD stencil leaves the cell; one the slow list has no room for
+            // is not marked, so that its record is formed all the same, as if inside its
+            // cell: the outputs are NaN, and the passes read no record nobody wrote)
             uint32_t* act = a.act + base;
             const uint32_t tb = (uint32_t)t.begin;
             for (int qi = tid; qi < cnt; qi += BLOCK) {
                 int rem = qi, ww = 0;
                 while (rem >= s_wcount[ww]) { rem -= s_wcount[ww]; ++ww; }
                 const uint32_t e = s_queue[ww * span + rem];
-                const bool slow = (e >> 15) != 0u;
-                act[qi] = (tb + (e & 0x7fffu)) | (slow ? kActSlow : 0u);
+                bool slow = (e >> 15) != 0u;
                 if (slow) {
                     const int si = atomicAdd(a.counters + CNT_SLOW, 1);
-                    if (si < a.slow_cap) a.slow[si] = SlowDev{(uint32_t)(base + qi), t.inst};
+                    slow = si < a.slow_cap;
+                    if (slow) a.slow[si] = SlowDev{(uint32_t)(base + qi), t.inst};
                     else atomicOr(a.counters + CNT_OVERFLOW, 1);
                 }
+                act[qi] = (tb + (e & 0x7fffu)) | (slow ? kActSlow : 0u);
             }
         }
         __syncthreads();

@@ -880,8 +880,8 @@ ATAC_HD void cell_of_c(const GridDev& G, const double c[3], int idx[3], double f
         const double fl = floor(c[a]);
         fd[a] = c[a] - fl;
         int i = (int)fl;
-        i = i < 0 ? 0 : (i > G.n[a] - 2 ? G.n[a] - 2 : i);
-        idx[a] = i;
+        i = i > G.n[a] - 2 ? G.n[a] - 2 : i;
+        idx[a] = i < 0 ? 0 : i;   // (last: an axis of one node has cell 0)
     }
 }
 

@@ -1,0 +1,58 @@
+"""Contacts whose finite-difference stencil leaves their cell: a face of points on a cell
+plane, where every contact takes the slow path."""
+import numpy as np
+import pytest
+import torch
+
+from atac.batch import ContactBatch, DeviceGrid, DevicePoints, make_instance
+
+pytestmark = pytest.mark.gpu
+
+N = 64
+H = 2.0 / (N - 1)
+AXIS = -1.0 + H * np.arange(N)
+PLANE = float(np.float32(AXIS[30]))   # of nodes, below the face z = 0
+
+
+def _batch(sizes, tuning=None):
+    """A half space z < 0 and point sets of these sizes on the node plane."""
+    z = np.ascontiguousarray(np.broadcast_to(AXIS[:, None, None], (N, N, N)).astype(np.float32))
+    grid = DeviceGrid(z, np.full(3, -1.0), np.full(3, -1.0 + H * (N - 1)), np.full(3, H))
+    rng = np.random.default_rng(5)
+    sets = []
+    for s in sizes:
+        p = rng.uniform(-0.9, 0.9, (s, 3))
+        p[:, 2] = PLANE
+        sets.append(p)
+    return ContactBatch([grid], [DevicePoints(np.concatenate(sets), np.cumsum([0] + list(sizes)).astype(np.int64))],
+                        _poses(len(sizes), 0.0), tuning=tuning)
+
+
+def _poses(n, lift):
+    """Aligned with the grid, raised by `lift` cells."""
+    rng = np.random.default_rng(6)
+    E1 = np.eye(4)
+    E1[2, 3] = lift * H
+    return [make_instance(0, 0, i, E1, rng.normal(0, 0.1, 6), np.eye(4), np.zeros(6), 0.01, 1e4, 1e3, 0.3, 10.0)
+            for i in range(n)]
+
+
+@pytest.mark.parametrize("precise", [False, True], ids=["fp32", "precise"])
+def test_more_than_the_slow_list_holds(gpu, precise):
+    """The pipeline's slow list holds 4,096 contacts here: an evaluation with 6,000 is reported as overflowed, in
+    NaN and n_active -1, whatever the pass that follows detection; the next one with fewer is right again."""
+    b = _batch([2000, 2000, 2000], tuning={"max_active": -1})
+    g = torch.ones((3, 12), dtype=torch.float64, device="cuda")
+    for kw in ({}, {"p6": True}, {"deriv": True}):
+        out = b.eval(precise=precise, **kw)
+        grads = b.vjp(g)
+        torch.cuda.synchronize()
+        assert (out["n_active"] == -1).all() and b.workspace()["overflowed"]
+        assert all(torch.isnan(v).all() for k, v in (*out.items(), *grads.items()) if k != "n_active")
+    out, grads = b.eval_vjp(g, precise=precise)
+    assert (out["n_active"] == -1).all() and torch.isnan(out["fm"]).all() and torch.isnan(grads["g_q1"]).all()
+    b.set_instances(_poses(3, 0.4))   # off the plane: no slow contact
+    out = b.eval(precise=precise, deriv=True)
+    torch.cuda.synchronize()
+    assert (out["n_active"] == 2000).all() and not b.workspace()["overflowed"]
+    assert all(torch.isfinite(v).all() for v in out.values())
