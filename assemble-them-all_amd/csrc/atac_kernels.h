@@ -118,7 +118,7 @@ struct ReduceArgs {
 // One workgroup per instance (instance_kernel): instances of at most that many points
 // (mode 0: the wrench alone).
 constexpr int kInstBlock = 512;
-constexpr int inst_points(int mode) { return mode == 0 ? 8192 : 2048; }
+constexpr int inst_points(int mode) { return mode == 0 ? 3072 : 2048; }
 struct InstanceArgs {
     InstDev* inst;
     const GridDev* grids;

@@ -877,9 +877,13 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
 // launches of the pipeline above are each a chain of dependent reads, with a drain
 // and a launch between them; this is one chain. 64 instances of 500 points: 14 us
 // against 30 (wrench), 21 against 33 (Km/Dm); of 2,000 points 18 against 34 and 37
-// against 37; of 8,000 points 43 against 43 and 113 against 47 (8 instances: 37
-// against 41): inst_points lies where the steps in turn have used up the gain (a round
-// of 512 contacts takes some 20 us for Km/Dm).
+// against 37. What an instance's points cost depends on the contacts among them, which
+// no rule knows beforehand: of 3,000 points with 5 % contacts (12 instances) 14.5 us
+// against 25.5, with nothing else 37.4 against 30.8; one of 8,000 17 against 24, but 84
+// against 31 (Km/Dm: a round of 512 contacts takes some 20 us). inst_points lies where
+// an instance of contacts alone takes as long as the passes of one tile each once took.
+// Slow-path contacts: 102 among 2,048 points 15 us against 23, 500 of 500 26 against
+// 26, but 2,048 of 2,048 85 against 34 (one workgroup against all of slow_kernel's).
 // Nothing is reserved with atomics: an instance's records start at its tile's slot
 // and its work items at InstDev::chunk0, so a batch needs a record per point. The
 // active list, records, work items and tile entries are left as the pipeline leaves
@@ -895,14 +899,16 @@ void instance_kernel(InstanceArgs a) {
     constexpr int NT = kInstBlock, NW = NT / 64, PPL = 4, SP = 64, ITEMS = NW / 4;
     constexpr bool JAC = MODE == 2;
     constexpr int NF = JAC ? (RIGID ? kJacRow : kJvpRow) : MODE == 1 ? 24 : 12;
-    constexpr int GROUPS = 64 / kStencil;
+    constexpr int SLOW = 128, SROW = kStencil + 1;   // slow contacts whose stencils the lanes share
     __shared__ uint16_t s_list[inst_points(MODE)];   // the active offsets in point order, bit 15 = slow path
-    __shared__ double s_stencil[NW][GROUPS][kStencil];
     __shared__ double s_val[NW][JAC ? JacColumns::SIZE : 64 * NF];
-    // until the contacts: the wavefronts' own active offsets, and the slow ones' places in s_list
-    static_assert(sizeof s_val >= 4 * inst_points(MODE), "both lists lie in s_val");
+    // until the contacts: the wavefronts' own active offsets, the slow ones' places in s_list,
+    // and of SLOW slow contacts the SDF-frame positions and the stencil's values
+    static_assert(sizeof s_val >= 4 * inst_points(MODE) + 8 * SLOW * (3 + SROW), "all of it lies in s_val");
     uint16_t* const s_q = reinterpret_cast<uint16_t*>(s_val);
     uint16_t* const s_slow = s_q + inst_points(MODE);
+    double* const s_pos = reinterpret_cast<double*>(s_slow + inst_points(MODE));
+    double* const s_stencil = s_pos + 3 * SLOW;
     __shared__ double s_part[NW][JAC ? (RIGID ? kJacRowPad : kJvpRowPad) : 1];
     __shared__ double s_row[ITEMS][JAC ? 1 : NF];
     __shared__ double s_sum[NF], s_m[JAC ? 288 : 1], s_R[9], s_t[3];
@@ -1002,38 +1008,69 @@ void instance_kernel(InstanceArgs a) {
         if (a.overflow_out) *a.overflow_out = 0;
     }
     __syncthreads();
-    // slow-path records: the 20 stencil evaluations of a contact on 20 lanes, as slow_kernel
+    // slow-path records. Many: a lane each. Up to SLOW: their positions, a lane each; the 20
+    // stencil evaluations of each over all lanes, SU of a lane's reads together; the record,
+    // a lane each
     Rec* rec = static_cast<Rec*>(a.rec) + slot0;
-    for (int base = w * GROUPS; base < s_nslow; base += NW * GROUPS) {
-        const int grp = lane / kStencil, st = lane % kStencil, k = base + grp;
-        const bool mine = grp < GROUPS && k < s_nslow;
-        const int j = mine ? s_slow[k] : 0;
+    const auto slow_point = [&](int k, Rec& r) {
+        const int j = s_slow[k];
+        const uint32_t off = s_list[j] & 0x7fffu;
+        r.a[0] = px[off]; r.a[1] = py[off]; r.a[2] = pz[off]; r.a[3] = __uint_as_float(off);
+        return j;
+    };
+    int base = 0;
+    for (; s_nslow - base > SLOW; base += NT) {
+        if (base + tid >= s_nslow) continue;
         Rec r;
-        if (mine) {
-            const uint32_t off = s_list[j] & 0x7fffu;
-            r.a[0] = px[off]; r.a[1] = py[off]; r.a[2] = pz[off]; r.a[3] = __uint_as_float(off);
-            double x[3], q[3];
-            bool accurate;
+        const int j = slow_point(base + tid, r);
+        record_slow(G, in, r, a.slow_diag ? a.slow_diag + 4 * (slot0 + j) : nullptr);
+        mark_slow_index(r, (int)(slot0 + j));
+        store_rec(rec + j, r);
+    }
+    if (base < s_nslow) {
+        constexpr int SU = 2;
+        const int m = s_nslow - base, samples = m * kStencil;
+        Rec r;
+        int j = 0;
+        if (tid < m) {
+            j = slow_point(base + tid, r);
+            double x[3];
             body2_point(in, (double)r.a[0], (double)r.a[1], (double)r.a[2], x);
-            stencil_point(x, st, q, accurate);
-            s_stencil[w][grp][st] = query_sdf64(G, q[0], q[1], q[2], accurate);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (mine && st == 0) {
-            double v[kStencil], val, g[3], H[6];
 #pragma unroll
-            for (int q = 0; q < kStencil; ++q) v[q] = s_stencil[w][grp][q];
-            stencil_combine(v, val, g, H);
+            for (int k = 0; k < 3; ++k) s_pos[3 * tid + k] = x[k];
+        }
+        __syncthreads();
+        for (int t0 = tid; t0 < samples; t0 += SU * NT) {
+            double p[SU][3];
+            Axis64 t[SU][3];
+            float v[SU][8];
+            bool accurate[SU];
+#pragma unroll
+            for (int u = 0; u < SU; ++u) {   // (past the end: the last sample again)
+                const int e = min(t0 + u * NT, samples - 1);
+                stencil_point(s_pos + 3 * (e / kStencil), e % kStencil, p[u], accurate[u]);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) t[u][k] = axis64(G, k, p[u][k]);   // (nodes in the grid for any p)
+            }
+#pragma unroll
+            for (int u = 0; u < SU; ++u) trilinear64_nodes(G, t[u][0], t[u][1], t[u][2], v[u]);
+#pragma unroll
+            for (int u = 0; u < SU; ++u) {
+                double val = trilinear64_value(t[u][0], t[u][1], t[u][2], v[u]);
+                if (!inside_box64(G, p[u][0], p[u][1], p[u][2])) val = query_sdf64(G, p[u][0], p[u][1], p[u][2], accurate[u]);
+                const int e = t0 + u * NT;
+                if (e < samples) s_stencil[SROW * (e / kStencil) + e % kStencil] = val;
+            }
+        }
+        __syncthreads();
+        if (tid < m) {
+            double val, g[3], H[6];
+            stencil_combine(reinterpret_cast<const double (&)[kStencil]>(s_stencil[SROW * tid]), val, g, H);
             float* diag = a.slow_diag ? a.slow_diag + 4 * (slot0 + j) : nullptr;
             record_slow_fill(in, val, g, H, r, diag);
             mark_slow_index(r, (int)(slot0 + j));
             store_rec(rec + j, r);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     __syncthreads();
     // ITEMS work items at a time, a wavefront per 64 contacts

@@ -123,30 +123,52 @@ ATAC_HD int64_t grid_index(const GridDev& G, int i, int j, int k) {
 
 // Trilinear interpolation at x (SDF body frame) in FP64, in the reference's
 // i -> j -> k order and with its i_pos clamp at the last node
-// (BodySDFObj.cpp:130-155). Caller guarantees x is inside [min_box, max_box].
+// (BodySDFObj.cpp:130-155): the place along each axis, the 8 nodes and the value from
+// them. Caller guarantees x is inside [min_box, max_box] (the nodes are in the grid for
+// any x; a grid has fewer than 2^27).
+struct Axis64 {
+    uint32_t at, d;   // the lower node, and how far the upper one is (0 at the last)
+    double f;
+};
+ATAC_HD Axis64 axis64(const GridDev& G, int a, double x) {
+    const double c = (x - G.minb[a]) / G.d[a];
+    int i = (int)floor(c);
+    Axis64 t;
+    t.f = c - i;
+    i = i < 0 ? 0 : (i > G.n[a] - 1 ? G.n[a] - 1 : i);
+    const uint32_t stride = a == 0 ? 1u : (uint32_t)G.n[0] * (a == 1 ? 1u : (uint32_t)G.n[1]);
+    t.at = (uint32_t)i * stride;
+    t.d = i == G.n[a] - 1 ? 0u : stride;
+    return t;
+}
+ATAC_HD void trilinear64_nodes(const GridDev& G, const Axis64& X, const Axis64& Y, const Axis64& Z, float v[8]) {
+    const auto g = ATAC_GLOBAL(G.v);
+    const uint32_t o = X.at + Y.at + Z.at;
+    for (int q = 0; q < 8; ++q) v[q] = g[o + (q & 1 ? X.d : 0u) + (q & 2 ? Y.d : 0u) + (q & 4 ? Z.d : 0u)];
+}
+ATAC_HD double trilinear64_value(const Axis64& X, const Axis64& Y, const Axis64& Z, const float v[8]) {
+    double a = lerpd((double)v[0], (double)v[1], X.f);
+    double b = lerpd((double)v[2], (double)v[3], X.f);
+    double c = lerpd((double)v[4], (double)v[5], X.f);
+    double d = lerpd((double)v[6], (double)v[7], X.f);
+    return lerpd(lerpd(a, b, Y.f), lerpd(c, d, Y.f), Z.f);
+}
+ATAC_HD double trilinear64(const GridDev& G, const Axis64& X, const Axis64& Y, const Axis64& Z) {
+    float v[8];
+    trilinear64_nodes(G, X, Y, Z, v);
+    return trilinear64_value(X, Y, Z, v);
+}
 ATAC_HD double trilinear64_inside(const GridDev& G, double x0, double x1, double x2) {
-    double ci = (x0 - G.minb[0]) / G.d[0], cj = (x1 - G.minb[1]) / G.d[1], ck = (x2 - G.minb[2]) / G.d[2];
-    int i = (int)floor(ci), j = (int)floor(cj), k = (int)floor(ck);
-    ci = ci - i; cj = cj - j; ck = ck - k;
-    i = i < 0 ? 0 : (i > G.n[0] - 1 ? G.n[0] - 1 : i);
-    j = j < 0 ? 0 : (j > G.n[1] - 1 ? G.n[1] - 1 : j);
-    k = k < 0 ? 0 : (k > G.n[2] - 1 ? G.n[2] - 1 : k);
-    int ip = (i == G.n[0] - 1) ? i : i + 1;
-    int jp = (j == G.n[1] - 1) ? j : j + 1;
-    int kp = (k == G.n[2] - 1) ? k : k + 1;
-    const float* v = G.v;
-    double a = lerpd((double)v[grid_index(G, i, j, k)], (double)v[grid_index(G, ip, j, k)], ci);
-    double b = lerpd((double)v[grid_index(G, i, jp, k)], (double)v[grid_index(G, ip, jp, k)], ci);
-    double c = lerpd((double)v[grid_index(G, i, j, kp)], (double)v[grid_index(G, ip, j, kp)], ci);
-    double d = lerpd((double)v[grid_index(G, i, jp, kp)], (double)v[grid_index(G, ip, jp, kp)], ci);
-    return lerpd(lerpd(a, b, cj), lerpd(c, d, cj), ck);
+    return trilinear64(G, axis64(G, 0, x0), axis64(G, 1, x1), axis64(G, 2, x2));
 }
 
 // query_SDF(x, outside_accurate) in FP64 (BodySDFObj.cpp:123-174)
+ATAC_HD bool inside_box64(const GridDev& G, double x0, double x1, double x2) {
+    return x0 >= G.minb[0] && x0 <= G.maxb[0] && x1 >= G.minb[1] && x1 <= G.maxb[1] &&
+           x2 >= G.minb[2] && x2 <= G.maxb[2];
+}
 ATAC_HD double query_sdf64(const GridDev& G, double x0, double x1, double x2, bool outside_accurate) {
-    bool inside = x0 >= G.minb[0] && x0 <= G.maxb[0] && x1 >= G.minb[1] && x1 <= G.maxb[1] &&
-                  x2 >= G.minb[2] && x2 <= G.maxb[2];
-    if (inside) return trilinear64_inside(G, x0, x1, x2);
+    if (inside_box64(G, x0, x1, x2)) return trilinear64_inside(G, x0, x1, x2);
     if (!outside_accurate) return (double)FLT_MAX;
     double b0 = fmin(fmax(x0, G.minb[0]), G.maxb[0]);
     double b1 = fmin(fmax(x1, G.minb[1]), G.maxb[1]);
@@ -163,18 +185,13 @@ constexpr int kStencil = 20;
 
 ATAC_HD void stencil_point(const double x[3], int s, double p[3], bool& accurate) {
     const double h = kFdEps, hh = kFdEps / 2;
-    p[0] = x[0]; p[1] = x[1]; p[2] = x[2];
     accurate = s != 0;
-    if (s >= 2 && s < 8) {
-        const int ax = (s - 2) >> 1;
-        p[ax] = (s & 1) ? x[ax] - h : x[ax] + h;
-    } else if (s >= 8) {
-        const int pair = (s - 8) >> 2, k = (s - 8) & 3;   // pair 0 = xy, 1 = xz, 2 = yz
-        const int a0 = pair == 2 ? 1 : 0, a1 = pair == 0 ? 1 : 2;
-        const double s0 = (k == 0 || k == 2) ? hh : -hh, s1 = (k == 0 || k == 3) ? hh : -hh;
-        p[a0] = x[a0] + s0;
-        p[a1] = x[a1] + s1;
-    }
+    const bool one = s >= 2 && s < 8, two = s >= 8;
+    const int pair = (s - 8) >> 2, k = (s - 8) & 3;   // pair 0 = xy, 1 = xz, 2 = yz
+    const int a0 = one ? (s - 2) >> 1 : pair == 2 ? 1 : 0, a1 = pair == 0 ? 1 : 2;
+    const double s0 = one ? ((s & 1) ? -h : h) : (k == 0 || k == 2) ? hh : -hh, s1 = (k == 0 || k == 3) ? hh : -hh;
+    for (int a = 0; a < 3; ++a)   // selects: an index that is not a constant would put p in memory
+        p[a] = (one || two) && a == a0 ? x[a] + s0 : two && a == a1 ? x[a] + s1 : x[a];
 }
 
 // Value, gradient and Hessian from the 20 stencil values, in the reference's
@@ -206,6 +223,34 @@ ATAC_HD void sdf_stencil64(const GridDev& G, const double x[3], double& val, dou
         stencil_point(x, s, p, accurate);
         v[s] = query_sdf64(G, p[0], p[1], p[2], accurate);
     }
+    stencil_combine(v, val, g, H);
+}
+
+// The same for one lane per point: with the stencil inside the box its 20 places share
+// 15 positions along the axes (each with a division), formed once. The values are the
+// same bits: the same operations on the same numbers.
+ATAC_HD void sdf_stencil64_shared(const GridDev& G, const double x[3], double& val, double g[3], double H[6]) {
+    const double h = kFdEps, hh = kFdEps / 2;
+    if (!(inside_box64(G, x[0] - h, x[1] - h, x[2] - h) && inside_box64(G, x[0] + h, x[1] + h, x[2] + h)))
+        return sdf_stencil64(G, x, val, g, H);
+    double v[kStencil];
+    Axis64 c[3], p[3], m[3];
+    for (int a = 0; a < 3; ++a) { c[a] = axis64(G, a, x[a]); p[a] = axis64(G, a, x[a] + hh); m[a] = axis64(G, a, x[a] - hh); }
+    for (int pair = 0; pair < 3; ++pair)
+        for (int k = 0; k < 4; ++k) {
+            const int a0 = pair == 2 ? 1 : 0, a1 = pair == 0 ? 1 : 2;
+            const bool s0 = k == 0 || k == 2, s1 = k == 0 || k == 3;
+            Axis64 t[3] = {c[0], c[1], c[2]};
+            t[a0] = s0 ? p[a0] : m[a0];
+            t[a1] = s1 ? p[a1] : m[a1];
+            v[8 + 4 * pair + k] = trilinear64(G, t[0], t[1], t[2]);
+        }
+    v[0] = v[1] = trilinear64(G, c[0], c[1], c[2]);
+    for (int a = 0; a < 3; ++a)
+        for (int k = 0; k < 2; ++k) {
+            const Axis64 t = axis64(G, a, k ? x[a] - h : x[a] + h);
+            v[2 + 2 * a + k] = trilinear64(G, a == 0 ? t : c[0], a == 1 ? t : c[1], a == 2 ? t : c[2]);
+        }
     stencil_combine(v, val, g, H);
 }
 
@@ -1064,7 +1109,7 @@ template <typename Rec>
 ATAC_HD void record_slow(const GridDev& G, const InstDev& in, Rec& r, float* diag) {
     double x[3], val, g[3], H[6];
     body2_point(in, (double)r.a[0], (double)r.a[1], (double)r.a[2], x);
-    sdf_stencil64(G, x, val, g, H);
+    sdf_stencil64_shared(G, x, val, g, H);
     record_slow_fill(in, val, g, H, r, diag);
 }
 

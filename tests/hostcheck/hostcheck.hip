@@ -269,6 +269,19 @@ int hc_jacobian_blocks(const float* vals, const int32_t n[3], const double minb[
     return 0;
 }
 
+// The slow path's sample (value, gradient, Hessian: 10 values) of n points in the SDF
+// frame: place by place, and with the shared positions along the axes.
+int hc_stencils(const float* vals, const int32_t n[3], const double minb[3], const double maxb[3], const double d[3],
+                const double* x, int64_t npts, double* each, double* shared) {
+    HostGrid hg;
+    host_grid(vals, n, minb, maxb, d, hg);
+    for (int64_t i = 0; i < npts; ++i) {
+        sdf_stencil64(hg.G, x + 3 * i, each[10 * i], each + 10 * i + 1, each + 10 * i + 4);
+        sdf_stencil64_shared(hg.G, x + 3 * i, shared[10 * i], shared + 10 * i + 1, shared + 10 * i + 4);
+    }
+    return 0;
+}
+
 // Closest triangles of n points: mesh_closest's traversal (the 8 lanes of a group in
 // turn, their votes taken as the kernel takes them) and, next to it, every triangle
 // tested. Returns 0, or 1 when the mesh is refused.

@@ -167,3 +167,12 @@ def mesh_closest(V, F, x):
                               _vp(f), _vp(bd2), _vp(bf), C.byref(deepest))
     assert r == 0, "mesh refused"
     return d2, f, bd2, bf, deepest.value
+
+
+def stencils(grid, x):
+    """The slow path's samples (n, 10) at SDF-frame points, formed place by place and with shared positions."""
+    vals, n, mn, mx, d = _grid_args(grid)
+    x = np.ascontiguousarray(x, dtype=np.float64).reshape(-1, 3)
+    a, b = np.empty((len(x), 10)), np.empty((len(x), 10))
+    lib().hc_stencils(_vp(vals), _vp(n), _vp(mn), _vp(mx), _vp(d), _vp(x), C.c_int64(len(x)), _vp(a), _vp(b))
+    return a, b

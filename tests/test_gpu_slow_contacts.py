@@ -56,3 +56,23 @@ def test_more_than_the_slow_list_holds(gpu, precise):
     torch.cuda.synchronize()
     assert (out["n_active"] == 2000).all() and not b.workspace()["overflowed"]
     assert all(torch.isfinite(v).all() for v in out.values())
+
+
+@pytest.mark.parametrize("precise", [False, True], ids=["fp32", "precise"])
+@pytest.mark.parametrize("n", [1, 3, 127, 128, 129, 511, 512, 513, 640, 641, 2048, 3072])
+def test_one_workgroup_equals_the_pipeline(gpu, n, precise):
+    """Instances of slow contacts alone, around the numbers that one workgroup takes together: the samples have
+    the pipeline's bits, the sums its order (terms of a few ulp: FP32 2^-24, FP64 2^-53, cancelling by up to 1e3)."""
+    tol = 1e-12 if precise else 1e-4
+    g = torch.tensor(np.random.default_rng(n).normal(size=(2, 12)), device="cuda")
+    for kw in ({}, {"p6": True}, {"deriv": True}):
+        res = []
+        for tuning in (None, {"max_active": -1}):
+            b = _batch([n, min(n, 1000)], tuning=tuning)
+            out = b.eval(precise=precise, **kw)
+            res.append({**out, **b.vjp(g)})
+        torch.cuda.synchronize()
+        assert res[0]["n_active"].tolist() == [n, min(n, 1000)]
+        for k in res[0]:
+            p, q = res[0][k].double(), res[1][k].double()
+            assert torch.isfinite(p).all() and (p - q).abs().max() <= tol * q.abs().max(), k

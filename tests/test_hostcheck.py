@@ -352,3 +352,22 @@ def test_group_culling_box_inside_and_beyond_grid():
         for gs in (1, 16, 256):
             live, needed = _cull_checks(g, pts, ins, gs)
             assert needed.any()
+
+
+def test_shared_stencil_is_the_stencil():
+    """The FD stencil with its positions along the axes formed once: the same bits, on cell planes, at the
+    box's faces (the stencil partly outside) and at points that are not finite."""
+    w = W.peg_in_hole(n_points=10, n_poses=1)
+    g = w.grids[0]
+    rng = np.random.default_rng(13)
+    lo, hi, d = np.asarray(g.min_box), np.asarray(g.max_box), np.asarray(g.dxyz)
+    x = rng.uniform(lo, hi, (6000, 3))
+    k = rng.integers(0, 3, 6000)
+    r = np.arange(6000)
+    x[r[:3000], k[:3000]] = (lo + d * rng.integers(0, 40, (6000, 3)))[r[:3000], k[:3000]] + rng.choice([0.0, 4e-6, -8e-6], 3000)
+    x[r[3000:4500], k[3000:4500]] = lo[k[3000:4500]] + rng.uniform(-2e-5, 2e-5, 1500)
+    x[r[4500:], k[4500:]] = hi[k[4500:]] + rng.uniform(-2e-5, 2e-5, 1500)
+    x[-3:] = [[np.nan, 0.0, 0.0], [np.inf, 0.0, 0.0], [0.0, -np.inf, 1e300]]
+    a, b = H.stencils(g, x)
+    assert np.array_equal(a, b, equal_nan=True)
+    assert np.isfinite(a[:3000]).all()
