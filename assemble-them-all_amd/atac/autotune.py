@@ -17,7 +17,8 @@ import time
 import numpy as np
 import torch
 
-DEFAULT_CANDIDATES = [
+# the default plan first: small batches have a path of their own there
+DEFAULT_CANDIDATES = [{}] + [
     {"tile_points": tp, "detect_block": blk, "points_per_lane": ppl, "order": order}
     for order in (1, 4)
     for tp in (1024, 2048, 4096, 8192)

@@ -556,13 +556,6 @@ static int wave_span_of(int tile_points, int block) {
     return (ng + nw - 1) / nw * kGroup;
 }
 
-static bool default_tuning(const atac_tuning& t) {
-    const atac_tuning zero{};
-    return t.tile_points == zero.tile_points && t.detect_block == zero.detect_block && t.blocks_per_cu == zero.blocks_per_cu &&
-           t.order == zero.order && t.points_per_lane == zero.points_per_lane && t.max_active == zero.max_active &&
-           t.group_cull == zero.group_cull;
-}
-
 static int plan(atac_batch b, const atac_tuning* t) {
     ++b->buf_gen;   // the tile plan and its buffers are rebuilt: cached graphs are stale
     atac_tuning tu = t ? *t : atac_tuning{};
@@ -577,11 +570,10 @@ static int plan(atac_batch b, const atac_tuning* t) {
     // use. 256, 512 and 1024 threads: 250 tiles (96 FP64 instances) 65.0, 59.7, 57.8 us
     // an evaluation and its adjoint, 512 tiles (Km/Dm of 256) 61.9, 60.5, 65.5, 1,500
     // tiles 75.7, 73.8, 90.6, 7,200 tiles 175.8 and 185.4
-    if (tu.detect_block <= 0) {
-        int64_t n_tiles = 0;
-        for (const InstDev& d : b->inst_dev) n_tiles += (d.pt_count + tu.tile_points - 1) / tu.tile_points;
-        tu.detect_block = n_tiles <= b->n_cu ? 1024 : n_tiles <= 8 * (int64_t)b->n_cu ? 512 : 256;
-    }
+    int64_t n_tiles = 0;
+    for (const InstDev& d : b->inst_dev) n_tiles += (d.pt_count + tu.tile_points - 1) / tu.tile_points;
+    const int by_tiles = n_tiles <= b->n_cu ? 1024 : n_tiles <= 8 * (int64_t)b->n_cu ? 512 : 256;
+    if (tu.detect_block <= 0) tu.detect_block = by_tiles;
     if (tu.detect_block != 64 && tu.detect_block != 128 && tu.detect_block != 256 && tu.detect_block != 512 &&
         tu.detect_block != 1024)
         return fail(ATAC_ERR_INVALID, "detect_block must be 64, 128, 256, 512 or 1024");
@@ -637,13 +629,16 @@ static int plan(atac_batch b, const atac_tuning* t) {
     b->chunk_cap = std::min<int64_t>(chunks, b->rec_cap / kChunk + b->tiles.size());
     b->n_tiles = (int32_t)b->tiles.size();
     b->chunk_total = (int32_t)std::min<int64_t>(chunks, INT32_MAX);
-    // one workgroup per instance (instance_kernel): default plans of small instances, as
-    // many as the GPU holds at once (two per CU); with 1,024 instances of 500 points the
-    // pipeline's finer pieces fill it better (37 us against 42; 512: 34 against 25)
+    // one workgroup per instance (instance_kernel): default plans (left out or with the
+    // default values written out) of small instances, as many as the GPU holds at once (two
+    // per CU); with 1,024 instances of 500 points the pipeline's finer pieces fill it better
+    // (37 us against 42; 512: 34 against 25)
     static_assert(kGroup % kChunk == 0, "an instance's items are as many over its tiles as over its points");
     b->most_points = 0;
     for (const InstDev& d : b->inst_dev) b->most_points = std::max(b->most_points, (int64_t)d.pt_count);
-    b->one_per_instance = (!t || default_tuning(*t)) && b->rec_cap == slot &&
+    const bool default_plan = tu.tile_points == 4096 && tu.detect_block == by_tiles && tu.blocks_per_cu == 0 && tu.order == 1 &&
+                              tu.points_per_lane == 4 && tu.max_active == 0 && tu.group_cull == 1;
+    b->one_per_instance = default_plan && b->rec_cap == slot &&
                           b->inst_dev.size() <= (size_t)(2 * b->n_cu) && b->most_points <= inst_points(0);
     // tile queues: 1 = one queue in instance order; 2 = one queue grouped by grid;
     // 3 = grouped by grid and cut into one queue per XCD with balanced point counts;

@@ -76,3 +76,24 @@ def test_one_workgroup_equals_the_pipeline(gpu, n, precise):
         for k in res[0]:
             p, q = res[0][k].double(), res[1][k].double()
             assert torch.isfinite(p).all() and (p - q).abs().max() <= tol * q.abs().max(), k
+
+
+def test_default_values_written_out(gpu):
+    """A plan with the default values written out, or a plan's own values given back, is the default plan: small
+    instances run in one workgroup, which holds 6,000 slow contacts where the pipeline's list overflows."""
+    b = _batch([2000, 2000, 2000])
+    info = b.info()
+    own = {k: info[k] for k in ("tile_points", "detect_block", "blocks_per_cu", "order", "points_per_lane", "max_active", "group_cull")}
+    for tuning in (None, {}, {"tile_points": 4096, "order": 1, "points_per_lane": 4}, {"group_cull": 1}, own):
+        assert _batch([2000, 2000, 2000], tuning=tuning).eval()["n_active"].tolist() == [2000, 2000, 2000], tuning
+        b.retune(tuning or {})
+        assert b.eval()["n_active"].tolist() == [2000, 2000, 2000], tuning
+    for tuning in ({"order": 4}, {"points_per_lane": 2}, {"detect_block": 64}, {"blocks_per_cu": 1}, {"max_active": 6000},
+                   {"group_cull": -1}, {"tile_points": 2048}, {"tile_points": 8192}):
+        b.retune(tuning)
+        assert b.eval()["n_active"].tolist() == [-1, -1, -1], tuning
+
+
+def test_autotune_times_the_default_plan():
+    from atac.autotune import DEFAULT_CANDIDATES
+    assert DEFAULT_CANDIDATES[0] == {}
