@@ -688,7 +688,9 @@ static int plan(atac_batch b, const atac_tuning* t) {
     if (!rc) rc = dalloc(&b->d_tile_chunk0, b->n_tiles);
     if (!rc) rc = dalloc(&b->d_chunks, (size_t)b->chunk_cap);
     if (rc) return rc;
-    ATAC_HIP(hipMemset(b->d_counters, 0, sizeof(int32_t) * CNT_ALL));   // no stale work-item count before the first evaluation
+    // no stale counts before the first evaluation
+    ATAC_HIP(hipMemset(b->d_counters, 0, sizeof(int32_t) * CNT_ALL));
+    if (b->n_tiles > 0) ATAC_HIP(hipMemset(b->d_tile_active, 0, sizeof(int32_t) * b->n_tiles));
     ATAC_HIP(hipMemcpy(b->d_tq_begin, tq.data(), sizeof(int32_t) * tq.size(), hipMemcpyHostToDevice));
     if (b->n_tiles > 0) {
         ATAC_HIP(hipMemcpy(b->d_tiles, b->tiles.data(), sizeof(TileDev) * b->n_tiles, hipMemcpyHostToDevice));

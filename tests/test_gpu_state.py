@@ -137,3 +137,19 @@ def test_record_pool_bound_and_overflow(gpu):
     assert torch.isnan(g["g_q1"]).all()
     with pytest.raises(L.AtacError, match="record pool"):
         small.active_ids(0)
+
+
+def test_workspace_before_an_evaluation(gpu):
+    """No evaluation, no contacts in use: on a new batch, where its memory was another's before, and after a re-plan."""
+    w = W.peg_in_hole(n_points=2000, n_poses=64)
+    for tuning in (None, {"max_active": -1}):
+        b = batch_from_workload(w, tuning=tuning)
+        for plan in (tuning, {"tile_points": 1024}, {"tile_points": 256}):
+            b.retune(plan or {})
+            assert b.workspace()["used"] == 0 and not b.workspace()["overflowed"]
+            b.eval()
+            torch.cuda.synchronize()
+            assert b.workspace()["used"] > 0
+        # the memory of this plan's counts, filled, goes to the next batch
+        junk = [torch.full((k,), 77, dtype=torch.int32, device="cuda") for k in (64, 128, 512, 1024)]
+        del b, junk
