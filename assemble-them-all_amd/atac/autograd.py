@@ -115,7 +115,7 @@ class ContactWrench(torch.autograd.Function):
         if not torch.is_grad_enabled() and all(E is None or _on_device(E, (batch.n, 4, 4)) for E in (E1, E2)):
             if E1 is not None or E2 is not None:
                 gE1, gE2, singular = batch.pose_gradients(E1, g["g_q1"], E2, g["g_q2"])
-                if singular:   # torch's error
+                if singular:   # torch's error, or its values
                     gE1, gE2 = (None if E is None else tangent_pairing_matrix(E, g[k]) for E, k in ((E1, "g_q1"), (E2, "g_q2")))
         else:
             gE1 = None if E1 is None else tangent_pairing_matrix(E1, g["g_q1"])

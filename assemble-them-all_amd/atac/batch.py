@@ -300,7 +300,7 @@ class ContactBatch:
 
     def pose_gradients(self, E1, g_q1, E2, g_q2):
         """The matrix gradients of atac.autograd for contiguous FP64 poses on the device (None: left out),
-        and the number of poses that have no inverse."""
+        and the number of poses that have no inverse or next to none."""
         gE1, gE2 = (None if E is None else torch.empty_like(E) for E in (E1, E2))
         bad = C.c_int32()
         p = [None if t is None else t.data_ptr() for t in (E1, g_q1, gE1, E2, g_q2, gE2)]

@@ -200,7 +200,7 @@ constexpr int kPoseRow = 46;
 hipError_t launch_pose_rows(const double* E1, const double* E2, const double* phi1, const double* phi2, const double* kn,
                             const double* kt, double* rows, int32_t* done, int32_t call, int n, hipStream_t st);
 // gE = E^-T M(g) of two lists of n poses (either may be null); done[2 i + body] = call
-// (-call: E is singular)
+// (-call: E has no inverse, or none to about 2^-40)
 hipError_t launch_pose_gradients(const double* E1, const double* g1, double* gE1, const double* E2, const double* g2,
                                  double* gE2, int32_t* done, int32_t call, int n, hipStream_t st);
 hipError_t launch_grid_setup(const GridDev& G, float4* cells, hipStream_t st);

@@ -1193,7 +1193,9 @@ __global__ __launch_bounds__(64) void pose_rows_kernel(const double* E1, const d
     if (k == 0) __hip_atomic_store(done + i, call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// A lane per pose: E^T X = M by elimination with row exchanges, in registers.
+// A lane per pose: E^T X = M by elimination with row exchanges, in registers. A pose
+// with a pivot within 2^-40 of its largest entry (or no number) is reported: a matrix
+// without an inverse leaves a rounding (2^-52 of that entry) there as often as a zero.
 __global__ __launch_bounds__(64) void pose_gradients_kernel(const double* E1, const double* g1, double* gE1,
                                                             const double* E2, const double* g2, double* gE2,
                                                             int32_t* done, int32_t call, int n) {
@@ -1217,6 +1219,12 @@ __global__ __launch_bounds__(64) void pose_gradients_kernel(const double* E1, co
         m[1][4] = w2;  m[1][6] = -w0;
         m[2][4] = -w1; m[2][5] = w0;
         m[0][7] = g[6 * i + 3]; m[1][7] = g[6 * i + 4]; m[2][7] = g[6 * i + 5];
+        double least = 0.0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) least = fmax(least, fabs(m[r][c]));
+        least *= 0x1p-40;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
 #pragma unroll
@@ -1229,7 +1237,7 @@ __global__ __launch_bounds__(64) void pose_gradients_kernel(const double* E1, co
                     m[r][c] = swap ? a : b;
                 }
             }
-            singular = singular || m[k][k] == 0.0;
+            singular = singular || !(fabs(m[k][k]) > least);
 #pragma unroll
             for (int r = k + 1; r < 4; ++r) {
                 const double f = m[r][k] / m[k][k];

@@ -147,8 +147,10 @@ int atac_batch_set_instances(atac_batch b, const atac_instance* inst, int32_t n_
 int atac_batch_set_poses(atac_batch b, const double* E1, const double* E2, const double* phi1, const double* phi2,
                          const double* kn, const double* kt, atac_instance* inst, int32_t n_inst, void* stream);
 /* Matrix gradients of poses from twist gradients g = (g_w, g_v): g_E = E^-T M(g),
- * M(g) = [[skew(g_w) / 2, g_v], [0, 0]] (n x 16; a null g_E is left out). singular:
- * the number of poses without an inverse. Device pointers; waits for the result. */
+ * M(g) = [[skew(g_w) / 2, g_v], [0, 0]] (n x 16; a null g_E is left out). Device
+ * pointers; g_E is ready in the stream's order. singular: the number of poses that have
+ * no inverse or a pivot within 2^-40 of their largest entry, whose g_E may be of no use;
+ * this number (alone) is waited for. */
 int atac_batch_pose_gradients(atac_batch b, const double* E1, const double* g_q1, double* g_E1, const double* E2,
                               const double* g_q2, double* g_E2, int32_t* singular, void* stream);
 /* Re-plans tiles and launch shape (used by the autotuner). */

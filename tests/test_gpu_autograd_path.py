@@ -90,3 +90,45 @@ def test_second_derivative_keeps_its_graph(gpu):
     x = [t.requires_grad_() for t in _inputs(w)]
     gE, = torch.autograd.grad(contact_wrench(b, *x).sum(), x[:1], create_graph=True)
     assert gE.requires_grad and torch.isfinite(torch.autograd.grad(gE.sum(), x[0])[0]).all()
+
+
+def _same_rows(E): E[2] = E[0]
+def _same_columns(E): E[:, 2] = E[:, 0]
+def _sum_of_rows(E): E[2] = E[0] + E[1]
+def _ones(E): E[:] = 1.0
+def _flat(E): E[:3, :3] = np.outer(E[:3, 0], E[0, :3])
+def _near(E): E[2] = E[0] * (1 + 1e-15)
+def _nan(E): E[3, 3] = np.nan
+def _tall(E): E[:3, 3] = [1e9, -2e9, 3e8]
+
+
+@pytest.mark.parametrize("change", [_same_rows, _same_columns, _sum_of_rows, _ones, _flat, _near, _nan, _tall])
+def test_poses_without_an_inverse(gpu, change):
+    """What torch refuses to invert is refused, also where the elimination leaves a rounding in place of a zero;
+    what torch inverts gives torch's gradient."""
+    w = W.peg_in_hole(n_points=100, n_poses=6)
+    b = batch_from_workload(w)
+    rng = np.random.default_rng(9)
+    for k in range(6):
+        x = _inputs(w)
+        E = np.eye(4)
+        E[:3, :3], E[:3, 3] = W.random_rotation(rng), rng.uniform(-2, 2, 3)
+        change(E)
+        x[1][k] = torch.tensor(E, device="cuda")
+        x = [t.requires_grad_() for t in x]
+        g = torch.tensor(rng.normal(size=(6, 12)), device="cuda")
+        fm = contact_wrench(b, *x)
+        try:
+            torch.linalg.inv(x[1].detach())
+        except torch.linalg.LinAlgError:
+            with pytest.raises(torch.linalg.LinAlgError):
+                torch.autograd.grad(fm, x, g)
+            continue
+        got = torch.autograd.grad(fm, x, g)[1]
+        want = tangent_pairing_matrix(x[1].detach(), b.vjp(g)["g_q2"])
+        ok = torch.isfinite(want)
+        assert torch.equal(ok, torch.isfinite(got))
+        # FP64, a condition of up to 1e19 (tall): of each pose's largest entry
+        scale = torch.where(ok, want, 0).abs().amax((1, 2), keepdim=True).clamp(min=1e-300)
+        tol = 1e-12 if change is not _tall else 1e-6
+        assert (torch.where(ok, got - want, 0).abs() <= tol * scale).all(), (k, change.__name__)
