@@ -453,10 +453,20 @@ __global__ __launch_bounds__(1024) void bvh_reduce_kernel(BvhForceArgs a, int nb
     }
 }
 
-hipError_t launch_mesh_distance(const MeshQueryArgs& a, hipStream_t st) {
-    if (a.n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(mesh_distance_kernel, dim3((unsigned)((a.n + 31) / 32)), dim3(256), 0, st, a);
-    return hipGetLastError();
+hipError_t launch_mesh_distance(MeshQueryArgs a, hipStream_t st) {
+    // a launch holds fewer than 2^32 threads, eight per point
+    constexpr int64_t kMost = (int64_t)1 << 28;
+    for (int64_t left = a.n; left > 0; left -= kMost) {
+        a.n = left < kMost ? left : kMost;
+        hipLaunchKernelGGL(mesh_distance_kernel, dim3((unsigned)((a.n + 31) / 32)), dim3(256), 0, st, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        a.xw += 3 * a.n;
+        a.d += a.n;
+        if (a.normal) a.normal += 3 * a.n;
+        if (a.face) a.face += a.n;
+    }
+    return hipSuccess;
 }
 
 // ------------------------------------------------------------------ fixed scratch

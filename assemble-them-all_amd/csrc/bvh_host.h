@@ -58,7 +58,7 @@ inline int64_t bvh_block_points(int64_t n) {
 }
 inline int64_t bvh_force_blocks(int64_t n) { return n > 0 ? (n + bvh_block_points(n) - 1) / bvh_block_points(n) : 1; }
 
-hipError_t launch_mesh_distance(const MeshQueryArgs& a, hipStream_t st);
+hipError_t launch_mesh_distance(MeshQueryArgs a, hipStream_t st);
 hipError_t launch_bvh_force(BvhForceArgs a, hipStream_t st);
 
 // Fixed scratch of atac_bvh_force_noalloc: the partial rows and counts of the at

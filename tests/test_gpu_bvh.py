@@ -71,6 +71,32 @@ def test_equally_near_triangles(points):
         np.testing.assert_allclose(n, on, rtol=0, atol=1e-15)
 
 
+def test_more_points_than_one_launch_holds(gpu):
+    """Eight lanes a point: 2^29 points and more are several launches. All but the last few lie outside."""
+    import ctypes as C
+    import torch
+    V, F = MESHES["cube"]()
+    m = BVHMesh(V, F)
+    x = np.random.default_rng(4).uniform(V.min(0), V.max(0), (100, 3))
+    E = np.eye(4)
+    want = m.distance_normal(x, E, 0.01)
+    n = (1 << 29) + 57
+    xw = torch.full((n, 3), 10.0, dtype=torch.float64, device="cuda")
+    d = torch.zeros(n, dtype=torch.float64, device="cuda")
+    face = torch.zeros(n, dtype=torch.int32, device="cuda")
+    at = [(1 << 28) - 50, (1 << 29) - 43]     # across the ends of the launches
+    for a in at:
+        xw[a:a + 100] = torch.tensor(x, device="cuda")
+    p = lambda t: C.c_void_p(t.data_ptr())
+    L.check(L.lib().atac_mesh_distance_normal(m.handle, L.dptr(E), 0.01, p(xw), n, p(d), None, p(face), None))
+    torch.cuda.synchronize()
+    for a in at:
+        assert np.array_equal(d[a:a + 100].cpu().numpy(), want[0]) and np.array_equal(face[a:a + 100].cpu().numpy(), want[2])
+        d[a:a + 100] = 10.0
+        face[a:a + 100] = -1
+    assert bool((d == 10.0).all()) and bool((face == -1).all())
+
+
 def test_bad_meshes():
     V, F = box_mesh(1.0)
     with pytest.raises(L.AtacError):
