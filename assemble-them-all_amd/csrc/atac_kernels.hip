@@ -789,12 +789,12 @@ __global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
 // threads form the 288 entries of Km and Dm from the block sums (jac_entry). Rows
 // of tangent columns (InstDev::rigid 0) have two components a thread.
 template <bool RIGID>
-__global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a) {
+__global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a, int first) {
     constexpr int kRows = 64 * 32;   // a tile holds at most 8192 / kChunk items
     __shared__ int s_rows[kRows];
     __shared__ int s_nrows, s_nact;
     __shared__ double s_sum[RIGID ? kJacRow : kJvpRow], s_m[288], s_R[9], s_t[3];
-    const int k = (int)threadIdx.x, i = (int)blockIdx.x;
+    const int k = (int)threadIdx.x, i = first + (int)blockIdx.x;
     const bool ovf = a.counters[CNT_OVERFLOW] != 0;
     if (a.overflow_out && i == 0 && k == 0) *a.overflow_out = ovf ? 1 : 0;
     const InstDev in = as_const(a.inst)[i];
@@ -1615,10 +1615,15 @@ hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st) {
 }
 
 hipError_t launch_reduce_jacobian(const ReduceArgs& a, bool rigid, hipStream_t st) {
-    if (a.n_inst <= 0) return hipSuccess;
-    if (rigid) hipLaunchKernelGGL(reduce_jacobian_kernel<true>, dim3(a.n_inst), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(reduce_jacobian_kernel<false>, dim3(a.n_inst), dim3(256), 0, st, a);
-    return hipGetLastError();
+    constexpr int64_t kMost = 1 << 23;   // a launch holds fewer than 2^32 threads
+    for (int64_t first = 0; first < a.n_inst; first += kMost) {
+        const dim3 grid((unsigned)(a.n_inst - first < kMost ? a.n_inst - first : kMost));
+        if (rigid) hipLaunchKernelGGL(reduce_jacobian_kernel<true>, grid, dim3(256), 0, st, a, (int)first);
+        else hipLaunchKernelGGL(reduce_jacobian_kernel<false>, grid, dim3(256), 0, st, a, (int)first);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <int MODE, bool RIGID>
