@@ -1803,8 +1803,6 @@ int atac_mesh_create(const double* V, int64_t nv, const int64_t* F, int64_t nf, 
     D.nodes = m->d_nodes; D.tri = m->d_tri; D.tv = m->d_tv; D.F = m->d_F;
     D.FN = m->d_FN; D.FE = m->d_FE; D.EN = m->d_EN; D.VN = m->d_VN;
     for (int a = 0; a < 3; ++a) { D.bmin[a] = h.bmin[a]; D.bmax[a] = h.bmax[a]; }
-    D.n_leaves = (int32_t)(h.tri.size() / kBvhWidth);
-    D.nf = (int32_t)nf;
     *out = m;
     return ATAC_OK;
 }

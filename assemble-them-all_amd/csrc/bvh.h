@@ -40,7 +40,6 @@ struct MeshDev {
     const double* EN;       // ne x 3 edge normals
     const double* VN;       // nv x 3 vertex normals
     double bmin[3], bmax[3];  // the vertices' bounding box (BodyMeshObj.cpp:179-182)
-    int32_t n_leaves, nf;
 };
 
 // Entries waiting during a traversal: each visited node leaves at most 7 of its 8,
