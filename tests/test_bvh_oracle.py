@@ -135,7 +135,12 @@ def test_pose_and_col_th():
     d_w, n_w, f_w = O.mesh_distance_normal(V, F, xw, E2=E2, col_th=0.02)
     ins = d_body != 10.0
     np.testing.assert_allclose(d_w[ins], d_body[ins] + 0.02, atol=1e-13)
-    np.testing.assert_array_equal(f_w, f_body)
+    # where two faces are equally near (the closest point on their edge), the rounding of the
+    # posed points decides between them: then both hold the closest point
+    for i in np.flatnonzero(f_w != f_body):
+        near = [tri_dist(V, F[f][None], x_body[i][None])[0] for f in (f_w[i], f_body[i])]
+        np.testing.assert_allclose(near, abs(d_body[i]), rtol=0, atol=1e-13)
+    assert (f_w != f_body).mean() < 0.05
 
 
 def test_degenerate_triangle_is_its_edges():

@@ -26,7 +26,8 @@ FORMS = {"strided": lambda t: torch.stack([t, t], -1)[..., 0], "cpu": lambda t: 
 def test_routes_agree(gpu, form, n):
     """Forward, instances kept and gradients: the same values reach the same kernels, so equal
     bits; the pose gradients are solved in another order (FP64, condition of a pose: below 1e2)."""
-    w = W.peg_in_hole(n_points=700, n_poses=n)
+    w = W.peg_in_hole(n_points=700, n_poses=33)
+    w.instances = w.instances[1:1 + n] if n < 33 else w.instances   # (pose 0 touches nothing)
     g = torch.tensor(np.random.default_rng(n).normal(size=(n, 12)), device="cuda")
     res = []
     for change in (lambda t: t, FORMS[form]):
@@ -43,7 +44,7 @@ def test_routes_agree(gpu, form, n):
             grads = list(torch.autograd.grad(fm, x, g))
         res.append((fm.detach(), grads, bytes(b.instances)))
     assert torch.equal(res[0][0], res[1][0]) and res[0][2] == res[1][2]
-    assert res[0][0].abs().max() > 0 or n < 33   # (the first poses touch nothing)
+    assert res[0][0].abs().max() > 0
     for k, (p, q) in enumerate(zip(res[0][1], res[1][1])):
         if q is None:
             continue

@@ -223,12 +223,12 @@ def test_degenerate_triangles():
 
 
 def test_force_many_workgroups():
-    """A force evaluation over several 2,048-point workgroups (their partial rows
-    added in workgroup order) equals the oracle."""
+    """A force evaluation over many 64-point workgroups (their partial rows added in
+    a fixed order) equals the oracle."""
     V, F = MESHES["torus"]()
     rng = np.random.default_rng(8)
     P, _ = icosphere(0.35, levels=4)
-    xi = np.concatenate([P, P * 0.95, P * 0.9])           # 7,686 points: 4 workgroups
+    xi = np.concatenate([P, P * 0.95, P * 0.9])           # 7,686 points: 121 workgroups
     E1 = O.se3_exp(np.concatenate([rng.normal(size=3) * 0.3, np.zeros(3)]))
     E1[:3, 3] = V[rng.integers(len(V))] * 1.02
     E2 = np.eye(4)
@@ -243,3 +243,27 @@ def test_force_many_workgroups():
     for key in ("fm", "dfm_dp6", "Km", "Dm"):
         a, b = np.asarray(got[key]), np.asarray(ref[key])
         assert np.abs(a - b).max() <= 1e-9 * max(np.abs(b).max(), 1e-12), key
+
+
+@pytest.mark.parametrize("n", [32768, 32769, 65600, 100003])
+def test_force_several_steps_per_workgroup(n):
+    """Past 512 workgroups of 64 points each one takes several steps: the result equals the sum of calls over
+    parts that take one step each (FP64 sums in another order: some 1e4 contacts, 2^-53 each)."""
+    V, F = MESHES["torus"]()
+    rng = np.random.default_rng(n)
+    u = rng.normal(size=(n, 3))
+    xi = 0.35 * u / np.linalg.norm(u, axis=1, keepdims=True) * rng.uniform(0.9, 1.0, (n, 1))
+    E1 = O.se3_exp(np.concatenate([rng.normal(size=3) * 0.3, np.zeros(3)]))
+    E1[:3, 3] = V[5] * 1.02
+    phi1, phi2 = rng.normal(size=6) * 0.2, rng.normal(size=6) * 0.1
+    args = (0.005, 3e4, 1e3, 0.6, 5.0, 1.1, 0.9)
+    m = BVHMesh(V, F)
+    cuts = np.linspace(0, n, 6).astype(int)
+    for kw in (dict(deriv=True, p6=True), dict(p6=True), {}):
+        f = lambda p: m.force(p, E1, phi1, np.eye(4), phi2, *args, **kw)
+        got, parts = f(xi), [f(xi[a:b]) for a, b in zip(cuts[:-1], cuts[1:])]
+        assert got["n_active"] == sum(p["n_active"] for p in parts) > 1000
+        for key in got:
+            if key != "n_active":
+                want = sum(p[key] for p in parts)
+                assert np.abs(got[key] - want).max() <= 1e-11 * max(np.abs(p[key]).max() for p in parts), key

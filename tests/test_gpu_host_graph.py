@@ -1,7 +1,7 @@
-"""atac_batch_eval_instances_host: set_instances + eval_host replayed as one captured
-graph. The same bits as the two eager calls, at changing poses, for each flag
-combination, after the batch's buffers change (re-capture), and with the adjoint
-records left for atac_batch_vjp_host."""
+"""atac_batch_eval_instances_host: set_instances + eval_host in one call, for small
+instances one launch, else replayed as one captured graph. The same bits as the two
+eager calls, at changing poses, for each flag combination, after the batch's buffers
+change (re-capture), and with the adjoint records left for atac_batch_vjp_host."""
 import ctypes as C
 
 import numpy as np
@@ -47,9 +47,12 @@ def _run(b, inst, flags, graph):
     return {"fm": fm, "Km": Km, "Dm": Dm, "p6": p6, "na": na}
 
 
-def test_graph_replay_matches_eager_calls(gpu):
-    w = W.peg_in_hole(n_poses=10)
-    b = batch_from_workload(w)
+@pytest.mark.parametrize("n_points,tuning", [(5000, None), (1500, None), (1500, {"max_active": -1})],
+                         ids=["graphs", "launches", "graphs_small"])
+def test_graph_replay_matches_eager_calls(gpu, n_points, tuning):
+    """Small instances of the default plan take one launch; larger ones and other plans replay graphs."""
+    w = W.peg_in_hole(n_points=n_points, n_poses=10)
+    b = batch_from_workload(w, tuning=tuning)
     L = lib()
     for flags in (0, 1 | 2, 8, 1 | 8):     # force; Km/Dm + p6; precise force (new buffers); precise Km/Dm
         for shift in (0.0, 0.004, -0.003):

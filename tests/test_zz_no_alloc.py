@@ -52,7 +52,8 @@ def _host(m, inst, xi, flags):
 
 def test_noalloc_matches_host_variant(gpu):
     flags = L.EVAL_DERIV | L.EVAL_P6
-    for seed, shells in ((3, 4), (4, 1)):   # 10,248 then 2,562 points: 6 then 2 workgroups
+    # 10,248 then 2,562 points: 161 then 41 workgroups of a step each; 35,868: 281 of two steps
+    for seed, shells in ((3, 4), (4, 1), (3, 14)):
         V, F, xi, inst = _case(seed, shells)
         m = BVHMesh(V, F)
         print("no-alloc BVH force:", len(xi), "points, seed", seed, flush=True)
