@@ -112,6 +112,10 @@ struct atac_batch_s {
     InstDev* pin_pose = nullptr;      // pinned: the records atac_batch_set_poses uploads
     hipEvent_t pose_read = nullptr;   // ... read
     int32_t chunk_total = 0;          // work items if every point were a contact
+    int32_t n_more = 0;               // instance_kernel: tiles that are not their instance's first, ...
+    int32_t* d_more = nullptr;        // ... which,
+    double* d_tile_sum = nullptr;     // the tiles' sums
+    int32_t* d_tiles_done = nullptr;  // and per instance the tiles finished (InstanceArgs)
     int32_t* d_tile_chunk0 = nullptr;
     ChunkDev* d_chunks = nullptr;
     int32_t* d_counters = nullptr;    // CNT_ALL
@@ -504,7 +508,7 @@ static void release_plan(atac_batch b) {
     dfree(b->d_tiles); dfree(b->d_order); dfree(b->d_tq_begin); dfree(b->d_counters);
     dfree(b->d_tile_active); dfree(b->d_tile_chunk0); dfree(b->d_chunks); dfree(b->d_tile_live);
     dfree(b->d_act); dfree(b->d_rec32); dfree(b->d_rec64); dfree(b->d_slow); dfree(b->d_slow_diag);
-    dfree(b->d_part);
+    dfree(b->d_part); dfree(b->d_more); dfree(b->d_tile_sum); dfree(b->d_tiles_done);
     b->part_width = 0;
     b->rec_valid = false;
     b->rec_captured = false;
@@ -640,6 +644,16 @@ static int plan(atac_batch b, const atac_tuning* t) {
                               tu.points_per_lane == 4 && tu.max_active == 0 && tu.group_cull == 1;
     b->one_per_instance = default_plan && b->rec_cap == slot &&
                           b->inst_dev.size() <= (size_t)(2 * b->n_cu) && b->most_points <= inst_points(0);
+    // of instances with several tiles a workgroup per tile, up to three for two CUs: a
+    // wrench of 8 x 8,000 points takes 25 us against 38 with one per instance, of 100 29 and
+    // 39, of 200 (400 tiles) 40.4 and 43.0 (FP64 50.1 and 50.2), of 256 44.3 and 43.5, of
+    // 400 x 6,000 56 and 43.5; and where the second tile is at least half full (host call of
+    // 12 x 6,240 points 41.5 and 43.0, of 26 x 5,000 48.0 and 43.3)
+    std::vector<int32_t> more;
+    if (b->one_per_instance && 2 * b->tiles.size() <= (size_t)(3 * b->n_cu) && 2 * b->most_points > 3 * (int64_t)T)
+        for (int32_t t = 0; t < (int32_t)b->tiles.size(); ++t)
+            if (b->tiles[t].begin > 0) more.push_back(t);
+    b->n_more = (int32_t)more.size();
     // tile queues: 1 = one queue in instance order; 2 = one queue grouped by grid;
     // 3 = grouped by grid and cut into one queue per XCD with balanced point counts;
     // 4 = one queue per XCD by the tile's place in its instance's point order: a
@@ -687,7 +701,14 @@ static int plan(atac_batch b, const atac_tuning* t) {
     if (!rc) rc = dalloc(&b->d_tile_live, b->n_tiles);
     if (!rc) rc = dalloc(&b->d_tile_chunk0, b->n_tiles);
     if (!rc) rc = dalloc(&b->d_chunks, (size_t)b->chunk_cap);
+    if (!rc && b->n_more) rc = dalloc(&b->d_more, more.size());
+    if (!rc && b->n_more) rc = dalloc(&b->d_tile_sum, b->tiles.size() * 12);
+    if (!rc && b->n_more) rc = dalloc(&b->d_tiles_done, b->inst_dev.size());
     if (rc) return rc;
+    if (b->n_more) {
+        ATAC_HIP(hipMemcpy(b->d_more, more.data(), sizeof(int32_t) * more.size(), hipMemcpyHostToDevice));
+        ATAC_HIP(hipMemset(b->d_tiles_done, 0, sizeof(int32_t) * b->inst_dev.size()));
+    }
     // no stale counts before the first evaluation
     ATAC_HIP(hipMemset(b->d_counters, 0, sizeof(int32_t) * CNT_ALL));
     if (b->n_tiles > 0) ATAC_HIP(hipMemset(b->d_tile_active, 0, sizeof(int32_t) * b->n_tiles));
@@ -895,7 +916,7 @@ static int eval_done(atac_batch b, bool fused, bool precise, hipStream_t st) {
 // 2,000 points 60 against 45; 256 of them 22 against 34 and 41 against 39.
 static bool takes_one_per_instance(atac_batch b, uint32_t flags) {
     return b->one_per_instance && !(flags & ATAC_EVAL_ALL_ACTIVE) && b->n_tiles > 0 &&
-           b->most_points <= inst_points(mode_of(flags)) && (mode_of(flags) < 2 || b->inst.size() <= (size_t)b->n_cu);
+           (mode_of(flags) == 0 || b->most_points <= inst_points(mode_of(flags))) && (mode_of(flags) < 2 || b->inst.size() <= (size_t)b->n_cu);
 }
 
 // overflow_out (optional) receives the evaluation's overflow flag from the reduction.
@@ -945,7 +966,9 @@ static int enqueue_eval(atac_batch b, uint32_t flags, const atac_outputs* out, h
         if (out) { ia.fm = out->fm; ia.p6 = out->dfm_dp6; ia.Km = out->Km; ia.Dm = out->Dm; ia.n_active = out->n_active; }
         ia.overflow_out = overflow_out; ia.host_dst = overflow_out ? 1 : 0; ia.done = done;
         ia.call = call; ia.src = call ? b->pin_inst : nullptr;
-        ATAC_HIP(launch_instance(ia, mode, precise, rigid, (int)b->inst.size(), st));
+        ia.n_inst = (int32_t)b->inst.size(); ia.more = b->d_more; ia.n_more = b->n_more;
+        ia.tile_points = b->tune.tile_points; ia.tile_sum = b->d_tile_sum; ia.tiles_done = b->d_tiles_done;
+        ATAC_HIP(launch_instance(ia, mode, precise, rigid, st));
         return eval_done(b, false, precise, st);
     }
     if (!cull) ATAC_HIP(launch_reset(b->d_counters, CNT_WORDS, st));

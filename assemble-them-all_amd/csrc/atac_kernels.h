@@ -116,9 +116,9 @@ struct ReduceArgs {
 };
 
 // One workgroup per instance (instance_kernel): instances of at most that many points
-// (mode 0: the wrench alone).
+// (mode 0: the wrench alone, also by tiles).
 constexpr int kInstBlock = 512;
-constexpr int inst_points(int mode) { return mode == 0 ? 3072 : 2048; }
+constexpr int inst_points(int mode) { return mode == 0 ? 8192 : 2048; }
 struct InstanceArgs {
     InstDev* inst;
     const GridDev* grids;
@@ -141,7 +141,15 @@ struct InstanceArgs {
     int32_t* done;              // optional, in host memory: receives `call` behind the instance's outputs
     const InstDev* src;         // optional, in host memory: the instances, copied to inst first
     int32_t call;
-    int32_t pad;
+    int32_t n_inst;
+    // mode 0, n_more > 0: a workgroup per tile. The tiles that are not their instance's
+    // first (behind the instances' own), the tiles' sums (12 each) and the finished tiles
+    // per instance (zero between launches)
+    const int32_t* more;
+    int32_t n_more;
+    int32_t tile_points;
+    double* tile_sum;
+    int32_t* tiles_done;
 };
 
 struct PlainArgs {
@@ -188,7 +196,7 @@ hipError_t launch_fused(const ContactArgs& a, bool precise, bool split, int grid
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t st);
 // the same after the Km/Dm pass: rows of kJvpRow, dst = fm, dfm_dp6, Km, Dm
 hipError_t launch_reduce_jacobian(const ReduceArgs& a, bool rigid, hipStream_t st);
-hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, bool rigid, int n_inst, hipStream_t st);
+hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, bool rigid, hipStream_t st);
 // instance records, and (call != nullptr) the number of the call to counters[CNT_CALL],
 // from host memory the device can read
 hipError_t launch_upload(const InstDev* src, InstDev* dst, int n, const int32_t* call, int32_t* counters, hipStream_t st);

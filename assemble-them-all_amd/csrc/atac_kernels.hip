@@ -877,13 +877,16 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a, int 
 // launches of the pipeline above are each a chain of dependent reads, with a drain
 // and a launch between them; this is one chain. 64 instances of 500 points: 14 us
 // against 30 (wrench), 21 against 33 (Km/Dm); of 2,000 points 18 against 34 and 37
-// against 37. What an instance's points cost depends on the contacts among them, which
-// no rule knows beforehand: of 3,000 points with 5 % contacts (12 instances) 14.5 us
-// against 25.5, with nothing else 37.4 against 30.8; one of 8,000 17 against 24, but 84
-// against 31 (Km/Dm: a round of 512 contacts takes some 20 us). inst_points lies where
-// an instance of contacts alone takes as long as the passes of one tile each once took.
-// Slow-path contacts: 102 among 2,048 points 15 us against 23, 500 of 500 26 against
-// 26, but 2,048 of 2,048 85 against 34 (one workgroup against all of slow_kernel's).
+// against 37. What a workgroup's points cost depends on the contacts among them (a
+// round of 512 takes 4 us, for Km/Dm some 20), which no rule knows beforehand: of 3,000
+// points with 5 % contacts (12 instances) 13.7 us against 25.5, with nothing else 37.6
+// against 30.8. So inst_points is small for Km/Dm, and while the GPU is not full the
+// wrench of larger instances has a workgroup per tile (MORE), the last of which adds
+// the tiles' sums: one of 8,000 points takes 14.6 us with 5 % contacts and 48 with
+// nothing else (by one workgroup 16.7 and 84; the pipeline 24 and 31).
+// Slow-path contacts: 102 among 2,048 points 14.8 us against 23 in the pipeline, 500 of
+// 500 26 against 26, but 2,048 of 2,048 85 against 34 (slow_kernel has the whole GPU;
+// with 20 lanes per contact it was 206).
 // Nothing is reserved with atomics: an instance's records start at its tile's slot
 // and its work items at InstDev::chunk0, so a batch needs a record per point. The
 // active list, records, work items and tile entries are left as the pipeline leaves
@@ -891,29 +894,30 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a, int 
 // slot), for the adjoint; the sums run in the pipeline's order, per work item, then the
 // items in turn. A host call's instances are read from its pinned copy: an upload of
 // its own costs 4 us.
-// RIGID: as for jacobian_kernel (MODE 2).
-template <int MODE, typename R, bool RIGID>
+// RIGID: as for jacobian_kernel (MODE 2). MORE (MODE 0): a workgroup per tile.
+template <int MODE, typename R, bool RIGID, bool MORE>
 __global__ __launch_bounds__(kInstBlock) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 2 : 4)))
 void instance_kernel(InstanceArgs a) {
     using Rec = typename RecOf<R>::type;
     constexpr int NT = kInstBlock, NW = NT / 64, PPL = 4, SP = 64, ITEMS = NW / 4;
     constexpr bool JAC = MODE == 2;
     constexpr int NF = JAC ? (RIGID ? kJacRow : kJvpRow) : MODE == 1 ? 24 : 12;
-    constexpr int SLOW = 128, SROW = kStencil + 1;   // slow contacts whose stencils the lanes share
+    constexpr int GROUPS = 64 / kStencil, MANY = 96;
     __shared__ uint16_t s_list[inst_points(MODE)];   // the active offsets in point order, bit 15 = slow path
+    __shared__ double s_stencil[NW][GROUPS][kStencil];
     __shared__ double s_val[NW][JAC ? JacColumns::SIZE : 64 * NF];
-    // until the contacts: the wavefronts' own active offsets, the slow ones' places in s_list,
-    // and of SLOW slow contacts the SDF-frame positions and the stencil's values
-    static_assert(sizeof s_val >= 4 * inst_points(MODE) + 8 * SLOW * (3 + SROW), "all of it lies in s_val");
+    // until the contacts: the wavefronts' own active offsets, and the slow ones' places in s_list
+    static_assert(sizeof s_val >= 4 * inst_points(MODE), "both lists lie in s_val");
     uint16_t* const s_q = reinterpret_cast<uint16_t*>(s_val);
     uint16_t* const s_slow = s_q + inst_points(MODE);
-    double* const s_pos = reinterpret_cast<double*>(s_slow + inst_points(MODE));
-    double* const s_stencil = s_pos + 3 * SLOW;
     __shared__ double s_part[NW][JAC ? (RIGID ? kJacRowPad : kJvpRowPad) : 1];
     __shared__ double s_row[ITEMS][JAC ? 1 : NF];
     __shared__ double s_sum[NF], s_m[JAC ? 288 : 1], s_R[9], s_t[3];
-    __shared__ int s_count[NW], s_nslow;
-    const int tid = (int)threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), i = (int)blockIdx.x;
+    __shared__ int s_count[NW], s_nslow, s_last;
+    const int tid = (int)threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool first = !MORE || (int)blockIdx.x < a.n_inst;   // the instance's first (or only) tile
+    const int tile = first ? 0 : as_const(a.more)[(int)blockIdx.x - a.n_inst];
+    const int i = first ? (int)blockIdx.x : as_const(a.tiles)[tile].inst;
     const uint64_t lt_mask = (1ull << lane) - 1ull;
     if (tid == 0) s_nslow = 0;
     if (a.src) {
@@ -924,6 +928,11 @@ void instance_kernel(InstanceArgs a) {
     __syncthreads();
     const InstDev* inst = a.inst;
     asm volatile("" : "+s"(inst));   // its reads stay behind the copy
+    // the tile's points: `begin` on, `np` of them
+    const auto part = [&](const InstDev& in, int& begin, int& np) {
+        begin = first ? 0 : (tile - in.tile_begin) * a.tile_points;
+        np = MORE ? min(a.tile_points, (int)in.pt_count - begin) : (int)in.pt_count;
+    };
     // detection: wavefront w takes a contiguous range of the steps of 64 points, PPL
     // steps at a time: their point reads, then their table reads, then their cells are
     // out together, so a pass over 2,048 points waits three times
@@ -931,9 +940,11 @@ void instance_kernel(InstanceArgs a) {
     {
         const InstDev in = as_const(inst)[i];
         const GridDev G = as_const(a.grids)[in.grid];
-        const int np = (int)in.pt_count, ns = (np + SP - 1) / SP, st1 = (w + 1) * ns / NW;
+        int begin, np;
+        part(in, begin, np);
+        const int ns = (np + SP - 1) / SP, st1 = (w + 1) * ns / NW;
         st0 = w * ns / NW;
-        const auto px = as_global(in.px), py = as_global(in.py), pz = as_global(in.pz);
+        const auto px = as_global(in.px) + begin, py = as_global(in.py) + begin, pz = as_global(in.pz) + begin;
         const ClsConsts kc = cls_consts_vgpr(G, in);
         const auto cells = ATAC_GLOBAL(G.cells);
         const float cth = (float)in.col_th;
@@ -975,102 +986,89 @@ void instance_kernel(InstanceArgs a) {
     asm volatile("" : "+s"(again));
     const InstDev in = as_const(again)[i];
     const GridDev G = as_const(a.grids)[in.grid];
-    const int np = (int)in.pt_count;
-    const auto px = as_global(in.px), py = as_global(in.py), pz = as_global(in.pz);
+    int begin, np;
+    part(in, begin, np);
+    const auto px = as_global(in.px) + begin, py = as_global(in.py) + begin, pz = as_global(in.pz) + begin;
     // the active list in point order, for the adjoint too, and the slow-path contacts
     int before = 0, cnt = 0;
     for (int k = 0; k < NW; ++k) {
         if (k < w) before += s_count[k];
         cnt += s_count[k];
     }
-    const int64_t slot0 = in.tile_count ? as_const(a.tiles)[in.tile_begin].slot : 0;
+    const int64_t slot0 = in.tile_count ? as_const(a.tiles)[in.tile_begin].slot + begin : 0;
     for (int k = lane; k < wcount; k += 64) {
         const uint32_t e = s_q[st0 * SP + k];
         const int j = before + k;
         s_list[j] = (uint16_t)e;
-        a.act[slot0 + j] = (e & 0x7fffu) | (e >> 15 ? kActSlow : 0u);
+        a.act[slot0 + j] = ((uint32_t)begin + (e & 0x7fffu)) | (e >> 15 ? kActSlow : 0u);
         if (e >> 15) s_slow[atomicAdd(&s_nslow, 1)] = (uint16_t)j;
     }
     // work items: kChunk contacts each
     const int items = (cnt + kChunk - 1) / kChunk;
+    const int tile_at = first ? in.tile_begin : tile, chunk0 = in.chunk0 + begin / kChunk;
     if (tid == 0 && in.tile_count) {
-        for (int t = 0; t < in.tile_count; ++t) a.tile_active[in.tile_begin + t] = t ? 0 : cnt;
-        a.tile_chunk0[in.tile_begin] = in.chunk0;
+        a.tile_active[tile_at] = cnt;
+        a.tile_chunk0[tile_at] = chunk0;
+        if constexpr (!MORE)   // one workgroup for all of the instance's tiles
+            for (int t = 1; t < in.tile_count; ++t) a.tile_active[tile_at + t] = 0;
     }
     if (tid < (np + kChunk - 1) / kChunk)
-        a.chunks[in.chunk0 + tid] = tid < items ? ChunkDev{i, min(kChunk, cnt - tid * kChunk), slot0 + tid * kChunk}
-                                                : ChunkDev{i, 0, 0};
-    if (i == 0 && tid == 0) {
+        a.chunks[chunk0 + tid] = tid < items ? ChunkDev{i, min(kChunk, cnt - tid * kChunk), slot0 + tid * kChunk}
+                                             : ChunkDev{i, 0, 0};
+    if (blockIdx.x == 0 && tid == 0) {
         a.counters[CNT_RECS] = 0;   // counted by the tiles' entries
         a.counters[CNT_CHUNKS] = a.chunk_total;
         a.counters[CNT_SLOW] = 0;
         a.counters[CNT_OVERFLOW] = 0;
-        if (a.overflow_out) *a.overflow_out = 0;
     }
     __syncthreads();
-    // slow-path records. Many: a lane each. Up to SLOW: their positions, a lane each; the 20
-    // stencil evaluations of each over all lanes, SU of a lane's reads together; the record,
-    // a lane each
+    // slow-path records: the 20 stencil evaluations of a contact on 20 lanes, as slow_kernel
+    // (2.4 us for 24 contacts); many: a lane per contact, the stencil's positions along the
+    // axes formed once (14 us for 512)
     Rec* rec = static_cast<Rec*>(a.rec) + slot0;
     const auto slow_point = [&](int k, Rec& r) {
         const int j = s_slow[k];
         const uint32_t off = s_list[j] & 0x7fffu;
-        r.a[0] = px[off]; r.a[1] = py[off]; r.a[2] = pz[off]; r.a[3] = __uint_as_float(off);
+        r.a[0] = px[off]; r.a[1] = py[off]; r.a[2] = pz[off]; r.a[3] = __uint_as_float((uint32_t)begin + off);
         return j;
     };
-    int base = 0;
-    for (; s_nslow - base > SLOW; base += NT) {
-        if (base + tid >= s_nslow) continue;
+    const auto diag_of = [&](int j) { return a.slow_diag ? a.slow_diag + 4 * (slot0 + j) : nullptr; };
+    const int many = s_nslow > MANY ? s_nslow : 0;
+    for (int k = tid; k < many; k += NT) {
         Rec r;
-        const int j = slow_point(base + tid, r);
-        record_slow(G, in, r, a.slow_diag ? a.slow_diag + 4 * (slot0 + j) : nullptr);
+        const int j = slow_point(k, r);
+        record_slow(G, in, r, diag_of(j));
         mark_slow_index(r, (int)(slot0 + j));
         store_rec(rec + j, r);
     }
-    if (base < s_nslow) {
-        constexpr int SU = 2;
-        const int m = s_nslow - base, samples = m * kStencil;
+    for (int base = many + w * GROUPS; base < s_nslow; base += NW * GROUPS) {
+        const int grp = lane / kStencil, st = lane % kStencil;
+        const bool mine = grp < GROUPS && base + grp < s_nslow;
         Rec r;
         int j = 0;
-        if (tid < m) {
-            j = slow_point(base + tid, r);
-            double x[3];
+        if (mine) {
+            j = slow_point(base + grp, r);
+            double x[3], q[3];
+            bool accurate;
             body2_point(in, (double)r.a[0], (double)r.a[1], (double)r.a[2], x);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) s_pos[3 * tid + k] = x[k];
+            stencil_point(x, st, q, accurate);
+            s_stencil[w][grp][st] = query_sdf64(G, q[0], q[1], q[2], accurate);
         }
-        __syncthreads();
-        for (int t0 = tid; t0 < samples; t0 += SU * NT) {
-            double p[SU][3];
-            Axis64 t[SU][3];
-            float v[SU][8];
-            bool accurate[SU];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (mine && st == 0) {
+            double v[kStencil], val, g[3], H[6];
 #pragma unroll
-            for (int u = 0; u < SU; ++u) {   // (past the end: the last sample again)
-                const int e = min(t0 + u * NT, samples - 1);
-                stencil_point(s_pos + 3 * (e / kStencil), e % kStencil, p[u], accurate[u]);
-#pragma unroll
-                for (int k = 0; k < 3; ++k) t[u][k] = axis64(G, k, p[u][k]);   // (nodes in the grid for any p)
-            }
-#pragma unroll
-            for (int u = 0; u < SU; ++u) trilinear64_nodes(G, t[u][0], t[u][1], t[u][2], v[u]);
-#pragma unroll
-            for (int u = 0; u < SU; ++u) {
-                double val = trilinear64_value(t[u][0], t[u][1], t[u][2], v[u]);
-                if (!inside_box64(G, p[u][0], p[u][1], p[u][2])) val = query_sdf64(G, p[u][0], p[u][1], p[u][2], accurate[u]);
-                const int e = t0 + u * NT;
-                if (e < samples) s_stencil[SROW * (e / kStencil) + e % kStencil] = val;
-            }
-        }
-        __syncthreads();
-        if (tid < m) {
-            double val, g[3], H[6];
-            stencil_combine(reinterpret_cast<const double (&)[kStencil]>(s_stencil[SROW * tid]), val, g, H);
-            float* diag = a.slow_diag ? a.slow_diag + 4 * (slot0 + j) : nullptr;
-            record_slow_fill(in, val, g, H, r, diag);
+            for (int q = 0; q < kStencil; ++q) v[q] = s_stencil[w][grp][q];
+            stencil_combine(v, val, g, H);
+            record_slow_fill(in, val, g, H, r, diag_of(j));
             mark_slow_index(r, (int)(slot0 + j));
             store_rec(rec + j, r);
         }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     __syncthreads();
     // ITEMS work items at a time, a wavefront per 64 contacts
@@ -1087,7 +1085,8 @@ void instance_kernel(InstanceArgs a) {
             ContactFwd<R> s;
             R p6[12];
             const auto forward = [&](const InstDev& in, const InstR<R>& I) {
-                const Rec r = item_record(G, in, off | (e >> 15 ? kActSlow : 0u), px[off], py[off], pz[off], rec + j);
+                const Rec r = item_record(G, in, ((uint32_t)begin + off) | (e >> 15 ? kActSlow : 0u), px[off], py[off], pz[off],
+                                          rec + j);
                 record_decode(r, a.slow_diag, in, s);
                 contact_forward<R>(I, s, MODE >= 1 ? p6 : nullptr);
             };
@@ -1152,6 +1151,27 @@ void instance_kernel(InstanceArgs a) {
         }
     }
     __syncthreads();
+    if constexpr (MORE) {
+        if (in.tile_count > 1) {   // the last of the instance's workgroups adds the tiles' sums, in their order
+            if (tid < 12)
+                __hip_atomic_store(a.tile_sum + 12 * (int64_t)tile_at + tid, s_sum[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            if (tid == 0)   // one release and acquire for the workgroup: each writes the XCD's L2 back
+                s_last = __hip_atomic_fetch_add(a.tiles_done + i, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == in.tile_count - 1;
+            __syncthreads();
+            if (!s_last) return;
+            cnt = 0;
+            double sum = 0.0;
+            for (int t = in.tile_begin; t < in.tile_begin + in.tile_count; ++t) {
+                cnt += __hip_atomic_load(a.tile_active + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (tid < 12) sum += __hip_atomic_load(a.tile_sum + 12 * (int64_t)t + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (tid < 12) s_sum[tid] = sum;
+            if (tid == 0) __hip_atomic_store(a.tiles_done + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+        }
+    }
+    if (a.overflow_out && i == 0 && tid == 0) *a.overflow_out = 0;
     if (tid < 12 && a.fm) a.fm[(int64_t)i * 12 + tid] = s_sum[tid];
     if (MODE >= 1 && tid >= 12 && tid < 24 && a.p6) a.p6[(int64_t)i * 12 + tid - 12] = s_sum[MODE >= 1 ? tid : 0];
     if (tid == 0 && a.n_active) a.n_active[i] = cnt;
@@ -1626,18 +1646,20 @@ hipError_t launch_reduce_jacobian(const ReduceArgs& a, bool rigid, hipStream_t s
     return hipSuccess;
 }
 
-template <int MODE, bool RIGID>
-static void launch_instance_m(const InstanceArgs& a, bool precise, int n_inst, hipStream_t st) {
-    if (precise) hipLaunchKernelGGL((instance_kernel<MODE, double, RIGID>), dim3(n_inst), dim3(kInstBlock), 0, st, a);
-    else hipLaunchKernelGGL((instance_kernel<MODE, float, RIGID>), dim3(n_inst), dim3(kInstBlock), 0, st, a);
+template <int MODE, bool RIGID, bool MORE>
+static void launch_instance_m(const InstanceArgs& a, bool precise, hipStream_t st) {
+    const dim3 grid(a.n_inst + (MORE ? a.n_more : 0));
+    if (precise) hipLaunchKernelGGL((instance_kernel<MODE, double, RIGID, MORE>), grid, dim3(kInstBlock), 0, st, a);
+    else hipLaunchKernelGGL((instance_kernel<MODE, float, RIGID, MORE>), grid, dim3(kInstBlock), 0, st, a);
 }
 
-hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, bool rigid, int n_inst, hipStream_t st) {
-    if (n_inst <= 0) return hipSuccess;
-    if (mode == 0) launch_instance_m<0, true>(a, precise, n_inst, st);
-    else if (mode == 1) launch_instance_m<1, true>(a, precise, n_inst, st);
-    else if (rigid) launch_instance_m<2, true>(a, precise, n_inst, st);
-    else launch_instance_m<2, false>(a, precise, n_inst, st);
+hipError_t launch_instance(const InstanceArgs& a, int mode, bool precise, bool rigid, hipStream_t st) {
+    if (a.n_inst <= 0) return hipSuccess;
+    if (mode == 0 && a.n_more) launch_instance_m<0, true, true>(a, precise, st);
+    else if (mode == 0) launch_instance_m<0, true, false>(a, precise, st);
+    else if (mode == 1) launch_instance_m<1, true, false>(a, precise, st);
+    else if (rigid) launch_instance_m<2, true, false>(a, precise, st);
+    else launch_instance_m<2, false, false>(a, precise, st);
     return hipGetLastError();
 }
 

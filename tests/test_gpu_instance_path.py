@@ -84,3 +84,48 @@ def test_captured_and_replayed(gpu):
         torch.cuda.synchronize()
         for k in want:
             assert torch.equal(out[k], want[k]), k
+
+
+def test_several_tiles(gpu):
+    """Instances of more than one tile, beside small and empty ones: the tiles' workgroups finish in any order, and
+    every launch, replay and host call gives the same bits; the next launch starts from clear counts."""
+    import ctypes as C
+
+    import torch
+
+    from atac import _lib as L
+    sizes = [4097, 0, 8192, 100, 6240, 4096, 8191, 5000]
+    w = _workload(sizes, 0.05)
+    b, ref = batch_from_workload(w), batch_from_workload(w, tuning={"max_active": -1})
+    g = torch.tensor(np.random.default_rng(3).normal(size=(b.n, 12)), device="cuda")
+    for precise in (False, True):
+        want, grads = b.eval(precise=precise), b.vjp(g)
+        other, ograds = ref.eval(precise=precise), ref.vjp(g)
+        out = b.alloc_outputs()
+        for k, v in {**want, **grads}.items():
+            q = {**other, **ograds}[k].double()
+            assert (v - q).abs().max() <= (0 if k == "n_active" else TOL[precise]) * q.abs().max(), k
+        for _ in range(50):
+            b.eval(precise=precise, out=out)
+            assert torch.equal(out["fm"], want["fm"]) and torch.equal(out["n_active"], want["n_active"])
+        b.graph_capture(out, precise=precise)
+        for _ in range(3):
+            out["fm"].zero_()
+            b.graph_launch()
+            assert torch.equal(out["fm"], want["fm"])
+        fm, na = np.zeros((b.n, 12)), np.zeros(b.n, dtype=np.int32)
+        for _ in range(20):
+            fm[:] = 0.0
+            L.check(L.lib().atac_batch_eval_instances_host(b.handle, b.instances, b.n, b.flags(precise=precise),
+                                                           fm.ctypes.data_as(C.c_void_p), None, None, None,
+                                                           na.ctypes.data_as(C.c_void_p)))
+            assert np.array_equal(fm, want["fm"].cpu().numpy()) and np.array_equal(na, want["n_active"].cpu().numpy())
+        again = b.vjp(g)
+        assert all(torch.equal(again[k], grads[k]) for k in grads)
+        for i in (0, 4, 14):
+            assert np.array_equal(b.active_ids(i), ref.active_ids(i))
+
+
+def test_one_workgroup_for_several_tiles(gpu):
+    """More tiles than three for two CUs: a workgroup takes all tiles of its instance."""
+    _compare(_workload([4100, 8192] * 50, 0.05), {})
