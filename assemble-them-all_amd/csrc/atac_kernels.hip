@@ -529,11 +529,12 @@ __global__ __launch_bounds__(256) void contact_kernel(ContactArgs a) {
 // Work items of kChunk records, one workgroup each, wavefront w taking records
 // [64 w, 64 w + 64), one per lane: the wrench, the p6 column and the blocks Km and
 // Dm are made of (contact_jac), summed over the item into its partial row
-// (kJacRow of its kJvpRow values; poses that are not rotations fill it). Bound by instruction issue: about 1,700 instructions per 64
-// contacts, where 24 tangents per contact and their 288 wave sums took about 13,000
-// (an evaluation of 256 poses x 5,000 points with Km/Dm: 149 -> 57 us; of 26 poses
-// from host memory: 132 -> 80 us). 64 contacts per wavefront rather than 256:
-// small batches have few items and need the waves. RIGID: every instance's poses are
+// (kJacRow of its kJvpRow values; poses that are not rotations fill it). Bound by
+// instruction issue: about 1,700 instructions per 64 contacts, where 24 tangents per
+// contact and their 288 wave sums took about 13,000 (an evaluation of 256 poses x 5,000
+// points with Km/Dm: 149 us with these, 57 with the blocks, 47 with what the other
+// kernels gained since; this one 31). 64 contacts per wavefront rather than 256: small
+// batches have few items and need the waves. RIGID: every instance's poses are
 // rotations. Otherwise each item takes the form of its instance (InstDev::rigid), which
 // costs the blocks 4 % (FP32) and 25 % (FP64, spilled registers) of an evaluation.
 template <typename R, bool RIGID>
@@ -1467,8 +1468,7 @@ __global__ void distance_kernel(PointArgs a) {
 // of the 18 directions. The results wait in LDS (in the arithmetic's type) and
 // leave in memory order, 512 bytes per store: written by the lanes themselves,
 // each store touched 64 lines 1,080 bytes apart (120,000 points with derivatives:
-// 190 -> 58 us a call). Bound by the 1,168 bytes a point
-// writes.
+// 191 -> 51 us a call). Bound by the 1,168 bytes a point writes.
 constexpr int kCollPoints = 32, kCollLanes = 64 / kCollPoints;
 template <bool DERIV, typename R>
 __global__ __launch_bounds__(64) void collision_kernel(PointArgs a) {
