@@ -414,16 +414,17 @@ __global__ __launch_bounds__(kLsLanes) void ls_sweep_kernel(LsArgs a, LsSweep s)
 // One wavefront per x line: the parity of the crossings up to each node.
 __global__ __launch_bounds__(256) void ls_sign_kernel(LsArgs a) {
     const int lane = (int)threadIdx.x & 63;
-    const int64_t line = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (line >= (int64_t)a.nj * a.nk) return;
-    const int64_t row = line * a.ni;
-    unsigned odd = 0;
-    for (int i0 = 0; i0 < a.ni; i0 += 64) {
-        const int i = i0 + lane;
-        const uint64_t m = __ballot(i < a.ni && (a.count[row + (i < a.ni ? i : 0)] & 1));
-        const unsigned here = odd + (unsigned)__popcll(m & (~0ull >> (63 - lane)));
-        if (i < a.ni && (here & 1u)) a.phi[row + i] = -a.phi[row + i];
-        odd += (unsigned)__popcll(m);
+    const int64_t lines = (int64_t)a.nj * a.nk, step = (int64_t)gridDim.x * 4;
+    for (int64_t line = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); line < lines; line += step) {
+        const int64_t row = line * a.ni;
+        unsigned odd = 0;
+        for (int i0 = 0; i0 < a.ni; i0 += 64) {
+            const int i = i0 + lane;
+            const uint64_t m = __ballot(i < a.ni && (a.count[row + (i < a.ni ? i : 0)] & 1));
+            const unsigned here = odd + (unsigned)__popcll(m & (~0ull >> (63 - lane)));
+            if (i < a.ni && (here & 1u)) a.phi[row + i] = -a.phi[row + i];
+            odd += (unsigned)__popcll(m);
+        }
     }
 }
 
@@ -470,7 +471,8 @@ hipError_t ls_build(const LsArgs& a, hipStream_t st) {
             if (e != hipSuccess) return e;
         }
     }
-    hipLaunchKernelGGL(ls_sign_kernel, dim3((unsigned)(((int64_t)a.nj * a.nk + 3) / 4)), dim3(256), 0, st, a);
+    const int64_t blocks = std::min<int64_t>(((int64_t)a.nj * a.nk + 3) / 4, 65536);
+    hipLaunchKernelGGL(ls_sign_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

@@ -24,3 +24,19 @@ def test_tile_edges_bitwise(gpu, n):
     ref = O.make_level_set3(V.astype(np.float32), F, origin, d, n, 1)
     got = level_set(V, F, origin, d, n, 1)
     assert np.array_equal(np.asarray(got).view(np.uint32), np.asarray(ref).view(np.uint32))
+
+
+def test_more_lines_than_one_launch_holds(gpu):
+    """2^26 x lines and more, a wavefront each: the signs of a box in the last corner of a flat grid are those
+    of a small grid around it (coordinates of small whole numbers: the same distances)."""
+    from atac.sdfmesh import level_set
+    V, F = M.box(3.25)
+    big, small = (1, 8200, 8200), (1, 20, 20)
+    at = lambda n, off: (0.0, float(off - n[1]), float(off - n[2]))   # the box 10 nodes before the end
+    got = level_set(V, F, at(big, 10), (1.0, 1.0, 1.0), big, 1)
+    ref = level_set(V, F, at(small, 10), (1.0, 1.0, 1.0), small, 1)
+    corner = got[-20:, -20:]
+    assert np.array_equal(corner < 0, ref < 0) and (ref < 0).sum() == 49
+    near = np.abs(ref) < 2.0
+    assert np.array_equal(corner[near], ref[near])
+    assert (got < 0).sum() == 49
