@@ -86,7 +86,11 @@ typedef struct {
 
 /* Outputs of one evaluation, device pointers, any may be NULL. Per instance:
  * fm 12 = [tau1 f1 tau2 f2] (each body's frame, angular first), Km/Dm 144 row-major
- * (d fm / d [q1 q2], d fm / d [phi1 phi2], pose perturbation E <- E exp([w; v])),
+ * (d fm / d [q1 q2], d fm / d [phi1 phi2], pose perturbation E <- E exp([w; v])), the
+ * derivative of fm with the pose matrices as they are given: where R^T R differs from I
+ * by more than 2^-46 (poses from FP32 data, say) they come from a slower form; a Km/Dm
+ * evaluation captured in a graph of the caller's own holds kernels for both (4 % slower,
+ * 25 % in FP64; atac_batch_graph_capture records each when it is needed).
  * dfm_dp6 12 (d fm / d contact_scale as the reference assembles it), n_active 1. */
 typedef struct {
     double* fm;
