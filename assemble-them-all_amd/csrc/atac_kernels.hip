@@ -887,7 +887,10 @@ __global__ __launch_bounds__(256) void reduce_jacobian_kernel(ReduceArgs a, int 
 // nothing else (by one workgroup 16.7 and 84; the pipeline 24 and 31).
 // Slow-path contacts: 102 among 2,048 points 14.8 us against 23 in the pipeline, 500 of
 // 500 26 against 26, but 2,048 of 2,048 85 against 34 (slow_kernel has the whole GPU;
-// with 20 lanes per contact it was 206).
+// with 20 lanes per contact it was 206). One FP32 instance with a tenth, a quarter and
+// half of its points slow: of 1,000 14, 19 and 27 us against 22, 24 and 25; of 2,048 18,
+// 28 and 48 against 25, 26 and 29; of 8,000 29, 55 and 97 against 27, 31 and 39. So the
+// pipeline is the faster one for large faces on a cell plane, which no rule knows either.
 // Nothing is reserved with atomics: an instance's records start at its tile's slot
 // and its work items at InstDev::chunk0, so a batch needs a record per point. The
 // active list, records, work items and tile entries are left as the pipeline leaves
